@@ -1,0 +1,64 @@
+/*
+ * C ABI of the prompt forward (libmk_prefill.so): the dense Llama forward over a whole prompt that fills the KV cache
+ * before decoding starts (the reference runs it as a PyTorch module, megakernels/llama.py:232-296,328-348,384-403).
+ *
+ * Every function launches on `stream` (a hipStream_t, NULL = default stream) without synchronising and returns 0 or a
+ * negative error with a message in mk_prefill_last_error().  All tensors are contiguous device memory; bf16 tensors are
+ * passed as uint16_t bit patterns.  A "row" is one position of one sequence: rows = batch * seq.
+ */
+#ifndef MK_PREFILL_H
+#define MK_PREFILL_H
+
+#include <stdint.h>
+
+#ifdef __cplusplus
+extern "C" {
+#endif
+
+/* What the kernels need to know of the architecture and of this call. */
+typedef struct mk_prefill_shape {
+    int32_t batch, seq;
+    int32_t num_attention_heads, num_kv_heads, head_dim;   /* four query heads per KV head, head_dim 64 or 128 */
+    int32_t hidden_size, intermediate_size, vocab_size;
+    int32_t kv_max_len, rope_positions;
+    int32_t interleaved;                                   /* rotary pairs adjacent (1) or half a head apart (0) */
+    float rms_norm_eps;
+} mk_prefill_shape;
+
+/* Positions a sequence's keys and values are padded to in the workspace (mk_prefill_rope, mk_prefill_attention). */
+int mk_prefill_padded_seq(int seq);
+
+/* h[row] = embed[ids[row]]; x[row] = rms_norm(h[row]) * norm_weight.  An id outside the vocabulary or a position outside
+ * the rope tables or the cache (negative ones count from the end) aborts the kernel, as an index out of range does in
+ * PyTorch. */
+int mk_prefill_embed(const mk_prefill_shape *shape, const int64_t *ids, const int64_t *positions, const uint16_t *embed,
+                     const uint16_t *norm_weight, uint16_t *h, uint16_t *x, void *stream);
+
+/* h += y; x = rms_norm(h) * norm_weight */
+int mk_prefill_add_norm(const mk_prefill_shape *shape, const uint16_t *y, const uint16_t *norm_weight, uint16_t *h,
+                        uint16_t *x, void *stream);
+
+/* Rotates the query and key heads of qkv [rows, (H + 2 KVH) D], appends keys and values to the layer's cache
+ * [cache_batch, kv_max_len, KVH, D] and leaves q [rows, H D], keys [batch, KVH, padded, D] and transposed values
+ * [batch, KVH, D, padded] for mk_prefill_attention. */
+int mk_prefill_rope(const mk_prefill_shape *shape, const uint16_t *qkv, const int64_t *positions, const float *rope_cos,
+                    const float *rope_sin, uint16_t *k_cache, uint16_t *v_cache, uint16_t *q, uint16_t *keys,
+                    uint16_t *values_t, void *stream);
+
+/* Causal attention of every sequence over its own keys: out [rows, H D]. */
+int mk_prefill_attention(const mk_prefill_shape *shape, const uint16_t *q, const uint16_t *keys, const uint16_t *values_t,
+                         uint16_t *out, void *stream);
+
+/* out = silu(gate) * up, all [rows, intermediate_size] */
+int mk_prefill_silu_mul(const mk_prefill_shape *shape, const uint16_t *gate, const uint16_t *up, uint16_t *out,
+                        void *stream);
+
+/* ids[row] = index of the first maximum of logits[row, 0..vocab_size), a NaN counting as the largest value */
+int mk_prefill_argmax(const mk_prefill_shape *shape, const uint16_t *logits, int64_t *ids, void *stream);
+
+const char *mk_prefill_last_error(void);
+
+#ifdef __cplusplus
+}
+#endif
+#endif

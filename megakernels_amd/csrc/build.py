@@ -1,8 +1,9 @@
-"""Builds libmk_llama.so (the HIP megakernel and its C ABI) for gfx950.
+"""Builds libmk_llama.so (the HIP megakernel and its C ABI) and libmk_prefill.so (the prompt forward's kernels)
+for gfx950.
 
     python megakernels_amd/csrc/build.py
 
-The library is built in-tree next to its sources.  Flags that matter:
+The libraries are built in-tree next to their sources.  Flags that matter:
 ``-ffp-contract=off`` (only the explicit fmaf() calls fuse, so results are
 reproducible), and packed-fp32 code generation turned off.
 """
@@ -18,6 +19,8 @@ from pathlib import Path
 HERE = Path(__file__).resolve().parent
 SOURCE = HERE / "mk_llama.hip"
 LIBRARY = HERE / "libmk_llama.so"
+PREFILL_SOURCE = HERE / "mk_prefill.hip"
+PREFILL_LIBRARY = HERE / "libmk_prefill.so"
 
 HIPCC_FLAGS = [
     "-O3",
@@ -39,7 +42,13 @@ def find_hipcc() -> str:
 
 
 def build(verbose: bool = False) -> Path:
-    cmd = [find_hipcc(), *HIPCC_FLAGS, str(SOURCE), "-o", str(LIBRARY)]
+    for source, library in ((SOURCE, LIBRARY), (PREFILL_SOURCE, PREFILL_LIBRARY)):
+        compile_library(source, library, verbose)
+    return LIBRARY
+
+
+def compile_library(source: Path, library: Path, verbose: bool) -> None:
+    cmd = [find_hipcc(), *HIPCC_FLAGS, str(source), "-o", str(library)]
     if verbose:
         print(" ".join(cmd))
     proc = subprocess.run(cmd, capture_output=True, text=True)
@@ -51,7 +60,6 @@ def build(verbose: bool = False) -> Path:
     if proc.returncode != 0:
         sys.stderr.write(proc.stdout + proc.stderr)
         raise RuntimeError("hipcc failed")
-    return LIBRARY
 
 
 if __name__ == "__main__":

@@ -1,0 +1,492 @@
+// Prompt forward for MI355X (gfx950): what surrounds the matrix products of a dense Llama forward over a whole prompt.
+//
+// A prompt of a few thousand positions is bound by its matrix products; what a framework adds to them is traffic - the
+// same activations read and written once per small operation - and launches.  Here every stage between two products is
+// one kernel: residual add + RMS norm, rotary embedding + cache append + the layouts attention reads, attention itself,
+// SiLU * up, argmax.  Values are narrowed to bf16 exactly where the plain forward narrows them (megakernels/llama.py:38-47
+// for the norm, :136-174 for the rotation).
+#include <hip/hip_runtime.h>
+
+#include <cstdarg>
+#include <cstdint>
+#include <cstdio>
+
+#include "../../include/mk_prefill.h"
+
+namespace {
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+#define MK_LDS __attribute__((address_space(3)))
+#define MK_GLOBAL __attribute__((address_space(1)))
+
+__device__ __forceinline__ float bf16_lo(uint32_t pair) { return __builtin_bit_cast(float, pair << 16); }
+__device__ __forceinline__ float bf16_hi(uint32_t pair) { return __builtin_bit_cast(float, pair & 0xffff0000u); }
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+    const f32x2 v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+__device__ __forceinline__ float round_bf16(float v) { return bf16_lo(pack_bf16(v, 0.0f)); }
+__device__ __forceinline__ float bf16_f32(uint16_t v) { return __builtin_bit_cast(float, (uint32_t)v << 16); }
+
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+    for (int offset = 32; offset >= 1; offset /= 2) v += __shfl_xor(v, offset);
+    return v;
+}
+
+// ---------------------------------------------------------------------------------------------
+// Residual add + RMS norm, one block per row.  Bound by memory: two rows in, two out (the embedding
+// row instead of the two where the stream starts).
+// ---------------------------------------------------------------------------------------------
+constexpr int kNormThreads = 256;
+constexpr int kMaxHidden = 8192;
+constexpr int kNormChunks = kMaxHidden / (8 * kNormThreads);  // 16-byte pieces of a row per thread, at most
+
+// position as an index of a table of `count` rows: negative ones count from the end
+__device__ __forceinline__ int64_t wrap_position(int64_t position, int count) { return position < 0 ? position + count : position; }
+
+template <bool EMBED>
+__global__ __launch_bounds__(kNormThreads) void norm_kernel(mk_prefill_shape s, const int64_t *ids, const int64_t *positions,
+                                                            const uint16_t *src, const uint16_t *weight, uint16_t *h, uint16_t *x) {
+    const int row = blockIdx.x, hid = s.hidden_size, pieces = hid / 8;
+    const uint16_t *add = src + (size_t)row * hid;
+    if constexpr (EMBED) {
+        const int64_t id = ids[row], position = positions[row % s.seq];
+        const int64_t cache_row = wrap_position(position, s.kv_max_len), rope_row = wrap_position(position, s.rope_positions);
+        if (id < 0 || id >= s.vocab_size || cache_row < 0 || cache_row >= s.kv_max_len || rope_row < 0 || rope_row >= s.rope_positions)
+            __builtin_trap();
+        add = src + (size_t)id * hid;
+    }
+    uint16_t *const h_row = h + (size_t)row * hid;
+    u32x4 v[kNormChunks];
+    float sum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kNormChunks; i++) {
+        const int at = (int)threadIdx.x + i * kNormThreads;
+        if (at >= pieces) break;
+        v[i] = *(const u32x4 *)(add + (size_t)at * 8);
+        if constexpr (!EMBED) {
+            const u32x4 old = *(const u32x4 *)(h_row + (size_t)at * 8);
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[i][j] = pack_bf16(bf16_lo(old[j]) + bf16_lo(v[i][j]), bf16_hi(old[j]) + bf16_hi(v[i][j]));
+        }
+        *(u32x4 *)(h_row + (size_t)at * 8) = v[i];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const float lo = bf16_lo(v[i][j]), hi = bf16_hi(v[i][j]);
+            sum += lo * lo;
+            sum += hi * hi;
+        }
+    }
+    __shared__ float wave_sums[kNormThreads / 64];
+    sum = wave_sum(sum);
+    if (threadIdx.x % 64 == 0) wave_sums[threadIdx.x / 64] = sum;
+    __syncthreads();
+    sum = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kNormThreads / 64; w++) sum += wave_sums[w];
+    const float scale = rsqrtf(sum / (float)hid + s.rms_norm_eps);
+#pragma unroll
+    for (int i = 0; i < kNormChunks; i++) {
+        const int at = (int)threadIdx.x + i * kNormThreads;
+        if (at >= pieces) break;
+        const u32x4 w = *(const u32x4 *)(weight + (size_t)at * 8);
+        u32x4 out;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            out[j] = pack_bf16(bf16_lo(w[j]) * round_bf16(bf16_lo(v[i][j]) * scale), bf16_hi(w[j]) * round_bf16(bf16_hi(v[i][j]) * scale));
+        *(u32x4 *)(x + (size_t)row * hid + (size_t)at * 8) = out;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Rotary embedding, cache append, and the layouts attention reads.  One block per 64 positions of one
+// head (query, key or value).  Keys are copied to [KVH, padded, D] because the cache rows of a prompt need
+// not be consecutive.  Values are transposed to [KVH, D, padded] with the positions of every group of 16 in
+// the order 0-3, 8-11, 4-7, 12-15: the order in which attention's probabilities leave the matrix cores, so
+// that its second product reads both operands without exchanging lanes.  Padding positions hold zeros.
+// ---------------------------------------------------------------------------------------------
+constexpr int kPosTile = 64;
+
+__device__ __forceinline__ int slot_in_group(int position) {  // place of a position within its group of 16
+    return (position & 3) | ((position & 4) << 1) | ((position & 8) >> 1);
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void rope_kernel(mk_prefill_shape s, int padded, const uint16_t *qkv, const int64_t *positions,
+                                                   const float *rope_cos, const float *rope_sin, uint16_t *k_cache, uint16_t *v_cache,
+                                                   uint16_t *q, uint16_t *keys, uint16_t *values_t) {
+    constexpr int kPieces = D / 8;
+    const int H = s.num_attention_heads, KVH = s.num_kv_heads;
+    const int head = blockIdx.y, batch = blockIdx.z, first = blockIdx.x * kPosTile;
+    const size_t qkv_row = (size_t)(H + 2 * KVH) * D;
+    const bool is_value = head >= H + KVH;
+    const int kv_head = is_value ? head - H - KVH : head - H;
+    __shared__ uint16_t tile[D][kPosTile + 8];
+    for (int i = threadIdx.x; i < kPosTile * kPieces; i += 256) {
+        const int p = i / kPieces, piece = i % kPieces, seq_at = first + p;
+        u32x4 v = {0, 0, 0, 0};
+        if (seq_at < s.seq) {
+            const int64_t position = positions[seq_at];
+            const uint16_t *src = qkv + ((size_t)batch * s.seq + seq_at) * qkv_row + (size_t)head * D;
+            v = *(const u32x4 *)(src + piece * 8);
+            if (!is_value) {
+                const size_t rope_row = (size_t)wrap_position(position, s.rope_positions) * D + piece * 8;
+                u32x4 other = v;
+                if (!s.interleaved) other = *(const u32x4 *)(src + (piece * 8 + D / 2) % D);
+                const bool upper = piece * 8 >= D / 2;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const f32x2 c = *(const f32x2 *)(rope_cos + rope_row + 2 * j), sn = *(const f32x2 *)(rope_sin + rope_row + 2 * j);
+                    const float lo = bf16_lo(v[j]), hi = bf16_hi(v[j]);
+                    float part_lo = -hi, part_hi = lo;
+                    if (!s.interleaved) {
+                        part_lo = upper ? bf16_lo(other[j]) : -bf16_lo(other[j]);
+                        part_hi = upper ? bf16_hi(other[j]) : -bf16_hi(other[j]);
+                    }
+                    v[j] = pack_bf16(lo * c.x + part_lo * sn.x, hi * c.y + part_hi * sn.y);
+                }
+            }
+            if (head < H) {
+                *(u32x4 *)(q + (((size_t)batch * s.seq + seq_at) * H + head) * D + piece * 8) = v;
+            } else {
+                uint16_t *const cache = is_value ? v_cache : k_cache;
+                const size_t cache_row = (size_t)batch * s.kv_max_len + (size_t)wrap_position(position, s.kv_max_len);
+                *(u32x4 *)(cache + (cache_row * KVH + kv_head) * D + piece * 8) = v;
+            }
+        }
+        if (is_value) {
+            const int slot = (p & ~15) | slot_in_group(p & 15);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                tile[piece * 8 + 2 * j][slot] = (uint16_t)v[j];
+                tile[piece * 8 + 2 * j + 1][slot] = (uint16_t)(v[j] >> 16);
+            }
+        } else if (head >= H) {
+            *(u32x4 *)(keys + (((size_t)batch * KVH + kv_head) * padded + seq_at) * D + piece * 8) = v;
+        }
+    }
+    if (!is_value) return;
+    __syncthreads();
+    for (int i = threadIdx.x; i < D * (kPosTile / 8); i += 256) {
+        const int d = i / (kPosTile / 8), piece = i % (kPosTile / 8);
+        *(u32x4 *)(values_t + (((size_t)batch * KVH + kv_head) * D + d) * padded + first + piece * 8) = *(const u32x4 *)&tile[d][piece * 8];
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Causal attention.  A block works on one KV head and QB query positions: its waves are the four query
+// heads of the KV head times QB / 32 groups of 32 positions, and share the K and V tiles of 64 positions,
+// which go from memory straight into LDS (double-buffered, 16-byte pieces swizzled so that the reads of a
+// wave are spread over all banks).
+//
+// The scores are computed transposed, S^T = K Q^T: a query position is then a lane (lane % 32) and its
+// scores lie in that lane's registers, so the maximum and the sum over a tile need one exchange between
+// the two halves of the wave instead of a tree over lanes, rescaling the output is one factor per lane, and
+// the probabilities are already in the operand layout of O^T = V^T P^T.
+//
+// Bound by the vector units, not by the matrix cores, at head_dim 64: 2048 scores take 512 clocks of matrix
+// work per wave and about 900 of vector work (the exponential alone 512).
+// ---------------------------------------------------------------------------------------------
+constexpr int kKeyTile = 64;
+
+__device__ __forceinline__ float half_exchange_max(float v) {
+    uint32_t a = __builtin_bit_cast(uint32_t, v), b = a;
+    // written in assembly: the compiler's builtin for this instruction returns the first result twice
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    return fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+}
+__device__ __forceinline__ float half_exchange_sum(float v) {
+    uint32_t a = __builtin_bit_cast(uint32_t, v), b = a;
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
+}
+
+// 16 bytes per lane from memory into LDS at `dst` (the same in every lane) + 16 * lane
+__device__ __forceinline__ void load_to_lds(const void *src, MK_LDS void *dst) {
+    __builtin_amdgcn_global_load_lds((const MK_GLOBAL void *)src, dst, 16, 0, 0);
+}
+
+template <int D, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void attention_kernel(mk_prefill_shape s, int padded, float scale, const uint16_t *q,
+                                                               const uint16_t *keys, const uint16_t *values_t, uint16_t *out) {
+    constexpr int kGqa = 4, kQueries = 32 * WAVES / kGqa, kThreads = WAVES * 64;
+    constexpr int kKeyPieces = D / 8, kTileBytes = kKeyTile * D * 2, kPieces = kTileBytes / 16;
+    constexpr int kDepthSteps = D / 16, kOutTiles = D / 32;
+    static_assert(kPieces % kThreads == 0, "every thread moves whole pieces");
+    __shared__ alignas(16) unsigned char lds[2][2][kTileBytes];  // [buffer][keys, values]
+
+    const int H = s.num_attention_heads, KVH = s.num_kv_heads, seq = s.seq;
+    const int kv_head = blockIdx.x % KVH, batch = blockIdx.y, tiles = (seq + kQueries - 1) / kQueries;
+    // A tile's work grows with its position.  The first half of the blocks takes the heavy tiles in
+    // descending order, the second the light ones in ascending order: blocks that share a CU add up to the
+    // same work, and where there are more blocks than the chip holds, the light ones come last.
+    const int order = blockIdx.x / KVH, heavy = (tiles + 1) / 2;
+    const int tile = order < heavy ? tiles - 1 - order : order - heavy;
+    const int wave = (int)threadIdx.x / 64, lane = (int)threadIdx.x % 64, half = lane / 32;
+    const int head = kv_head * kGqa + wave % kGqa;
+    const int q_first = tile * kQueries + wave / kGqa * 32, q_at = q_first + lane % 32;
+    const int key_tiles = (min(tile * kQueries + kQueries, seq) + kKeyTile - 1) / kKeyTile;
+    const unsigned char *const key_src = (const unsigned char *)(keys + ((size_t)batch * KVH + kv_head) * padded * D);
+    const unsigned char *const value_src = (const unsigned char *)(values_t + ((size_t)batch * KVH + kv_head) * D * padded);
+
+    auto request = [&](int t, int buffer) {
+#pragma unroll
+        for (int i = 0; i < kPieces / kThreads; i++) {
+            const int wave_at = i * kThreads + wave * 64, at = wave_at + lane;
+            const int row = at / kKeyPieces, piece = (at % kKeyPieces) ^ (kKeyPieces == 8 ? (row >> 1) & 7 : row & 15);
+            load_to_lds(key_src + ((size_t)t * kKeyTile + row) * (D * 2) + piece * 16, (MK_LDS void *)&lds[buffer][0][wave_at * 16]);
+            const int vrow = at / 8, vpiece = (at % 8) ^ ((vrow >> 1) & 7);
+            load_to_lds(value_src + (size_t)vrow * padded * 2 + (size_t)t * (kKeyTile * 2) + vpiece * 16, (MK_LDS void *)&lds[buffer][1][wave_at * 16]);
+        }
+    };
+    request(0, 0);
+
+    bf16x8 query[kDepthSteps];
+    {
+        const uint16_t *const src = q + (((size_t)batch * seq + min(q_at, seq - 1)) * H + head) * D + half * 8;
+#pragma unroll
+        for (int i = 0; i < kDepthSteps; i++) query[i] = *(const bf16x8 *)(src + i * 16);
+    }
+    f32x16 acc[kOutTiles];
+#pragma unroll
+    for (int i = 0; i < kOutTiles; i++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) acc[i][r] = 0.0f;
+    float maximum = -INFINITY, sum = 0.0f;
+
+    for (int t = 0; t < key_tiles; t++) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (t + 1 < key_tiles) request(t + 1, (t + 1) & 1);
+        if (t * kKeyTile > q_first + 31) continue;  // wholly above the diagonal for this wave
+        const unsigned char *const key_tile = lds[t & 1][0], *const value_tile = lds[t & 1][1];
+
+        f32x16 score[2];
+#pragma unroll
+        for (int sub = 0; sub < 2; sub++) {
+#pragma unroll
+            for (int r = 0; r < 16; r++) score[sub][r] = 0.0f;
+            const int row = sub * 32 + lane % 32, swizzle = kKeyPieces == 8 ? (row >> 1) & 7 : row & 15;
+#pragma unroll
+            for (int i = 0; i < kDepthSteps; i++) {
+                const bf16x8 key = *(const bf16x8 *)(key_tile + row * (D * 2) + ((2 * i + half) ^ swizzle) * 16);
+                score[sub] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(key, query[i], score[sub], 0, 0, 0);
+            }
+        }
+        if (t * kKeyTile + kKeyTile - 1 > q_first) {
+#pragma unroll
+            for (int sub = 0; sub < 2; sub++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int key_at = t * kKeyTile + sub * 32 + 8 * (r / 4) + 4 * half + r % 4;
+                    if (key_at > q_at) score[sub][r] = -INFINITY;
+                }
+        }
+        float tile_max = score[0][0];
+#pragma unroll
+        for (int sub = 0; sub < 2; sub++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) tile_max = fmaxf(tile_max, score[sub][r]);
+        const float next = fmaxf(maximum, half_exchange_max(tile_max));
+        if (__any(next > maximum)) {
+            const float shrink = exp2f((maximum - next) * scale);
+            sum *= shrink;
+#pragma unroll
+            for (int i = 0; i < kOutTiles; i++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[i][r] *= shrink;
+            maximum = next;
+        }
+        const float offset = maximum * scale;
+        uint32_t prob[2][8];
+#pragma unroll
+        for (int sub = 0; sub < 2; sub++)
+#pragma unroll
+            for (int r = 0; r < 16; r += 2) {
+                const float a = __builtin_amdgcn_exp2f(fmaf(score[sub][r], scale, -offset));
+                const float b = __builtin_amdgcn_exp2f(fmaf(score[sub][r + 1], scale, -offset));
+                sum += a;
+                sum += b;
+                prob[sub][r / 2] = pack_bf16(a, b);
+            }
+#pragma unroll
+        for (int step = 0; step < 4; step++) {
+            const u32x4 words = {prob[step / 2][step % 2 * 4], prob[step / 2][step % 2 * 4 + 1], prob[step / 2][step % 2 * 4 + 2],
+                                 prob[step / 2][step % 2 * 4 + 3]};
+            const bf16x8 p = __builtin_bit_cast(bf16x8, words);
+#pragma unroll
+            for (int i = 0; i < kOutTiles; i++) {
+                const int row = i * 32 + lane % 32;
+                const bf16x8 value = *(const bf16x8 *)(value_tile + row * (kKeyTile * 2) + ((2 * step + half) ^ ((row >> 1) & 7)) * 16);
+                acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(value, p, acc[i], 0, 0, 0);
+            }
+        }
+    }
+    if (q_at >= seq) return;
+    const float inverse = 1.0f / half_exchange_sum(sum);
+    uint16_t *const dst = out + (((size_t)batch * seq + q_at) * H + head) * D;
+#pragma unroll
+    for (int i = 0; i < kOutTiles; i++)
+#pragma unroll
+        for (int g = 0; g < 4; g++) {
+            const u32x2 pairs = {pack_bf16(acc[i][4 * g] * inverse, acc[i][4 * g + 1] * inverse),
+                                 pack_bf16(acc[i][4 * g + 2] * inverse, acc[i][4 * g + 3] * inverse)};
+            *(u32x2 *)(dst + i * 32 + 8 * g + 4 * half) = pairs;
+        }
+}
+
+// ---------------------------------------------------------------------------------------------
+// SiLU(gate) * up, with the gate's activation narrowed to bf16 before the product.  Bound by memory.
+// ---------------------------------------------------------------------------------------------
+__device__ __forceinline__ float silu(float g) { return g / (1.0f + expf(-g)); }
+
+__global__ __launch_bounds__(256) void silu_mul_kernel(size_t pieces, const uint16_t *gate, const uint16_t *up, uint16_t *out) {
+    const size_t at = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (at >= pieces) return;
+    const u32x4 g = *(const u32x4 *)(gate + at * 8), u = *(const u32x4 *)(up + at * 8);
+    u32x4 o;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        o[j] = pack_bf16(round_bf16(silu(bf16_lo(g[j]))) * bf16_lo(u[j]), round_bf16(silu(bf16_hi(g[j]))) * bf16_hi(u[j]));
+    *(u32x4 *)(out + at * 8) = o;
+}
+
+// ---------------------------------------------------------------------------------------------
+// First maximum of every row of logits: the row's values as integers that order like the values, a NaN
+// above everything, with the complement of the index below them, so that the largest key is the answer.
+// ---------------------------------------------------------------------------------------------
+__device__ __forceinline__ uint32_t order_bits(uint32_t bf16) {
+    if ((bf16 & 0x7fffu) > 0x7f80u) return 0xffffu;
+    if (bf16 == 0x8000u) bf16 = 0;  // minus zero equals zero
+    return (bf16 & 0x8000u) ? ~bf16 & 0xffffu : bf16 | 0x8000u;
+}
+
+__global__ __launch_bounds__(1024) void argmax_kernel(int vocab, const uint16_t *logits, int64_t *ids) {
+    const uint16_t *const row = logits + (size_t)blockIdx.x * vocab;
+    uint64_t best = 0;
+    for (int at = (int)threadIdx.x; at < vocab / 8; at += 1024) {
+        const u32x4 v = *(const u32x4 *)(row + (size_t)at * 8);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const uint64_t key = (uint64_t)order_bits((v[j / 2] >> (j % 2 * 16)) & 0xffffu) << 32 | (uint32_t)~(uint32_t)(at * 8 + j);
+            best = key > best ? key : best;
+        }
+    }
+#pragma unroll
+    for (int offset = 32; offset >= 1; offset /= 2) {
+        const uint64_t other = __shfl_xor(best, offset);
+        best = other > best ? other : best;
+    }
+    __shared__ uint64_t of_wave[16];
+    if (threadIdx.x % 64 == 0) of_wave[threadIdx.x / 64] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 16; w++) best = of_wave[w] > best ? of_wave[w] : best;
+        ids[blockIdx.x] = (int64_t)(uint32_t)~(uint32_t)best;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// host side
+// ---------------------------------------------------------------------------------------------
+thread_local char g_error[256];
+
+int fail(int code, const char *format, ...) {
+    va_list args;
+    va_start(args, format);
+    vsnprintf(g_error, sizeof g_error, format, args);
+    va_end(args);
+    return code;
+}
+int launched(const char *what) {
+    const hipError_t e = hipGetLastError();
+    return e == hipSuccess ? 0 : fail(-5, "%s: %s", what, hipGetErrorString(e));
+}
+int check_shape(const mk_prefill_shape *s) {
+    if (!s) return fail(-1, "no shape");
+    if (s->batch < 1 || s->seq < 1 || s->batch > 65535 || (int64_t)s->batch * s->seq > (1 << 22)) return fail(-2, "batch %d x seq %d", s->batch, s->seq);
+    if (s->head_dim != 64 && s->head_dim != 128) return fail(-2, "head_dim %d: 64 or 128", s->head_dim);
+    if (s->num_kv_heads < 1 || s->num_attention_heads != 4 * s->num_kv_heads) return fail(-2, "four query heads per KV head");
+    if (s->hidden_size < 8 || s->hidden_size % 8 || s->hidden_size > kMaxHidden) return fail(-2, "hidden_size %d", s->hidden_size);
+    if (s->intermediate_size < 8 || s->intermediate_size % 8) return fail(-2, "intermediate_size %d", s->intermediate_size);
+    if (s->vocab_size < 8 || s->vocab_size % 8) return fail(-2, "vocab_size %d", s->vocab_size);
+    if (s->kv_max_len < 1 || s->rope_positions < 1) return fail(-2, "empty cache or rope table");
+    return 0;
+}
+int padded_seq(int seq) { return (seq + kPosTile - 1) / kPosTile * kPosTile; }
+
+template <int D>
+int launch_attention(const mk_prefill_shape &s, const uint16_t *q, const uint16_t *keys, const uint16_t *values_t, uint16_t *out, hipStream_t stream) {
+    const float scale = 1.44269504088896341f / sqrtf((float)D);
+    const int padded = padded_seq(s.seq);
+    // Eight waves share a tile's loads among 64 positions; four leave twice as many blocks, which matters
+    // while there is less than one block of eight per CU and half.
+    if ((int64_t)s.batch * s.num_kv_heads * ((s.seq + 63) / 64) >= 512) {
+        const dim3 grid((s.seq + 63) / 64 * s.num_kv_heads, s.batch);
+        attention_kernel<D, 8><<<grid, 512, 0, stream>>>(s, padded, scale, q, keys, values_t, out);
+    } else {
+        const dim3 grid((s.seq + 31) / 32 * s.num_kv_heads, s.batch);
+        attention_kernel<D, 4><<<grid, 256, 0, stream>>>(s, padded, scale, q, keys, values_t, out);
+    }
+    return launched("attention");
+}
+
+}  // namespace
+
+extern "C" {
+
+int mk_prefill_padded_seq(int seq) { return padded_seq(seq); }
+
+int mk_prefill_embed(const mk_prefill_shape *shape, const int64_t *ids, const int64_t *positions, const uint16_t *embed,
+                     const uint16_t *norm_weight, uint16_t *h, uint16_t *x, void *stream) {
+    if (int rc = check_shape(shape)) return rc;
+    norm_kernel<true><<<shape->batch * shape->seq, kNormThreads, 0, (hipStream_t)stream>>>(*shape, ids, positions, embed, norm_weight, h, x);
+    return launched("embed");
+}
+
+int mk_prefill_add_norm(const mk_prefill_shape *shape, const uint16_t *y, const uint16_t *norm_weight, uint16_t *h, uint16_t *x, void *stream) {
+    if (int rc = check_shape(shape)) return rc;
+    norm_kernel<false><<<shape->batch * shape->seq, kNormThreads, 0, (hipStream_t)stream>>>(*shape, nullptr, nullptr, y, norm_weight, h, x);
+    return launched("add_norm");
+}
+
+int mk_prefill_rope(const mk_prefill_shape *shape, const uint16_t *qkv, const int64_t *positions, const float *rope_cos,
+                    const float *rope_sin, uint16_t *k_cache, uint16_t *v_cache, uint16_t *q, uint16_t *keys,
+                    uint16_t *values_t, void *stream) {
+    if (int rc = check_shape(shape)) return rc;
+    const int padded = padded_seq(shape->seq);
+    const dim3 grid(padded / kPosTile, shape->num_attention_heads + 2 * shape->num_kv_heads, shape->batch);
+    auto *kernel = shape->head_dim == 64 ? rope_kernel<64> : rope_kernel<128>;
+    kernel<<<grid, 256, 0, (hipStream_t)stream>>>(*shape, padded, qkv, positions, rope_cos, rope_sin, k_cache, v_cache, q, keys, values_t);
+    return launched("rope");
+}
+
+int mk_prefill_attention(const mk_prefill_shape *shape, const uint16_t *q, const uint16_t *keys, const uint16_t *values_t,
+                         uint16_t *out, void *stream) {
+    if (int rc = check_shape(shape)) return rc;
+    return shape->head_dim == 64 ? launch_attention<64>(*shape, q, keys, values_t, out, (hipStream_t)stream)
+                                 : launch_attention<128>(*shape, q, keys, values_t, out, (hipStream_t)stream);
+}
+
+int mk_prefill_silu_mul(const mk_prefill_shape *shape, const uint16_t *gate, const uint16_t *up, uint16_t *out, void *stream) {
+    if (int rc = check_shape(shape)) return rc;
+    const size_t pieces = (size_t)shape->batch * shape->seq * shape->intermediate_size / 8;
+    silu_mul_kernel<<<(unsigned)((pieces + 255) / 256), 256, 0, (hipStream_t)stream>>>(pieces, gate, up, out);
+    return launched("silu_mul");
+}
+
+int mk_prefill_argmax(const mk_prefill_shape *shape, const uint16_t *logits, int64_t *ids, void *stream) {
+    if (int rc = check_shape(shape)) return rc;
+    argmax_kernel<<<shape->batch * shape->seq, 1024, 0, (hipStream_t)stream>>>(shape->vocab_size, logits, ids);
+    return launched("argmax");
+}
+
+const char *mk_prefill_last_error(void) { return g_error; }
+
+}  // extern "C"

@@ -32,6 +32,7 @@ import torch
 import torch.nn.functional as F
 from torch import Tensor
 
+from megakernels_amd import prefill
 from megakernels_amd.model_types import BatchState, DeviceType, ExtraModelConfig
 
 
@@ -478,6 +479,9 @@ class LlamaForCausalLM:
         if pos.ndim == 2:
             pos = pos[0]
         B, S = ids.shape
+        if prefill.covers(self, ids):
+            h, output_ids = prefill.forward(self, ids, pos)
+            return BatchState(input_ids=ids, position_ids=pos, seq_len=S, hidden_states=h, output_ids=output_ids)
         H, KVH, D = c.num_attention_heads, c.num_key_value_heads, c.head_dim
         cos, sin = self.model.rope_cos[pos], self.model.rope_sin[pos]
         rope = apply_rotary_pos_emb_interleaved if self.extra_config.interleave_rope else apply_rotary_pos_emb

@@ -1,0 +1,113 @@
+"""The prompt forward's HIP kernels against the plain PyTorch forward on the CPU: hidden states, cache rows and greedy
+ids, at the sizes where tiles, waves and position groups begin and end."""
+
+import math
+
+import pytest
+import torch
+
+from helpers import config_1b_slice, config_8b_slice, config_tiny
+from megakernels_amd import prefill
+from megakernels_amd.llama import LlamaForCausalLM, rms_norm
+from megakernels_amd.model_types import BatchState, ExtraModelConfig
+
+pytestmark = pytest.mark.gpu
+
+
+def _model(cfg, max_len, batch=1, interleave=True, seed=3):
+    model = LlamaForCausalLM.from_random(
+        cfg, ExtraModelConfig(interleave_rope=interleave, max_len_override=max_len, max_batch_size=batch), seed=seed)
+    model.model.embed_tokens.weight.mul_(50)   # unit embedding rows: attention over unlike positions
+    return model
+
+
+def _compare(cfg, seq, batch=1, interleave=True, positions=None, max_len=None):
+    print(f"prefill hidden={cfg.hidden_size} D={cfg.head_dim} seq={seq} batch={batch} interleave={interleave}", flush=True)
+    model = _model(cfg, max_len or seq + 3, batch, interleave)
+    model_gpu = model.to("cuda:0")
+    ids = torch.randint(0, cfg.vocab_size, (batch, seq), generator=torch.Generator().manual_seed(seq))
+    positions = torch.arange(seq) if positions is None else positions
+    assert prefill.covers(model_gpu, ids.to("cuda:0"))
+    ref = model(BatchState(input_ids=ids, position_ids=positions))
+    out = model_gpu(BatchState(input_ids=ids.to("cuda:0"), position_ids=positions.to("cuda:0")))
+    # Both forwards round to bf16 at the same points and sum in fp32 in different orders, so any of the dozen roundings
+    # of a layer may fall the other way: 2^-9 of a value each, independent of each other.
+    bound = math.sqrt(12 * cfg.num_hidden_layers) * 2.0**-9
+    for name, a, b in (("hidden", out.hidden_states, ref.hidden_states),
+                       ("k", model_gpu.stacked_kv_cache[0], model.stacked_kv_cache[0]),
+                       ("v", model_gpu.stacked_kv_cache[1], model.stacked_kv_cache[1])):
+        a, b = a.cpu().double(), b.double()
+        assert a.shape == b.shape and float((a - b).norm() / b.norm()) <= bound, name
+    # greedy ids: the chosen token's logit is the largest one up to what the hidden states differ by
+    x = rms_norm(ref.hidden_states, model.lm_head.input_norm.weight, cfg.rms_norm_eps).float()
+    logits = x @ model.lm_head.lm_head.weight.float().T
+    chosen = logits.gather(-1, out.output_ids.cpu()[..., None])[..., 0]
+    slack = 6 * bound * logits.std(dim=-1) + 2.0**-7 * logits.amax(-1).abs()
+    assert bool((chosen >= logits.amax(-1) - slack).all())
+    assert out.output_ids.shape == (batch, seq) and out.output_ids.dtype == torch.int64
+
+
+@pytest.mark.parametrize("seq", [2, 15, 31, 32, 33, 63, 64, 65, 127, 130, 257])
+def test_prefill_tiny(seq):
+    _compare(config_tiny(), seq)
+
+
+@pytest.mark.parametrize("seq", [5, 64, 193])
+def test_prefill_1b_layers(seq):
+    _compare(config_1b_slice(), seq)
+
+
+@pytest.mark.parametrize("seq", [33, 192])
+def test_prefill_8b_layer(seq):
+    _compare(config_8b_slice(), seq)
+
+
+@pytest.mark.parametrize("interleave", [True, False])
+def test_prefill_batch_and_both_rotary_layouts(interleave):
+    _compare(config_tiny(), 70, batch=3, interleave=interleave)
+    _compare(config_8b_slice(), 40, batch=2, interleave=interleave)
+
+
+def test_prefill_at_positions_out_of_order_and_from_the_end():
+    seq = 66
+    order = torch.randperm(100, generator=torch.Generator().manual_seed(1))[:seq]
+    _compare(config_tiny(), seq, positions=order, max_len=100)
+    # negative positions count from the end of the cache and of the rotary table
+    _compare(config_tiny(), seq, positions=torch.arange(seq) - seq, max_len=1024)
+
+
+def test_prefill_long_enough_for_blocks_of_eight_waves():
+    # 2 sequences x 2 KV heads x 128 tiles of 64 positions
+    cfg = config_tiny(layers=1)
+    cfg.max_position_embeddings = 8192
+    _compare(cfg, 64 * 127 + 5, batch=2)
+
+
+def test_argmax_takes_the_first_maximum_and_nan_above_all():
+    lib = prefill.load_library()
+    import ctypes
+
+    vocab = 1024
+    logits = torch.randn(5, vocab).to(torch.bfloat16)
+    logits[0] = -3.0
+    logits[1, [700, 9, 300]] = 50.0
+    logits[2, [40, 600]] = float("nan")
+    logits[3] = -float("inf")
+    logits[4] = -0.0
+    logits[4, 17] = 0.0
+    on_gpu = logits.to("cuda:0")
+    ids = torch.full((5,), -1, dtype=torch.int64, device="cuda:0")
+    shape = prefill.Shape(1, 5, 8, 2, 64, 512, 1024, vocab, 8, 8, 1, 1e-5)
+    assert lib.mk_prefill_argmax(ctypes.byref(shape), on_gpu.data_ptr(), ids.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    assert ids.cpu().tolist() == [0, 9, 40, 0, 0] == logits.argmax(-1).tolist()
+
+
+def test_shapes_outside_the_kernels_are_refused():
+    import ctypes
+
+    lib = prefill.load_library()
+    for field, value in (("head_dim", 96), ("num_attention_heads", 16), ("hidden_size", 516), ("seq", 0), ("vocab_size", 1001)):
+        shape = prefill.Shape(1, 5, 8, 2, 64, 512, 1024, 1024, 8, 8, 1, 1e-5)
+        setattr(shape, field, value)
+        assert lib.mk_prefill_argmax(ctypes.byref(shape), None, None, None) < 0
+        assert lib.mk_prefill_last_error()
