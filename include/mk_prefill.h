@@ -56,6 +56,21 @@ int mk_prefill_silu_mul(const mk_prefill_shape *shape, const uint16_t *gate, con
 /* ids[row] = index of the first maximum of logits[row, 0..vocab_size), a NaN counting as the largest value */
 int mk_prefill_argmax(const mk_prefill_shape *shape, const uint16_t *logits, int64_t *ids, void *stream);
 
+/* The weights and the cache of a model; matrices are [out, in], stacked over the layers. */
+typedef struct mk_prefill_model {
+    const uint16_t *embed, *attn_norm, *qkv, *o, *mlp_norm, *gate, *up, *down, *final_norm, *head;
+    const float *rope_cos, *rope_sin;
+    uint16_t *k_cache, *v_cache;                           /* [layers, cache_batch, kv_max_len, KVH, D] */
+    int32_t num_layers, cache_batch;
+} mk_prefill_model;
+
+/* The whole forward where batch * seq is small: matrix products included, all in kernels of this library.
+ * h [rows, hidden_size] becomes the hidden states, out_ids [rows] the greedy ids.  The workspace's size is
+ * mk_prefill_rows_workspace_bytes (0: too many rows, or widths that are no multiple of 64; negative: an error). */
+int64_t mk_prefill_rows_workspace_bytes(const mk_prefill_shape *shape);
+int mk_prefill_rows_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids,
+                            const int64_t *positions, uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream);
+
 const char *mk_prefill_last_error(void);
 
 #ifdef __cplusplus

@@ -18,6 +18,7 @@ namespace {
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -50,16 +51,21 @@ constexpr int kNormChunks = kMaxHidden / (8 * kNormThreads);  // 16-byte pieces 
 // position as an index of a table of `count` rows: negative ones count from the end
 __device__ __forceinline__ int64_t wrap_position(int64_t position, int count) { return position < 0 ? position + count : position; }
 
+// an id or a position outside its table aborts the kernel
+__device__ __forceinline__ void check_token(const mk_prefill_shape &s, int64_t id, int64_t position) {
+    const int64_t cache_row = wrap_position(position, s.kv_max_len), rope_row = wrap_position(position, s.rope_positions);
+    if (id < 0 || id >= s.vocab_size || cache_row < 0 || cache_row >= s.kv_max_len || rope_row < 0 || rope_row >= s.rope_positions)
+        __builtin_trap();
+}
+
 template <bool EMBED>
 __global__ __launch_bounds__(kNormThreads) void norm_kernel(mk_prefill_shape s, const int64_t *ids, const int64_t *positions,
                                                             const uint16_t *src, const uint16_t *weight, uint16_t *h, uint16_t *x) {
     const int row = blockIdx.x, hid = s.hidden_size, pieces = hid / 8;
     const uint16_t *add = src + (size_t)row * hid;
     if constexpr (EMBED) {
-        const int64_t id = ids[row], position = positions[row % s.seq];
-        const int64_t cache_row = wrap_position(position, s.kv_max_len), rope_row = wrap_position(position, s.rope_positions);
-        if (id < 0 || id >= s.vocab_size || cache_row < 0 || cache_row >= s.kv_max_len || rope_row < 0 || rope_row >= s.rope_positions)
-            __builtin_trap();
+        const int64_t id = ids[row];
+        check_token(s, id, positions[row % s.seq]);
         add = src + (size_t)id * hid;
     }
     uint16_t *const h_row = h + (size_t)row * hid;
@@ -367,6 +373,23 @@ __device__ __forceinline__ uint32_t order_bits(uint32_t bf16) {
     return (bf16 & 0x8000u) ? ~bf16 & 0xffffu : bf16 | 0x8000u;
 }
 
+// the block's largest key to ids[blockIdx.x], as an index
+template <int THREADS>
+__device__ __forceinline__ void write_best(uint64_t best, int64_t *ids) {
+#pragma unroll
+    for (int offset = 32; offset >= 1; offset /= 2) {
+        const uint64_t other = __shfl_xor(best, offset);
+        best = other > best ? other : best;
+    }
+    __shared__ uint64_t of_wave[THREADS / 64];
+    if (threadIdx.x % 64 == 0) of_wave[threadIdx.x / 64] = best;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < THREADS / 64; w++) best = of_wave[w] > best ? of_wave[w] : best;
+        ids[blockIdx.x] = (int64_t)(uint32_t)~(uint32_t)best;
+    }
+}
+
 __global__ __launch_bounds__(1024) void argmax_kernel(int vocab, const uint16_t *logits, int64_t *ids) {
     const uint16_t *const row = logits + (size_t)blockIdx.x * vocab;
     uint64_t best = 0;
@@ -378,19 +401,10 @@ __global__ __launch_bounds__(1024) void argmax_kernel(int vocab, const uint16_t 
             best = key > best ? key : best;
         }
     }
-#pragma unroll
-    for (int offset = 32; offset >= 1; offset /= 2) {
-        const uint64_t other = __shfl_xor(best, offset);
-        best = other > best ? other : best;
-    }
-    __shared__ uint64_t of_wave[16];
-    if (threadIdx.x % 64 == 0) of_wave[threadIdx.x / 64] = best;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < 16; w++) best = of_wave[w] > best ? of_wave[w] : best;
-        ids[blockIdx.x] = (int64_t)(uint32_t)~(uint32_t)best;
-    }
+    write_best<1024>(best, ids);
 }
+
+#include "mk_prefill_rows.h"
 
 // ---------------------------------------------------------------------------------------------
 // host side
@@ -437,9 +451,126 @@ int launch_attention(const mk_prefill_shape &s, const uint16_t *q, const uint16_
     return launched("attention");
 }
 
+// ---- few rows: the whole forward, products included ----
+
+// Blocks over which K is split.  A block reads all of X's rows once per column tile, so with a long K the 128 blocks of a
+// 2048-wide product spend their time on X: 32 rows, K = 8192: 16.4 us whole, 12.2 us as two tiles a block and K in four;
+// 4096 wide, K = 14336: 31.1 and 28.0.  The blocks' meeting costs 3 us, too much for a short K (K = 2048: 4.9 and 7.4).
+int rows_split(int k) { return k >= 6144 ? 4 : 1; }
+
+template <int MT, int NT, int WAVES, int STAGES, int EPI, bool NORM>
+int launch_rows(const RowsArgs &a, int split, const char *what, hipStream_t stream) {
+    const int width = EPI == kRowsSilu ? 16 : NT * 16, bytes = RowsLds<MT, NT, WAVES, STAGES, NORM>::bytes(a.k);
+    auto *kernel = rows_kernel<MT, NT, WAVES, STAGES, EPI, NORM>;
+    const hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) return fail(-5, "%s: %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
+    kernel<<<dim3((a.n + width - 1) / width, split), WAVES * 64, bytes, stream>>>(a);
+    return launched(what);
+}
+// Two tiles a block: two or three blocks of four waves fit a CU, and one's meeting is hidden by the others' loads.
+template <int MT, int EPI, bool NORM>
+int launch_rows_wide(const RowsArgs &a, int split, const char *what, hipStream_t stream) {
+    return launch_rows<MT, 2, 4, MT == 4 ? 1 : 2, EPI, NORM>(a, split, what, stream);
+}
+// One tile a block: where there is at most one block per CU it has eight waves, so that the CU has enough loads in flight.
+template <int MT, int EPI, bool NORM>
+int launch_rows_narrow(const RowsArgs &a, const char *what, hipStream_t stream) {
+    if constexpr (!NORM)
+        if (rows_split(a.k) > 1) return launch_rows_wide<MT, EPI, NORM>(a, rows_split(a.k), what, stream);
+    if (a.n / 16 <= 256) return launch_rows<MT, 1, 8, MT == 4 ? 1 : 2, EPI, NORM>(a, 1, what, stream);
+    return launch_rows<MT, 1, 4, 1, EPI, NORM>(a, 1, what, stream);
+}
+template <int NT, int EPI, bool NORM>
+int launch_rows(const RowsArgs &a, const char *what, hipStream_t stream) {
+    if constexpr (NT == 1) {
+        if (a.rows <= 16) return launch_rows_narrow<1, EPI, NORM>(a, what, stream);
+        if (a.rows <= 32) return launch_rows_narrow<2, EPI, NORM>(a, what, stream);
+        return launch_rows_narrow<4, EPI, NORM>(a, what, stream);
+    } else {
+        if (a.rows <= 16) return launch_rows_wide<1, EPI, NORM>(a, 1, what, stream);
+        if (a.rows <= 32) return launch_rows_wide<2, EPI, NORM>(a, 1, what, stream);
+        return launch_rows_wide<4, EPI, NORM>(a, 1, what, stream);
+    }
+}
+
+// the workspace of the forward for few rows, in elements of 2 bytes; every part a multiple of 16 bytes
+struct RowsWorkspace {
+    size_t q, attn, prod, keys, values_t, arrived, best, partial, total;  // values_t and arrived: zero at the start
+    explicit RowsWorkspace(const mk_prefill_shape &s) {
+        const size_t rows = (size_t)s.batch * s.seq, heads = rows * s.num_attention_heads * s.head_dim;
+        const size_t kv = (size_t)s.batch * s.num_kv_heads * s.head_dim * padded_seq(s.seq);
+        q = 0;
+        attn = q + heads;
+        prod = attn + heads;
+        keys = prod + rows * s.intermediate_size;
+        values_t = keys + kv;
+        arrived = values_t + kv;
+        best = arrived + (s.hidden_size / 32 + 3) / 4 * 4 * 2;
+        partial = best + rows * ((s.vocab_size + 31) / 32 + 1) / 2 * 2 * 4;
+        const size_t sums = (rows <= 16 ? 16 : rows <= 32 ? 32 : 64) * (size_t)s.hidden_size;  // of one part of K
+        const int split = max(rows_split(s.intermediate_size), rows_split(s.num_attention_heads * s.head_dim));
+        total = partial + (split > 1 ? split * sums * 2 : 0);
+    }
+};
+bool rows_covers(const mk_prefill_shape &s) {
+    return (int64_t)s.batch * s.seq <= kRowsMax && s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0;
+}
+
 }  // namespace
 
 extern "C" {
+
+int64_t mk_prefill_rows_workspace_bytes(const mk_prefill_shape *shape) {
+    if (int rc = check_shape(shape)) return rc;
+    return rows_covers(*shape) ? (int64_t)RowsWorkspace(*shape).total * 2 : 0;
+}
+
+int mk_prefill_rows_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids, const int64_t *positions,
+                            uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream_) {
+    if (int rc = check_shape(shape)) return rc;
+    const mk_prefill_shape &s = *shape;
+    if (!rows_covers(s)) return fail(-2, "%d x %d rows of %d, %d: more than the forward for few rows takes", s.batch, s.seq, s.hidden_size, s.intermediate_size);
+    if (!model || model->num_layers < 1 || model->cache_batch < s.batch) return fail(-2, "no layers, or a cache of fewer sequences than the call");
+    hipStream_t stream = (hipStream_t)stream_;
+    const mk_prefill_model &w = *model;
+    const RowsWorkspace at(s);
+    const int rows = s.batch * s.seq, H = s.num_attention_heads, KVH = s.num_kv_heads, D = s.head_dim, hid = s.hidden_size, inter = s.intermediate_size;
+    uint16_t *const q = workspace + at.q, *const attn = workspace + at.attn, *const prod = workspace + at.prod;
+    uint16_t *const keys = workspace + at.keys, *const values_t = workspace + at.values_t;
+    uint64_t *const best = (uint64_t *)(workspace + at.best);
+
+    const int value_pieces = (int)((at.best - at.values_t) / 8);  // with the arrivals behind them
+    rows_embed_kernel<<<rows + (value_pieces + 1023) / 1024, 256, 0, stream>>>(s, rows, ids, positions, w.embed, h, (u32x4 *)values_t, value_pieces);
+    if (int rc = launched("embed")) return rc;
+
+    RowsArgs base{};
+    base.s = s, base.rows = rows, base.padded = padded_seq(s.seq), base.positions = positions;
+    base.rope_cos = w.rope_cos, base.rope_sin = w.rope_sin, base.keys = keys, base.values_t = values_t, base.best = best;
+    base.arrived = (int *)(workspace + at.arrived), base.partial = (float *)(workspace + at.partial);
+    const size_t qkv_rows = (size_t)(H + 2 * KVH) * D, cache_layer = (size_t)w.cache_batch * s.kv_max_len * KVH * D;
+    for (int layer = 0; layer < w.num_layers; layer++) {
+        RowsArgs a = base;
+        a.n = (int)qkv_rows, a.k = hid, a.x = h, a.norm_weight = w.attn_norm + (size_t)layer * hid, a.w0 = w.qkv + layer * qkv_rows * hid, a.out = q;
+        a.k_cache = w.k_cache + layer * cache_layer, a.v_cache = w.v_cache + layer * cache_layer;
+        if (int rc = launch_rows<1, kRowsRope, true>(a, "qkv", stream)) return rc;
+        if (int rc = mk_prefill_attention(shape, q, keys, values_t, attn, stream)) return rc;
+        a = base;
+        a.n = hid, a.k = H * D, a.x = attn, a.w0 = w.o + (size_t)layer * hid * H * D, a.out = h;
+        if (int rc = launch_rows<1, kRowsResidual, false>(a, "o", stream)) return rc;
+        a = base;
+        a.n = inter, a.k = hid, a.x = h, a.norm_weight = w.mlp_norm + (size_t)layer * hid, a.out = prod;
+        a.w0 = w.gate + (size_t)layer * inter * hid, a.w1 = w.up + (size_t)layer * inter * hid;
+        if (int rc = launch_rows<2, kRowsSilu, true>(a, "gate and up", stream)) return rc;
+        a = base;
+        a.n = hid, a.k = inter, a.x = prod, a.w0 = w.down + (size_t)layer * hid * inter, a.out = h;
+        if (int rc = launch_rows<1, kRowsResidual, false>(a, "down", stream)) return rc;
+    }
+    RowsArgs a = base;
+    a.n = s.vocab_size, a.k = hid, a.x = h, a.norm_weight = w.final_norm, a.w0 = w.head;
+    if (int rc = launch_rows<2, kRowsArgmax, true>(a, "head", stream)) return rc;
+    rows_best_kernel<<<rows, 256, 0, stream>>>((s.vocab_size + 31) / 32, best, out_ids);
+    return launched("best");
+}
 
 int mk_prefill_padded_seq(int seq) { return padded_seq(seq); }
 

@@ -479,7 +479,7 @@ class LlamaForCausalLM:
         if pos.ndim == 2:
             pos = pos[0]
         B, S = ids.shape
-        if prefill.covers(self, ids):
+        if prefill.covers(self, ids, pos):
             h, output_ids = prefill.forward(self, ids, pos)
             return BatchState(input_ids=ids, position_ids=pos, seq_len=S, hidden_states=h, output_ids=output_ids)
         H, KVH, D = c.num_attention_heads, c.num_key_value_heads, c.head_dim

@@ -28,6 +28,14 @@ class Shape(ctypes.Structure):
         "kv_max_len", "rope_positions", "interleaved")] + [("rms_norm_eps", ctypes.c_float)]
 
 
+class Model(ctypes.Structure):
+    """``mk_prefill_model`` of ``include/mk_prefill.h``."""
+
+    _fields_ = [(n, _P) for n in (
+        "embed", "attn_norm", "qkv", "o", "mlp_norm", "gate", "up", "down", "final_norm", "head", "rope_cos", "rope_sin",
+        "k_cache", "v_cache")] + [("num_layers", _I), ("cache_batch", _I)]
+
+
 _POINTERS = {"embed": 6, "add_norm": 4, "rope": 9, "attention": 4, "silu_mul": 3, "argmax": 2}
 _lib = None
 
@@ -42,20 +50,38 @@ def load_library():
             function = getattr(lib, f"mk_prefill_{name}")
             function.argtypes = [ctypes.POINTER(Shape)] + [_P] * (count + 1)  # ... and the stream
             function.restype = ctypes.c_int
+        lib.mk_prefill_rows_workspace_bytes.argtypes = [ctypes.POINTER(Shape)]
+        lib.mk_prefill_rows_workspace_bytes.restype = ctypes.c_int64
+        lib.mk_prefill_rows_forward.argtypes = [ctypes.POINTER(Shape), ctypes.POINTER(Model)] + [_P] * 6
+        lib.mk_prefill_rows_forward.restype = ctypes.c_int
         lib.mk_prefill_last_error.restype = ctypes.c_char_p
         _lib = lib
     return _lib
 
 
-def covers(model, ids: Tensor) -> bool:
-    """Whether the HIP forward takes this call: more than one position per sequence, bf16 weights on the GPU, and an
-    architecture its kernels are built for (head_dim 64 or 128, four query heads per KV head, widths in 16-byte pieces).
-    Everything else runs through the plain PyTorch forward."""
+def _tensors(model) -> list[Tensor]:
+    """The model's bf16 tensors in the order of ``Model``, the rope tables left out."""
+    p = model.stacked_params
+    return [model.model.embed_tokens.weight, p.attn_ln_weight, p.qkv_proj, p.o_proj, p.mlp_ln_weight, p.gate_proj, p.up_proj,
+            p.down_proj, model.lm_head.input_norm.weight, model.lm_head.lm_head.weight, *model.stacked_kv_cache]
+
+
+def covers(model, ids: Tensor, positions: Tensor) -> bool:
+    """Whether the HIP forward takes this call: more than one position per sequence, bf16 weights on the GPU in the layout
+    that the model's constructors make, and an architecture its kernels are built for (head_dim 64 or 128, four query heads
+    per KV head, widths in 16-byte pieces).  Everything else runs through the plain PyTorch forward, which also says what
+    is wrong with indices of another type or shape."""
     c = model.config
-    return (ids.is_cuda and ids.shape[-1] > 1 and ids.device == model.device and model.dtype == torch.bfloat16
+    index = (torch.int64, torch.int32)
+    rope = (model.model.rope_cos, model.model.rope_sin)
+    return (ids.is_cuda and ids.shape[-1] > 1 and ids.device == model.device and ids.dtype in index and positions.dtype in index
+            and positions.shape == ids.shape[1:] and 0 < ids.shape[0] <= model.stacked_kv_cache[0].shape[1]
+            and ids.shape[0] <= 65535 and ids.numel() <= 1 << 22
             and c.head_dim in (64, 128) and c.num_attention_heads == 4 * c.num_key_value_heads
             and c.hidden_size % 8 == 0 and c.hidden_size <= 8192 and c.intermediate_size % 8 == 0 and c.vocab_size % 8 == 0
-            and model.model.rope_cos.dtype == torch.float32)
+            and all(t.dtype == torch.bfloat16 and t.device == ids.device and t.is_contiguous() and t.data_ptr() % 16 == 0
+                    for t in _tensors(model))
+            and all(t.dtype == torch.float32 and t.device == ids.device and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in rope))
 
 
 def forward(model, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
@@ -67,12 +93,15 @@ def forward(model, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
     H, KVH, D = c.num_attention_heads, c.num_key_value_heads, c.head_dim
     device = ids.device
     k_cache, v_cache = model.stacked_kv_cache
-    if B > k_cache.shape[1] or positions.shape != (S,):
-        raise RuntimeError(f"{B} sequences of {S} tokens at positions {tuple(positions.shape)} do not fit the cache {tuple(k_cache.shape)}")
     ids = ids.to(torch.int64).contiguous()
     positions = positions.to(device=device, dtype=torch.int64).contiguous()
     shape = Shape(B, S, H, KVH, D, c.hidden_size, c.intermediate_size, c.vocab_size, k_cache.shape[2],
                   model.model.rope_cos.shape[0], int(bool(model.extra_config.interleave_rope)), c.rms_norm_eps)
+    workspace_bytes = lib.mk_prefill_rows_workspace_bytes(ctypes.byref(shape))
+    if workspace_bytes < 0:
+        raise RuntimeError(f"mk_prefill_rows_workspace_bytes: {lib.mk_prefill_last_error().decode()}")
+    if workspace_bytes:
+        return _forward_rows(lib, model, shape, workspace_bytes, ids, positions)
     padded = lib.mk_prefill_padded_seq(S)
 
     def rows(width):
@@ -100,4 +129,22 @@ def forward(model, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
             norm = model.lm_head.input_norm.weight if last else p.attn_ln_weight[layer + 1]
             call("add_norm", F.linear(prod, p.down_proj[layer]), norm, h, x)
         call("argmax", F.linear(x, model.lm_head.lm_head.weight), out_ids)
+    return h, out_ids
+
+
+def _forward_rows(lib, model, shape, workspace_bytes: int, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
+    """A prompt of few positions: one call launches the whole forward, matrix products included.  Issued one by one from
+    Python, its launches took longer than the GPU needs for them."""
+    c, device = model.config, ids.device
+    *weights, k_cache, v_cache = (t.data_ptr() for t in _tensors(model))
+    pointers = Model(*weights, model.model.rope_cos.data_ptr(), model.model.rope_sin.data_ptr(), k_cache, v_cache,
+                     c.num_hidden_layers, model.stacked_kv_cache[0].shape[1])
+    h = torch.empty(*ids.shape, c.hidden_size, dtype=torch.bfloat16, device=device)
+    workspace = torch.empty(workspace_bytes, dtype=torch.uint8, device=device)
+    out_ids = torch.empty(ids.shape, dtype=torch.int64, device=device)
+    with torch.cuda.device(device):
+        stream = torch.cuda.current_stream(device).cuda_stream
+        if lib.mk_prefill_rows_forward(ctypes.byref(shape), ctypes.byref(pointers), ids.data_ptr(), positions.data_ptr(), h.data_ptr(),
+                                       workspace.data_ptr(), out_ids.data_ptr(), stream) != 0:
+            raise RuntimeError(f"mk_prefill_rows_forward: {lib.mk_prefill_last_error().decode()}")
     return h, out_ids
