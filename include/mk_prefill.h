@@ -64,11 +64,11 @@ typedef struct mk_prefill_model {
     int32_t num_layers, cache_batch;
 } mk_prefill_model;
 
-/* The whole forward where batch * seq is small: matrix products included, all in kernels of this library.
+/* The whole forward where batch * seq is not too large: matrix products included, all in kernels of this library.
  * h [rows, hidden_size] becomes the hidden states, out_ids [rows] the greedy ids.  The workspace's size is
- * mk_prefill_rows_workspace_bytes (0: too many rows, or widths that are no multiple of 64; negative: an error). */
-int64_t mk_prefill_rows_workspace_bytes(const mk_prefill_shape *shape);
-int mk_prefill_rows_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids,
+ * mk_prefill_workspace_bytes (0: too many rows, or widths that are no multiple of 64; negative: an error). */
+int64_t mk_prefill_workspace_bytes(const mk_prefill_shape *shape);
+int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids,
                             const int64_t *positions, uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream);
 
 const char *mk_prefill_last_error(void);

@@ -10,6 +10,7 @@
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
+#include <type_traits>
 
 #include "../../include/mk_prefill.h"
 
@@ -58,12 +59,14 @@ __device__ __forceinline__ void check_token(const mk_prefill_shape &s, int64_t i
         __builtin_trap();
 }
 
-template <bool EMBED>
+enum NormSource { kNormAdd, kNormEmbed, kNormPlain };  // h += src; h = embed row; h as it is
+
+template <NormSource SOURCE>
 __global__ __launch_bounds__(kNormThreads) void norm_kernel(mk_prefill_shape s, const int64_t *ids, const int64_t *positions,
                                                             const uint16_t *src, const uint16_t *weight, uint16_t *h, uint16_t *x) {
     const int row = blockIdx.x, hid = s.hidden_size, pieces = hid / 8;
     const uint16_t *add = src + (size_t)row * hid;
-    if constexpr (EMBED) {
+    if constexpr (SOURCE == kNormEmbed) {
         const int64_t id = ids[row];
         check_token(s, id, positions[row % s.seq]);
         add = src + (size_t)id * hid;
@@ -75,13 +78,13 @@ __global__ __launch_bounds__(kNormThreads) void norm_kernel(mk_prefill_shape s, 
     for (int i = 0; i < kNormChunks; i++) {
         const int at = (int)threadIdx.x + i * kNormThreads;
         if (at >= pieces) break;
-        v[i] = *(const u32x4 *)(add + (size_t)at * 8);
-        if constexpr (!EMBED) {
+        v[i] = *(const u32x4 *)((SOURCE == kNormPlain ? h_row : add) + (size_t)at * 8);
+        if constexpr (SOURCE == kNormAdd) {
             const u32x4 old = *(const u32x4 *)(h_row + (size_t)at * 8);
 #pragma unroll
             for (int j = 0; j < 4; j++) v[i][j] = pack_bf16(bf16_lo(old[j]) + bf16_lo(v[i][j]), bf16_hi(old[j]) + bf16_hi(v[i][j]));
         }
-        *(u32x4 *)(h_row + (size_t)at * 8) = v[i];
+        if constexpr (SOURCE != kNormPlain) *(u32x4 *)(h_row + (size_t)at * 8) = v[i];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const float lo = bf16_lo(v[i][j]), hi = bf16_hi(v[i][j]);
@@ -408,6 +411,7 @@ __global__ __launch_bounds__(1024) void argmax_kernel(int vocab, const uint16_t 
 }
 
 #include "mk_prefill_rows.h"
+#include "mk_prefill_tiles.h"
 
 // ---------------------------------------------------------------------------------------------
 // host side
@@ -515,64 +519,131 @@ struct RowsWorkspace {
         total = partial + (split > 1 ? split * sums * 2 : 0);
     }
 };
-bool rows_covers(const mk_prefill_shape &s) {
-    return (int64_t)s.batch * s.seq <= kRowsMax && s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0;
+// Whether the whole forward is this library's, products included.  Not for more than 2048 columns of hidden state: the
+// models that are wider are also deeper, and there another order of a product's sums, though as close to the forward
+// without roundings (1.56 % of the hidden states' norm at 4096 columns and 32 layers, either way), moves what is decoded
+// behind a short prompt by 2.8 to 3.1 % of its norm, more than one forward may differ from another.
+bool whole_covers(const mk_prefill_shape &s) {
+    return s.hidden_size <= 2048 && s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0;
 }
+bool rows_covers(const mk_prefill_shape &s) { return whole_covers(s) && (int64_t)s.batch * s.seq <= kRowsMax; }
+// From some thousand rows on the library's products are the faster ones (whole forwards of 16 layers, 2048 wide, library and
+// tiles, us: 253 rows 2241 and 1783, 777 rows 3431 and 3170, 1024 rows 3695 and 3550, 1500 rows 4713 and 5249).
+bool tiles_cover(const mk_prefill_shape &s) { return whole_covers(s) && (int64_t)s.batch * s.seq * s.hidden_size <= 1 << 21; }
+
+// ---- more rows: tiles ----
+
+// The shapes a product can be tiled in, with what a stage of 64 elements of K takes (us, measured with as many blocks as
+// there are slots) and how many blocks the chip holds at once.
+struct TileShape {
+    int rows, columns, slots;
+    float stage_us;
+};
+constexpr TileShape kTileShapes[] = {
+    {64, 128, 256, 0.42f},   // four stages in LDS: the least time for one tile
+    {128, 128, 256, 0.62f},  // four stages
+    {128, 128, 512, 1.05f},  // two stages, two blocks a CU
+    {256, 256, 256, 1.72f},  // the most work per byte of LDS: 1.23 PFLOP/s over whole rounds
+};
+struct TilePlan {
+    int shape, split, m_tiles, n_tiles;
+    float us;
+};
+// The plan with the least estimated time: rounds of blocks, 3 us to start and end, and for a split of K the blocks' meeting
+// and their sums' way through memory.  (rows 253: 2048 x 8192 estimated 25, measured 24.3 in 64 x 128 x 4 parts against
+// 52.9 whole; rows 777: 16384 x 2048 58 and 56.8 in 256 x 256 against 70.4 in 128 x 128.)  `columns`: gate's and up's
+// together for SiLU; `whole`: the epilogue takes no split.
+TilePlan tile_plan(int rows, int columns, int k, bool whole) {
+    TilePlan best{};
+    for (int shape = 0; shape < 4; shape++) {
+        const TileShape &t = kTileShapes[shape];
+        const int m_tiles = (rows + t.rows - 1) / t.rows, n_tiles = (columns + t.columns - 1) / t.columns, stages = k / kTileK;
+        for (int split = 1; split <= 8; split *= 2) {
+            if (split > 1 && (whole || stages / split < 8 || t.rows == 256)) break;
+            const int64_t rounds = ((int64_t)m_tiles * n_tiles * split + t.slots - 1) / t.slots;
+            const float meeting = split > 1 ? 3.0f + (float)split * rows * columns * 8 / 3e6f : 0.0f;
+            const float us = (float)rounds * ((stages + split - 1) / split) * t.stage_us + 3.0f + meeting;
+            if (best.split == 0 || us < best.us) best = {shape, split, m_tiles, n_tiles, us};
+        }
+    }
+    return best;
+}
+
+template <int WN, int MT, int STAGES, int EPI>
+int launch_tiles(const TileArgs &a, const TilePlan &plan, const char *what, hipStream_t stream) {
+    constexpr int bytes = STAGES * (MT * 64 + WN * 64) * kTileK * 2;
+    auto *kernel = tile_kernel<WN, MT, 2, STAGES, EPI>;
+    const hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    if (e != hipSuccess) return fail(-5, "%s: %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
+    kernel<<<dim3(8 * ((plan.n_tiles + 7) / 8) * plan.m_tiles, plan.split), WN * 128, bytes, stream>>>(a);
+    return launched(what);
+}
+template <int EPI>
+int launch_tiles(const TileArgs &a, const char *what, hipStream_t stream) {
+    const TilePlan plan = tile_plan(a.rows, EPI == kTileSilu ? 2 * a.n : a.n, a.k, EPI == kTileSilu || EPI == kTileArgmax);
+    switch (plan.shape) {
+    case 0: return launch_tiles<2, 1, 4, EPI>(a, plan, what, stream);
+    case 1: return launch_tiles<2, 2, 4, EPI>(a, plan, what, stream);
+    case 2: return launch_tiles<2, 2, 2, EPI>(a, plan, what, stream);
+    default: return launch_tiles<4, 4, 2, EPI>(a, plan, what, stream);
+    }
+}
+
+// The workspace, in elements of 2 bytes, as in RowsWorkspace.
+struct TilesWorkspace {
+    size_t x, q, attn, prod, keys, values_t, arrived, best, partial, total;
+    explicit TilesWorkspace(const mk_prefill_shape &s) {
+        const size_t rows = (size_t)s.batch * s.seq, heads = rows * s.num_attention_heads * s.head_dim;
+        const size_t kv = (size_t)s.batch * s.num_kv_heads * s.head_dim * padded_seq(s.seq);
+        x = 0;
+        q = x + rows * s.hidden_size;
+        attn = q + heads;
+        prod = attn + heads;
+        keys = prod + rows * s.intermediate_size;
+        values_t = keys + kv;
+        arrived = values_t + kv;
+        size_t counters = 0, sums = 0;
+        const int qkv = (s.num_attention_heads + 2 * s.num_kv_heads) * s.head_dim, products[3][2] = {
+            {qkv, s.hidden_size}, {s.hidden_size, s.num_attention_heads * s.head_dim}, {s.hidden_size, s.intermediate_size}};
+        for (const auto &nk : products) {
+            const TilePlan plan = tile_plan((int)rows, nk[0], nk[1], false);
+            if (plan.split == 1) continue;
+            const size_t tiles = (size_t)plan.m_tiles * plan.n_tiles;
+            counters = max(counters, tiles);
+            sums = max(sums, tiles * plan.split * kTileShapes[plan.shape].rows * kTileShapes[plan.shape].columns);
+        }
+        best = arrived + (counters + 3) / 4 * 4 * 2;
+        partial = best + ((s.vocab_size + 255) / 256 * 4 * rows + 1) / 2 * 2 * 4;
+        total = partial + sums * 2;
+    }
+};
+
+__global__ __launch_bounds__(256) void zero_kernel(u32x4 *dst, int pieces) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < pieces; i += gridDim.x * 256) dst[i] = u32x4{0, 0, 0, 0};
+}
+
+int rows_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const int64_t *ids, const int64_t *positions, uint16_t *h,
+                 uint16_t *workspace, int64_t *out_ids, hipStream_t stream);
+int tiles_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const int64_t *ids, const int64_t *positions, uint16_t *h,
+                  uint16_t *workspace, int64_t *out_ids, hipStream_t stream);
 
 }  // namespace
 
 extern "C" {
 
-int64_t mk_prefill_rows_workspace_bytes(const mk_prefill_shape *shape) {
+int64_t mk_prefill_workspace_bytes(const mk_prefill_shape *shape) {
     if (int rc = check_shape(shape)) return rc;
-    return rows_covers(*shape) ? (int64_t)RowsWorkspace(*shape).total * 2 : 0;
+    if (rows_covers(*shape)) return (int64_t)RowsWorkspace(*shape).total * 2;
+    return tiles_cover(*shape) ? (int64_t)TilesWorkspace(*shape).total * 2 : 0;
 }
 
-int mk_prefill_rows_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids, const int64_t *positions,
-                            uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream_) {
+int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids, const int64_t *positions,
+                       uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream) {
     if (int rc = check_shape(shape)) return rc;
-    const mk_prefill_shape &s = *shape;
-    if (!rows_covers(s)) return fail(-2, "%d x %d rows of %d, %d: more than the forward for few rows takes", s.batch, s.seq, s.hidden_size, s.intermediate_size);
-    if (!model || model->num_layers < 1 || model->cache_batch < s.batch) return fail(-2, "no layers, or a cache of fewer sequences than the call");
-    hipStream_t stream = (hipStream_t)stream_;
-    const mk_prefill_model &w = *model;
-    const RowsWorkspace at(s);
-    const int rows = s.batch * s.seq, H = s.num_attention_heads, KVH = s.num_kv_heads, D = s.head_dim, hid = s.hidden_size, inter = s.intermediate_size;
-    uint16_t *const q = workspace + at.q, *const attn = workspace + at.attn, *const prod = workspace + at.prod;
-    uint16_t *const keys = workspace + at.keys, *const values_t = workspace + at.values_t;
-    uint64_t *const best = (uint64_t *)(workspace + at.best);
-
-    const int value_pieces = (int)((at.best - at.values_t) / 8);  // with the arrivals behind them
-    rows_embed_kernel<<<rows + (value_pieces + 1023) / 1024, 256, 0, stream>>>(s, rows, ids, positions, w.embed, h, (u32x4 *)values_t, value_pieces);
-    if (int rc = launched("embed")) return rc;
-
-    RowsArgs base{};
-    base.s = s, base.rows = rows, base.padded = padded_seq(s.seq), base.positions = positions;
-    base.rope_cos = w.rope_cos, base.rope_sin = w.rope_sin, base.keys = keys, base.values_t = values_t, base.best = best;
-    base.arrived = (int *)(workspace + at.arrived), base.partial = (float *)(workspace + at.partial);
-    const size_t qkv_rows = (size_t)(H + 2 * KVH) * D, cache_layer = (size_t)w.cache_batch * s.kv_max_len * KVH * D;
-    for (int layer = 0; layer < w.num_layers; layer++) {
-        RowsArgs a = base;
-        a.n = (int)qkv_rows, a.k = hid, a.x = h, a.norm_weight = w.attn_norm + (size_t)layer * hid, a.w0 = w.qkv + layer * qkv_rows * hid, a.out = q;
-        a.k_cache = w.k_cache + layer * cache_layer, a.v_cache = w.v_cache + layer * cache_layer;
-        if (int rc = launch_rows<1, kRowsRope, true>(a, "qkv", stream)) return rc;
-        if (int rc = mk_prefill_attention(shape, q, keys, values_t, attn, stream)) return rc;
-        a = base;
-        a.n = hid, a.k = H * D, a.x = attn, a.w0 = w.o + (size_t)layer * hid * H * D, a.out = h;
-        if (int rc = launch_rows<1, kRowsResidual, false>(a, "o", stream)) return rc;
-        a = base;
-        a.n = inter, a.k = hid, a.x = h, a.norm_weight = w.mlp_norm + (size_t)layer * hid, a.out = prod;
-        a.w0 = w.gate + (size_t)layer * inter * hid, a.w1 = w.up + (size_t)layer * inter * hid;
-        if (int rc = launch_rows<2, kRowsSilu, true>(a, "gate and up", stream)) return rc;
-        a = base;
-        a.n = hid, a.k = inter, a.x = prod, a.w0 = w.down + (size_t)layer * hid * inter, a.out = h;
-        if (int rc = launch_rows<1, kRowsResidual, false>(a, "down", stream)) return rc;
-    }
-    RowsArgs a = base;
-    a.n = s.vocab_size, a.k = hid, a.x = h, a.norm_weight = w.final_norm, a.w0 = w.head;
-    if (int rc = launch_rows<2, kRowsArgmax, true>(a, "head", stream)) return rc;
-    rows_best_kernel<<<rows, 256, 0, stream>>>((s.vocab_size + 31) / 32, best, out_ids);
-    return launched("best");
+    if (!model || model->num_layers < 1 || model->cache_batch < shape->batch) return fail(-2, "no layers, or a cache of fewer sequences than the call");
+    if (rows_covers(*shape)) return rows_forward(*shape, *model, ids, positions, h, workspace, out_ids, (hipStream_t)stream);
+    if (tiles_cover(*shape)) return tiles_forward(*shape, *model, ids, positions, h, workspace, out_ids, (hipStream_t)stream);
+    return fail(-2, "%d x %d rows of %d, %d: not a call that the whole forward takes", shape->batch, shape->seq, shape->hidden_size, shape->intermediate_size);
 }
 
 int mk_prefill_padded_seq(int seq) { return padded_seq(seq); }
@@ -580,13 +651,13 @@ int mk_prefill_padded_seq(int seq) { return padded_seq(seq); }
 int mk_prefill_embed(const mk_prefill_shape *shape, const int64_t *ids, const int64_t *positions, const uint16_t *embed,
                      const uint16_t *norm_weight, uint16_t *h, uint16_t *x, void *stream) {
     if (int rc = check_shape(shape)) return rc;
-    norm_kernel<true><<<shape->batch * shape->seq, kNormThreads, 0, (hipStream_t)stream>>>(*shape, ids, positions, embed, norm_weight, h, x);
+    norm_kernel<kNormEmbed><<<shape->batch * shape->seq, kNormThreads, 0, (hipStream_t)stream>>>(*shape, ids, positions, embed, norm_weight, h, x);
     return launched("embed");
 }
 
 int mk_prefill_add_norm(const mk_prefill_shape *shape, const uint16_t *y, const uint16_t *norm_weight, uint16_t *h, uint16_t *x, void *stream) {
     if (int rc = check_shape(shape)) return rc;
-    norm_kernel<false><<<shape->batch * shape->seq, kNormThreads, 0, (hipStream_t)stream>>>(*shape, nullptr, nullptr, y, norm_weight, h, x);
+    norm_kernel<kNormAdd><<<shape->batch * shape->seq, kNormThreads, 0, (hipStream_t)stream>>>(*shape, nullptr, nullptr, y, norm_weight, h, x);
     return launched("add_norm");
 }
 
@@ -624,3 +695,97 @@ int mk_prefill_argmax(const mk_prefill_shape *shape, const uint16_t *logits, int
 const char *mk_prefill_last_error(void) { return g_error; }
 
 }  // extern "C"
+
+namespace {
+
+int rows_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const int64_t *ids, const int64_t *positions, uint16_t *h,
+                 uint16_t *workspace, int64_t *out_ids, hipStream_t stream) {
+    const RowsWorkspace at(s);
+    const int rows = s.batch * s.seq, H = s.num_attention_heads, KVH = s.num_kv_heads, D = s.head_dim, hid = s.hidden_size, inter = s.intermediate_size;
+    uint16_t *const q = workspace + at.q, *const attn = workspace + at.attn, *const prod = workspace + at.prod;
+    uint16_t *const keys = workspace + at.keys, *const values_t = workspace + at.values_t;
+    uint64_t *const best = (uint64_t *)(workspace + at.best);
+
+    const int value_pieces = (int)((at.best - at.values_t) / 8);  // with the arrivals behind them
+    rows_embed_kernel<<<rows + (value_pieces + 1023) / 1024, 256, 0, stream>>>(s, rows, ids, positions, w.embed, h, (u32x4 *)values_t, value_pieces);
+    if (int rc = launched("embed")) return rc;
+
+    RowsArgs base{};
+    base.s = s, base.rows = rows, base.padded = padded_seq(s.seq), base.positions = positions;
+    base.rope_cos = w.rope_cos, base.rope_sin = w.rope_sin, base.keys = keys, base.values_t = values_t, base.best = best;
+    base.arrived = (int *)(workspace + at.arrived), base.partial = (float *)(workspace + at.partial);
+    const size_t qkv_rows = (size_t)(H + 2 * KVH) * D, cache_layer = (size_t)w.cache_batch * s.kv_max_len * KVH * D;
+    for (int layer = 0; layer < w.num_layers; layer++) {
+        RowsArgs a = base;
+        a.n = (int)qkv_rows, a.k = hid, a.x = h, a.norm_weight = w.attn_norm + (size_t)layer * hid, a.w0 = w.qkv + layer * qkv_rows * hid, a.out = q;
+        a.k_cache = w.k_cache + layer * cache_layer, a.v_cache = w.v_cache + layer * cache_layer;
+        if (int rc = launch_rows<1, kRowsRope, true>(a, "qkv", stream)) return rc;
+        if (int rc = mk_prefill_attention(&s, q, keys, values_t, attn, stream)) return rc;
+        a = base;
+        a.n = hid, a.k = H * D, a.x = attn, a.w0 = w.o + (size_t)layer * hid * H * D, a.out = h;
+        if (int rc = launch_rows<1, kRowsResidual, false>(a, "o", stream)) return rc;
+        a = base;
+        a.n = inter, a.k = hid, a.x = h, a.norm_weight = w.mlp_norm + (size_t)layer * hid, a.out = prod;
+        a.w0 = w.gate + (size_t)layer * inter * hid, a.w1 = w.up + (size_t)layer * inter * hid;
+        if (int rc = launch_rows<2, kRowsSilu, true>(a, "gate and up", stream)) return rc;
+        a = base;
+        a.n = hid, a.k = inter, a.x = prod, a.w0 = w.down + (size_t)layer * hid * inter, a.out = h;
+        if (int rc = launch_rows<1, kRowsResidual, false>(a, "down", stream)) return rc;
+    }
+    RowsArgs a = base;
+    a.n = s.vocab_size, a.k = hid, a.x = h, a.norm_weight = w.final_norm, a.w0 = w.head;
+    if (int rc = launch_rows<2, kRowsArgmax, true>(a, "head", stream)) return rc;
+    rows_best_kernel<<<rows, 256, 0, stream>>>((s.vocab_size + 31) / 32, best, out_ids);
+    return launched("best");
+}
+
+int tiles_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const int64_t *ids, const int64_t *positions, uint16_t *h,
+                  uint16_t *workspace, int64_t *out_ids, hipStream_t stream) {
+    const TilesWorkspace at(s);
+    const int rows = s.batch * s.seq, H = s.num_attention_heads, KVH = s.num_kv_heads, D = s.head_dim, hid = s.hidden_size, inter = s.intermediate_size;
+    uint16_t *const x = workspace + at.x, *const q = workspace + at.q, *const attn = workspace + at.attn, *const prod = workspace + at.prod;
+    uint16_t *const keys = workspace + at.keys, *const values_t = workspace + at.values_t;
+    uint64_t *const best = (uint64_t *)(workspace + at.best);
+
+    const int pieces = (int)((at.best - at.values_t) / 8);  // the padding of the values, and the arrivals
+    zero_kernel<<<min((pieces + 1023) / 1024, 1024), 256, 0, stream>>>((u32x4 *)values_t, pieces);
+    if (int rc = launched("zero")) return rc;
+    if (int rc = mk_prefill_embed(&s, ids, positions, w.embed, w.attn_norm, h, x, stream)) return rc;
+
+    TileArgs base{};
+    base.s = s, base.rows = rows, base.padded = padded_seq(s.seq), base.positions = positions;
+    base.rope_cos = w.rope_cos, base.rope_sin = w.rope_sin, base.keys = keys, base.values_t = values_t, base.best = best;
+    base.arrived = (int *)(workspace + at.arrived), base.partial = (float *)(workspace + at.partial);
+    const size_t qkv_rows = (size_t)(H + 2 * KVH) * D, cache_layer = (size_t)w.cache_batch * s.kv_max_len * KVH * D;
+    auto norm = [&](const uint16_t *weight) {
+        norm_kernel<kNormPlain><<<rows, kNormThreads, 0, stream>>>(s, nullptr, nullptr, nullptr, weight, h, x);
+        return launched("norm");
+    };
+    for (int layer = 0; layer < w.num_layers; layer++) {
+        TileArgs a = base;
+        a.n = (int)qkv_rows, a.k = hid, a.x = x, a.w0 = w.qkv + layer * qkv_rows * hid, a.out = q;
+        a.k_cache = w.k_cache + layer * cache_layer, a.v_cache = w.v_cache + layer * cache_layer;
+        if (int rc = launch_tiles<kTileRope>(a, "qkv", stream)) return rc;
+        if (int rc = mk_prefill_attention(&s, q, keys, values_t, attn, stream)) return rc;
+        a = base;
+        a.n = hid, a.k = H * D, a.x = attn, a.w0 = w.o + (size_t)layer * hid * H * D, a.out = h;
+        if (int rc = launch_tiles<kTileResidual>(a, "o", stream)) return rc;
+        if (int rc = norm(w.mlp_norm + (size_t)layer * hid)) return rc;
+        a = base;
+        a.n = inter, a.k = hid, a.x = x, a.out = prod;
+        a.w0 = w.gate + (size_t)layer * inter * hid, a.w1 = w.up + (size_t)layer * inter * hid;
+        if (int rc = launch_tiles<kTileSilu>(a, "gate and up", stream)) return rc;
+        a = base;
+        a.n = hid, a.k = inter, a.x = prod, a.w0 = w.down + (size_t)layer * hid * inter, a.out = h;
+        if (int rc = launch_tiles<kTileResidual>(a, "down", stream)) return rc;
+        if (int rc = norm(layer + 1 == w.num_layers ? w.final_norm : w.attn_norm + (size_t)(layer + 1) * hid)) return rc;
+    }
+    TileArgs a = base;
+    a.n = s.vocab_size, a.k = hid, a.x = x, a.w0 = w.head;
+    if (int rc = launch_tiles<kTileArgmax>(a, "head", stream)) return rc;
+    const TilePlan plan = tile_plan(rows, s.vocab_size, hid, true);
+    tile_best_kernel<<<(rows + 63) / 64, 1024, 0, stream>>>(rows, plan.n_tiles * (kTileShapes[plan.shape].columns / 64), best, out_ids);
+    return launched("best");
+}
+
+}  // namespace

@@ -13,7 +13,7 @@
 // anyway, so it sums the squares on the way and scales the finished sums.  (One rounding, of h_k w_k, where the plain
 // forward has two.)
 // 32 rows of a 2.5 GB model: 2225 us as library products with Python launches, 916 here (weights over the copy rate of
-// 4.9 TB/s: 505); of 15 GB: 4513 and 3904 (3080).  64 rows: 1160.
+// 4.9 TB/s: 505).  64 rows: 1160.
 // The blocks of a product read X again and again from L2 (M * K * 2 bytes each): the reason for the limit of kRowsMax.
 constexpr int kRowsMax = 64;
 

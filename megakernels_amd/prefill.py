@@ -1,7 +1,7 @@
-"""The prompt forward on the GPU: the dense forward of ``llama.py`` over whole prompts with one HIP kernel between two
-matrix products (``csrc/mk_prefill.hip``) in place of a chain of small PyTorch operations.
+"""The prompt forward on the GPU: the dense forward of ``llama.py`` over whole prompts (``csrc/mk_prefill.hip``).
 
-PyTorch owns the memory and the stream and computes the plain matrix products; everything else - embedding, RMS norm,
+PyTorch owns the memory and the stream.  A prompt of up to some thousand positions runs as one call, its matrix products
+included.  For longer ones PyTorch computes the plain products, and everything between them - embedding, RMS norm,
 residual adds, rotary embedding, cache append, causal attention, SiLU, argmax - is this library's.  There is no
 fallback for a missing library: a GPU forward that it covers raises ``RuntimeError``.
 """
@@ -50,10 +50,10 @@ def load_library():
             function = getattr(lib, f"mk_prefill_{name}")
             function.argtypes = [ctypes.POINTER(Shape)] + [_P] * (count + 1)  # ... and the stream
             function.restype = ctypes.c_int
-        lib.mk_prefill_rows_workspace_bytes.argtypes = [ctypes.POINTER(Shape)]
-        lib.mk_prefill_rows_workspace_bytes.restype = ctypes.c_int64
-        lib.mk_prefill_rows_forward.argtypes = [ctypes.POINTER(Shape), ctypes.POINTER(Model)] + [_P] * 6
-        lib.mk_prefill_rows_forward.restype = ctypes.c_int
+        lib.mk_prefill_workspace_bytes.argtypes = [ctypes.POINTER(Shape)]
+        lib.mk_prefill_workspace_bytes.restype = ctypes.c_int64
+        lib.mk_prefill_forward.argtypes = [ctypes.POINTER(Shape), ctypes.POINTER(Model)] + [_P] * 6
+        lib.mk_prefill_forward.restype = ctypes.c_int
         lib.mk_prefill_last_error.restype = ctypes.c_char_p
         _lib = lib
     return _lib
@@ -97,11 +97,11 @@ def forward(model, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
     positions = positions.to(device=device, dtype=torch.int64).contiguous()
     shape = Shape(B, S, H, KVH, D, c.hidden_size, c.intermediate_size, c.vocab_size, k_cache.shape[2],
                   model.model.rope_cos.shape[0], int(bool(model.extra_config.interleave_rope)), c.rms_norm_eps)
-    workspace_bytes = lib.mk_prefill_rows_workspace_bytes(ctypes.byref(shape))
+    workspace_bytes = lib.mk_prefill_workspace_bytes(ctypes.byref(shape))
     if workspace_bytes < 0:
-        raise RuntimeError(f"mk_prefill_rows_workspace_bytes: {lib.mk_prefill_last_error().decode()}")
+        raise RuntimeError(f"mk_prefill_workspace_bytes: {lib.mk_prefill_last_error().decode()}")
     if workspace_bytes:
-        return _forward_rows(lib, model, shape, workspace_bytes, ids, positions)
+        return _forward_whole(lib, model, shape, workspace_bytes, ids, positions)
     padded = lib.mk_prefill_padded_seq(S)
 
     def rows(width):
@@ -132,9 +132,9 @@ def forward(model, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
     return h, out_ids
 
 
-def _forward_rows(lib, model, shape, workspace_bytes: int, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
-    """A prompt of few positions: one call launches the whole forward, matrix products included.  Issued one by one from
-    Python, its launches took longer than the GPU needs for them."""
+def _forward_whole(lib, model, shape, workspace_bytes: int, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
+    """A prompt that is not too long: one call launches the whole forward, matrix products included.  Issued one by one from
+    Python, the launches of a short prompt took longer than the GPU needs for them."""
     c, device = model.config, ids.device
     *weights, k_cache, v_cache = (t.data_ptr() for t in _tensors(model))
     pointers = Model(*weights, model.model.rope_cos.data_ptr(), model.model.rope_sin.data_ptr(), k_cache, v_cache,
@@ -144,7 +144,7 @@ def _forward_rows(lib, model, shape, workspace_bytes: int, ids: Tensor, position
     out_ids = torch.empty(ids.shape, dtype=torch.int64, device=device)
     with torch.cuda.device(device):
         stream = torch.cuda.current_stream(device).cuda_stream
-        if lib.mk_prefill_rows_forward(ctypes.byref(shape), ctypes.byref(pointers), ids.data_ptr(), positions.data_ptr(), h.data_ptr(),
+        if lib.mk_prefill_forward(ctypes.byref(shape), ctypes.byref(pointers), ids.data_ptr(), positions.data_ptr(), h.data_ptr(),
                                        workspace.data_ptr(), out_ids.data_ptr(), stream) != 0:
-            raise RuntimeError(f"mk_prefill_rows_forward: {lib.mk_prefill_last_error().decode()}")
+            raise RuntimeError(f"mk_prefill_forward: {lib.mk_prefill_last_error().decode()}")
     return h, out_ids

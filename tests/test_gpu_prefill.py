@@ -14,6 +14,13 @@ from megakernels_amd.model_types import BatchState, ExtraModelConfig
 pytestmark = pytest.mark.gpu
 
 
+def config_heads_of_128():
+    """As wide as the 1B layers, with heads of 128."""
+    cfg = config_1b_slice(layers=1, vocab=1024)
+    cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim, cfg.intermediate_size = 16, 4, 128, 4096
+    return cfg
+
+
 def _model(cfg, max_len, batch=1, interleave=True, seed=3):
     model = LlamaForCausalLM.from_random(
         cfg, ExtraModelConfig(interleave_rope=interleave, max_len_override=max_len, max_batch_size=batch), seed=seed)
@@ -72,12 +79,12 @@ def test_prefill_tiny(seq):
     _compare(config_tiny(), seq)
 
 
-@pytest.mark.parametrize("seq", [5, 64, 193])
+@pytest.mark.parametrize("seq", [5, 64, 193, 777])   # 777: the largest tiles, and a K of four parts
 def test_prefill_1b_layers(seq):
     _compare(config_1b_slice(), seq)
 
 
-@pytest.mark.parametrize("seq", [33, 192])
+@pytest.mark.parametrize("seq", [33, 192, 320])
 def test_prefill_8b_layer(seq):
     _compare(config_8b_slice(), seq)
 
@@ -86,13 +93,15 @@ def test_prefill_8b_layer(seq):
 def test_prefill_batch_and_both_rotary_layouts(interleave):
     _compare(config_tiny(), 70, batch=3, interleave=interleave)
     _compare(config_8b_slice(), 40, batch=2, interleave=interleave)
+    _compare(config_heads_of_128(), 50, batch=3, interleave=interleave)
+    _compare(config_heads_of_128(), 500, batch=2, interleave=interleave)   # the largest tiles
 
 
 @pytest.mark.parametrize("interleave", [True, False])
 @pytest.mark.parametrize("batch,seq", [(2, 8), (3, 16), (2, 17), (9, 7), (32, 2)])
 def test_prefill_of_few_rows_in_several_sequences(batch, seq, interleave):
     _compare(config_tiny(), seq, batch=batch, interleave=interleave)
-    _compare(config_8b_slice(), seq, batch=batch, interleave=interleave)
+    _compare(config_heads_of_128(), seq, batch=batch, interleave=interleave)
 
 
 def test_prefill_of_few_rows_at_positions_out_of_order():
@@ -113,7 +122,9 @@ def test_prefill_of_few_rows_takes_the_first_of_equal_logits():
         out = model_gpu(BatchState(input_ids=ids.to("cuda:0"), position_ids=torch.arange(33, device="cuda:0"))).output_ids.cpu()
         logit = rms_norm(model(BatchState(input_ids=ids, position_ids=torch.arange(33))).hidden_states,
                          model.lm_head.input_norm.weight, cfg.rms_norm_eps).float() @ model.model.embed_tokens.weight[5].float()
-        assert out.tolist() == torch.where(logit > 0, first, 0).tolist()
+        # a logit's sign is sure beyond six of its rounding errors, the dozen roundings of each of two layers
+        sure = logit.abs() > 6 * math.sqrt(24) * 2.0**-9 * logit.std()
+        assert bool(sure.sum() > 20) and bool((out == torch.where(logit > 0, first, 0))[sure].all())
         model.lm_head.lm_head.weight.zero_()
 
 
