@@ -143,6 +143,42 @@ def test_prefill_long_enough_for_blocks_of_eight_waves():
     _compare(cfg, 64 * 127 + 5, batch=2)
 
 
+def test_index_tensors_of_other_kinds():
+    cfg, seq = config_tiny(), 40
+    model = _model(cfg, seq).to("cuda:0")
+    ids = torch.randint(0, cfg.vocab_size, (1, seq), device="cuda:0")
+    positions = torch.arange(seq, device="cuda:0")
+    expected = model(BatchState(input_ids=ids, position_ids=positions))
+    strided = torch.stack((ids, ids + 1), dim=-1)[..., 0]
+    for other_ids, other_positions in ((ids.int(), positions.int()), (strided, positions.cpu()), (ids[0], positions[None])):
+        out = model(BatchState(input_ids=other_ids, position_ids=other_positions))
+        assert torch.equal(out.hidden_states, expected.hidden_states) and torch.equal(out.output_ids, expected.output_ids)
+    assert not prefill.covers(model, ids.double(), positions) and not prefill.covers(model, ids, positions[:1])
+    with pytest.raises(RuntimeError):
+        model(BatchState(input_ids=ids.double(), position_ids=positions))
+    model.stacked_params.gate_proj = model.stacked_params.gate_proj.transpose(1, 2).contiguous().transpose(1, 2)
+    assert not prefill.covers(model, ids, positions)   # another layout: the plain forward
+
+
+@pytest.mark.parametrize("seq", [40, 90])
+def test_whole_forward_in_a_captured_graph(seq):
+    cfg = config_tiny()
+    model = _model(cfg, seq).to("cuda:0")
+    batch = BatchState(input_ids=torch.randint(0, cfg.vocab_size, (1, seq), device="cuda:0"), position_ids=torch.arange(seq, device="cuda:0"))
+    expected = model(batch).hidden_states.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = model(batch)
+    for _ in range(3):
+        model.stacked_kv_cache[0].zero_()
+        with torch.inference_mode():
+            out.hidden_states.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.hidden_states, expected) and bool(model.stacked_kv_cache[0].any())
+
+
 def test_argmax_takes_the_first_maximum_and_nan_above_all():
     lib = prefill.load_library()
     import ctypes
