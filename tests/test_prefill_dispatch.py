@@ -1,0 +1,120 @@
+"""Which calls the HIP prompt forward takes.  Its kernels get bare addresses and sizes, so a call that does not fit must go
+to the plain PyTorch forward; decided on the host, and checked here without a GPU and without a launch."""
+
+import pytest
+import torch
+
+from helpers import config_tiny
+from megakernels_amd import prefill
+from megakernels_amd.llama import LlamaForCausalLM
+from megakernels_amd.model_types import BatchState, ExtraModelConfig
+
+
+class _OnGpu:
+    """What ``covers`` asks of the ids, said of ids on a GPU."""
+
+    is_cuda, device, dtype = True, torch.device("cpu"), torch.int64
+
+    def __init__(self, batch, seq):
+        self.shape = torch.Size((batch, seq))
+
+    def numel(self):
+        return self.shape.numel()
+
+
+def _model(cfg=None, batch=1):
+    return LlamaForCausalLM.from_random(cfg or config_tiny(), ExtraModelConfig(max_len_override=32, max_batch_size=batch))
+
+
+def _covers(model, batch=1, seq=8):
+    return prefill.covers(model, _OnGpu(batch, seq), torch.arange(seq))
+
+
+def _forward(model, seq=8):
+    return model(BatchState(input_ids=torch.arange(seq)[None], position_ids=torch.arange(seq)))
+
+
+def test_models_of_the_constructors_are_taken():
+    assert _covers(_model()) and _covers(_model(batch=3), batch=2)
+    assert not _covers(_model(), batch=2) and not _covers(_model(), seq=1)
+
+
+def _set_config(name, value):
+    return lambda m: setattr(m.config, name, value)
+
+
+def _cut_stacked(name, dim):
+    def change(m):
+        t = getattr(m.stacked_params, name)
+        setattr(m.stacked_params, name, t.narrow(dim, 0, t.shape[dim] - 8 if dim else t.shape[dim] - 1).contiguous())
+    return change
+
+
+def _cut_cache(which, dim):
+    def change(m):
+        caches = list(m.stacked_kv_cache)
+        for i in which:
+            caches[i] = caches[i].narrow(dim, 0, caches[i].shape[dim] // 2).contiguous()
+        m.stacked_kv_cache = tuple(caches)
+    return change
+
+
+def _cut_weight(get, dim, keep):
+    def change(m):
+        holder = get(m)
+        holder.weight = holder.weight.narrow(dim, 0, keep).contiguous()
+    return change
+
+
+MISFITS = {
+    "more layers than are stacked": _set_config("num_hidden_layers", 3),
+    "no layers": _set_config("num_hidden_layers", 0),
+    "a vocabulary larger than the embedding": _set_config("vocab_size", 1032),
+    "a vocabulary smaller than the embedding": _set_config("vocab_size", 1016),
+    "another intermediate size": _set_config("intermediate_size", 1088),
+    "another hidden size": _set_config("hidden_size", 576),
+    **{f"{name} of fewer {'layers' if dim == 0 else 'rows' if dim == 1 else 'columns'}": _cut_stacked(name, dim)
+       for name, dims in (("qkv_proj", 3), ("o_proj", 3), ("gate_proj", 3), ("up_proj", 3), ("down_proj", 3), ("attn_ln_weight", 2), ("mlp_ln_weight", 2))
+       for dim in range(dims)},
+    **{f"{'K' if 0 in which else ''}{'V' if 1 in which else ''} cache with half its dimension {dim}": _cut_cache(which, dim)
+       for which, dims in (((0,), (0, 1, 2, 3, 4)), ((1,), (0, 1, 2, 3, 4)), ((0, 1), (0, 3, 4))) for dim in dims},
+    "a shorter embedding": _cut_weight(lambda m: m.model.embed_tokens, 0, 1000),
+    "a narrower embedding": _cut_weight(lambda m: m.model.embed_tokens, 1, 448),
+    "a shorter head": _cut_weight(lambda m: m.lm_head.lm_head, 0, 1000),
+    "a shorter final norm": _cut_weight(lambda m: m.lm_head.input_norm, 0, 448),
+    "a sine table shorter than the cosine's": lambda m: setattr(m.model, "rope_sin", m.model.rope_sin[:100].contiguous()),
+    "rotary tables of half the width": lambda m: vars(m.model).update(rope_cos=m.model.rope_cos[:, :32].contiguous(),
+                                                                      rope_sin=m.model.rope_sin[:, :32].contiguous()),
+    "a norm weight of another rank": lambda m: setattr(m.stacked_params, "attn_ln_weight", m.stacked_params.attn_ln_weight[0, 0].clone()),
+}
+
+
+@pytest.mark.parametrize("misfit", MISFITS)
+def test_tensors_that_do_not_fit_the_configuration_are_not_taken(misfit):
+    cfg = config_tiny()
+    cfg.tie_word_embeddings = False
+    model = _model(cfg, batch=2)
+    assert _covers(model)
+    MISFITS[misfit](model)
+    assert not _covers(model)
+
+
+def test_what_the_plain_forward_refuses_or_takes_of_them():
+    model = _model()
+    model.config.num_hidden_layers = 3
+    with pytest.raises(IndexError):
+        _forward(model)
+    model = _model()
+    _cut_stacked("gate_proj", 2)(model)
+    with pytest.raises(RuntimeError):
+        _forward(model)
+    model = _model()
+    expected = _forward(model)
+    model.config.vocab_size = 1016   # the tensors' own sizes count
+    assert torch.equal(_forward(model).output_ids, expected.output_ids)
+
+
+def test_more_stacked_layers_than_are_run_are_taken():
+    model = _model(config_tiny(layers=3))
+    model.config.num_hidden_layers = 2
+    assert _covers(model)
