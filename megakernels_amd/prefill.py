@@ -83,11 +83,21 @@ def _shapes_match(model) -> bool:
             and cos == sin and len(cos) == 2 and cos[1] == D)
 
 
+def _recorded() -> bool:
+    """Whether someone writes down the operations that this call runs (``torch.compile``, ``torch.jit.trace``, a dispatch
+    mode such as ``make_fx``'s or a flop counter).  A launch through ctypes is none that they see: the record would hold
+    empty outputs."""
+    return torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._len_torch_dispatch_stack() > 0
+
+
 def covers(model, ids: Tensor, positions: Tensor) -> bool:
     """Whether the HIP forward takes this call: more than one position per sequence, bf16 weights on the GPU in the layout
     that the model's constructors make and of the shapes that its configuration says, and an architecture its kernels are
     built for (head_dim 64 or 128, four query heads per KV head, widths in 16-byte pieces).  Everything else runs through the
-    plain PyTorch forward, which also says what is wrong with indices or weights of another type or shape."""
+    plain PyTorch forward, which also says what is wrong with indices or weights of another type or shape, and so does every
+    call whose operations are being recorded."""
+    if _recorded():
+        return False
     c = model.config
     index = (torch.int64, torch.int32)
     rope = (model.model.rope_cos, model.model.rope_sin)

@@ -118,3 +118,25 @@ def test_more_stacked_layers_than_are_run_are_taken():
     model = _model(config_tiny(layers=3))
     model.config.num_hidden_layers = 2
     assert _covers(model)
+
+
+def test_calls_that_are_recorded_are_not_taken():
+    """Tracing, compiling and dispatch modes see PyTorch's operations only."""
+    from torch.fx.experimental.proxy_tensor import make_fx
+    from torch.utils.flop_counter import FlopCounterMode
+
+    model = _model()
+    taken = []
+
+    def step(x):
+        taken.append(_covers(model))
+        return x + 1
+
+    step(torch.zeros(2))
+    torch.jit.trace(step, (torch.zeros(2),), check_trace=False)
+    make_fx(step)(torch.zeros(2))
+    with FlopCounterMode(display=False):
+        step(torch.zeros(2))
+    step(torch.zeros(2))
+    assert taken == [True, False, False, False, True]
+    assert torch.equal(torch.compile(lambda x: x + int(_covers(model)), backend="eager", fullgraph=True)(torch.zeros(2)), torch.zeros(2))
