@@ -480,12 +480,14 @@ int launch_rows_wide(const RowsArgs &a, int split, const char *what, hipStream_t
     return launch_rows<MT, 2, 4, MT == 4 ? 1 : 2, EPI, NORM>(a, split, what, stream);
 }
 // One tile a block: where there is at most one block per CU it has eight waves, so that the CU has enough loads in flight.
+// More blocks than CUs only queries, keys and values can have (above 4096 columns: heads wider than the hidden state).
 template <int MT, int EPI, bool NORM>
 int launch_rows_narrow(const RowsArgs &a, const char *what, hipStream_t stream) {
     if constexpr (!NORM)
         if (rows_split(a.k) > 1) return launch_rows_wide<MT, EPI, NORM>(a, rows_split(a.k), what, stream);
-    if (a.n / 16 <= 256) return launch_rows<MT, 1, 8, MT == 4 ? 1 : 2, EPI, NORM>(a, 1, what, stream);
-    return launch_rows<MT, 1, 4, 1, EPI, NORM>(a, 1, what, stream);
+    if constexpr (EPI == kRowsRope)
+        if (a.n / 16 > 256) return launch_rows<MT, 1, 4, 1, EPI, NORM>(a, 1, what, stream);
+    return launch_rows<MT, 1, 8, MT == 4 ? 1 : 2, EPI, NORM>(a, 1, what, stream);
 }
 template <int NT, int EPI, bool NORM>
 int launch_rows(const RowsArgs &a, const char *what, hipStream_t stream) {
@@ -551,11 +553,13 @@ struct TilePlan {
 };
 // The plan with the least estimated time: rounds of blocks, 3 us to start and end, and for a split of K the blocks' meeting
 // and their sums' way through memory.  (rows 253: 2048 x 8192 estimated 25, measured 24.3 in 64 x 128 x 4 parts against
-// 52.9 whole; rows 777: 16384 x 2048 58 and 56.8 in 256 x 256 against 70.4 in 128 x 128.)  `columns`: gate's and up's
-// together for SiLU; `whole`: the epilogue takes no split.
-TilePlan tile_plan(int rows, int columns, int k, bool whole) {
+// 52.9 whole; rows 777: 16384 x 2048 58 and 56.8 in 256 x 256 against 70.4 in 128 x 128.)  The residual epilogue has no
+// 256 x 256: with at most 2^21 outputs (tiles_cover) there are at most two rounds of 64 x 128, 0.84 us a stage.
+TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k) {
+    const int columns = epilogue == kTileSilu ? 2 * n : n, shapes = epilogue == kTileResidual ? 3 : 4;
+    const bool whole = epilogue == kTileSilu || epilogue == kTileArgmax;  // no split of K
     TilePlan best{};
-    for (int shape = 0; shape < 4; shape++) {
+    for (int shape = 0; shape < shapes; shape++) {
         const TileShape &t = kTileShapes[shape];
         const int m_tiles = (rows + t.rows - 1) / t.rows, n_tiles = (columns + t.columns - 1) / t.columns, stages = k / kTileK;
         for (int split = 1; split <= 8; split *= 2) {
@@ -580,13 +584,14 @@ int launch_tiles(const TileArgs &a, const TilePlan &plan, const char *what, hipS
 }
 template <int EPI>
 int launch_tiles(const TileArgs &a, const char *what, hipStream_t stream) {
-    const TilePlan plan = tile_plan(a.rows, EPI == kTileSilu ? 2 * a.n : a.n, a.k, EPI == kTileSilu || EPI == kTileArgmax);
+    const TilePlan plan = tile_plan((TileEpilogue)EPI, a.rows, a.n, a.k);
     switch (plan.shape) {
     case 0: return launch_tiles<2, 1, 4, EPI>(a, plan, what, stream);
     case 1: return launch_tiles<2, 2, 4, EPI>(a, plan, what, stream);
     case 2: return launch_tiles<2, 2, 2, EPI>(a, plan, what, stream);
-    default: return launch_tiles<4, 4, 2, EPI>(a, plan, what, stream);
     }
+    if constexpr (EPI != kTileResidual) return launch_tiles<4, 4, 2, EPI>(a, plan, what, stream);
+    else return fail(-2, "%s: no such tiles", what);
 }
 
 // The workspace, in elements of 2 bytes, as in RowsWorkspace.
@@ -603,10 +608,9 @@ struct TilesWorkspace {
         values_t = keys + kv;
         arrived = values_t + kv;
         size_t counters = 0, sums = 0;
-        const int qkv = (s.num_attention_heads + 2 * s.num_kv_heads) * s.head_dim, products[3][2] = {
-            {qkv, s.hidden_size}, {s.hidden_size, s.num_attention_heads * s.head_dim}, {s.hidden_size, s.intermediate_size}};
-        for (const auto &nk : products) {
-            const TilePlan plan = tile_plan((int)rows, nk[0], nk[1], false);
+        for (const TilePlan &plan : {tile_plan(kTileRope, (int)rows, (s.num_attention_heads + 2 * s.num_kv_heads) * s.head_dim, s.hidden_size),
+                                     tile_plan(kTileResidual, (int)rows, s.hidden_size, s.num_attention_heads * s.head_dim),
+                                     tile_plan(kTileResidual, (int)rows, s.hidden_size, s.intermediate_size)}) {
             if (plan.split == 1) continue;
             const size_t tiles = (size_t)plan.m_tiles * plan.n_tiles;
             counters = max(counters, tiles);
@@ -783,7 +787,7 @@ int tiles_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const in
     TileArgs a = base;
     a.n = s.vocab_size, a.k = hid, a.x = x, a.w0 = w.head;
     if (int rc = launch_tiles<kTileArgmax>(a, "head", stream)) return rc;
-    const TilePlan plan = tile_plan(rows, s.vocab_size, hid, true);
+    const TilePlan plan = tile_plan(kTileArgmax, rows, s.vocab_size, hid);
     tile_best_kernel<<<(rows + 63) / 64, 1024, 0, stream>>>(rows, plan.n_tiles * (kTileShapes[plan.shape].columns / 64), best, out_ids);
     return launched("best");
 }

@@ -146,6 +146,7 @@ template <int MT, int NT, int WAVES, int STAGES, int EPI, bool NORM>
 __global__ __launch_bounds__(WAVES * 64) void rows_kernel(RowsArgs a) {
     typedef RowsLds<MT, NT, WAVES, STAGES, NORM> Lds;
     constexpr int kLoads = (NT + MT) * 2;  // load instructions of a step
+    static_assert(STAGES <= 2, "the wait for all loads but the last step's");
     extern __shared__ __align__(16) unsigned char lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = (int)threadIdx.x % 64, r = lane % 16, g = lane / 16;
     const int first_step = a.k / 64 * blockIdx.y / gridDim.y, steps = a.k / 64 * (blockIdx.y + 1) / gridDim.y - first_step;
@@ -192,7 +193,6 @@ __global__ __launch_bounds__(WAVES * 64) void rows_kernel(RowsArgs a) {
             // a wave reads only what it has loaded itself: no barrier, only its own loads' arrival, oldest first
             const int newer = mine - 1 - i;
             if (newer >= STAGES - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"i"((STAGES - 1) * kLoads) : "memory");
-            else if (STAGES > 2 && newer == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"i"(kLoads) : "memory");
             else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             const uint32_t slot = read_at + i % STAGES * Lds::kStep;
             u32x4 frag[2][NT + MT], norm[2];

@@ -85,7 +85,7 @@ __device__ __forceinline__ void tile_rope(const TileArgs &a, int row, int first,
 
 // 2 x WN waves of MT x NT tiles of 32 x 32
 template <int WN, int MT, int NT, int STAGES, int EPI>
-__global__ __launch_bounds__(WN * 128, MT * NT == 16 ? 1 : 2) void tile_kernel(TileArgs a) {
+__global__ __launch_bounds__(WN * 128, 2) void tile_kernel(TileArgs a) {
     constexpr int kRows = MT * 64, kTileN = WN * NT * 32, kThreads = WN * 128, kWaves = WN * 2;
     constexpr int kStage = (kRows + kTileN) * kTileK * 2, kLoads = kStage / 1024 / kWaves;  // bytes; load instructions of a wave
     extern __shared__ __align__(16) unsigned char lds[];
