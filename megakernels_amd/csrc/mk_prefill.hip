@@ -529,9 +529,17 @@ bool whole_covers(const mk_prefill_shape &s) {
     return s.hidden_size <= 2048 && s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0;
 }
 bool rows_covers(const mk_prefill_shape &s) { return whole_covers(s) && (int64_t)s.batch * s.seq <= kRowsMax; }
-// From some thousand rows on the library's products are the faster ones (whole forwards of 16 layers, 2048 wide, library and
-// tiles, us: 253 rows 2241 and 1783, 777 rows 3431 and 3170, 1024 rows 3695 and 3550, 1500 rows 4713 and 5249).
-bool tiles_cover(const mk_prefill_shape &s) { return whole_covers(s) && (int64_t)s.batch * s.seq * s.hidden_size <= 1 << 21; }
+// From some thousand rows on the library's products are the faster ones.  Whole forwards of eight layers, intermediate size
+// four times the width, vocabulary 32768, library's products and tiles, us:
+//   2048 wide: 512 rows 1237 and 1176, 768 rows 1542 and 1555, 1024 rows 1808 and 1712, 1536 rows 2291 and 2567
+//   1024 wide: 1024 rows 1130 and 889, 2048 rows 1471 and 1365, 3000 rows 1886 and 1950, 4096 rows 2308 and 2430
+//    512 wide: 2048 rows 1150 and 866, 3000 rows 1268 and 1282, 4096 rows 1564 and 1536, 8192 rows 2664 and 2885
+//    256 wide: 2048 rows 1131 and 672, 4096 rows 1187 and 1180, 8192 rows 2016 and 2215
+//     64 wide: 4096 rows 1129 and 981, 8192 rows 1636 and 1782, 32768 rows 7208 and 8451
+bool tiles_cover(const mk_prefill_shape &s) {
+    const int64_t rows = (int64_t)s.batch * s.seq;
+    return whole_covers(s) && rows <= 4096 && rows * s.hidden_size <= 1 << 21;
+}
 
 // ---- more rows: tiles ----
 

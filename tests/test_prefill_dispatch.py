@@ -1,6 +1,8 @@
 """Which calls the HIP prompt forward takes.  Its kernels get bare addresses and sizes, so a call that does not fit must go
 to the plain PyTorch forward; decided on the host, and checked here without a GPU and without a launch."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -140,3 +142,15 @@ def test_calls_that_are_recorded_are_not_taken():
     step(torch.zeros(2))
     assert taken == [True, False, False, False, True]
     assert torch.equal(torch.compile(lambda x: x + int(_covers(model)), backend="eager", fullgraph=True)(torch.zeros(2)), torch.zeros(2))
+
+
+def _workspace(rows, hidden, batch=1):
+    shape = prefill.Shape(batch, rows // batch, 32, 8, 64, hidden, 4 * hidden, 32768, rows, rows, 1, 1e-5)
+    return prefill.load_library().mk_prefill_workspace_bytes(ctypes.byref(shape))
+
+
+@pytest.mark.parametrize("hidden,most", [(2048, 1024), (1024, 2048), (512, 4096), (256, 4096), (64, 4096)])
+def test_prompts_beyond_the_measured_crossing_take_the_librarys_products(hidden, most):
+    assert _workspace(most, hidden) > 0 and _workspace(most, hidden, batch=2) > 0
+    assert _workspace(most + 1, hidden) == 0 and _workspace(8192, hidden, batch=4) == 0
+    assert _workspace(40, 4096) == 0 and _workspace(40, hidden + 8) == 0
