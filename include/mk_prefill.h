@@ -3,7 +3,8 @@
  * before decoding starts (the reference runs it as a PyTorch module, megakernels/llama.py:232-296,328-348,384-403).
  *
  * Every function launches on `stream` (a hipStream_t, NULL = default stream) without synchronising and returns 0 or a
- * negative error with a message in mk_prefill_last_error().  All tensors are contiguous device memory; bf16 tensors are
+ * negative error with a message in mk_prefill_last_error(); a null pointer or a shape outside the kernels is such an error,
+ * and nothing is launched then.  All tensors are contiguous device memory; bf16 tensors are
  * passed as uint16_t bit patterns.  A "row" is one position of one sequence: rows = batch * seq.
  */
 #ifndef MK_PREFILL_H

@@ -440,6 +440,11 @@ int check_shape(const mk_prefill_shape *s) {
     if (s->kv_max_len < 1 || s->rope_positions < 1) return fail(-2, "empty cache or rope table");
     return 0;
 }
+template <typename... P>
+int check(const mk_prefill_shape *s, const P *...pointers) {
+    if (int rc = check_shape(s)) return rc;
+    return (... && pointers) ? 0 : fail(-2, "null device pointer");
+}
 int padded_seq(int seq) { return (seq + kPosTile - 1) / kPosTile * kPosTile; }
 
 template <int D>
@@ -651,8 +656,11 @@ int64_t mk_prefill_workspace_bytes(const mk_prefill_shape *shape) {
 
 int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids, const int64_t *positions,
                        uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream) {
-    if (int rc = check_shape(shape)) return rc;
-    if (!model || model->num_layers < 1 || model->cache_batch < shape->batch) return fail(-2, "no layers, or a cache of fewer sequences than the call");
+    if (int rc = check(shape, ids, positions, h, workspace, out_ids)) return rc;
+    if (!model) return fail(-1, "no model");
+    const mk_prefill_model &m = *model;
+    if (int rc = check(shape, m.embed, m.attn_norm, m.qkv, m.o, m.mlp_norm, m.gate, m.up, m.down, m.final_norm, m.head, m.rope_cos, m.rope_sin, m.k_cache, m.v_cache)) return rc;
+    if (model->num_layers < 1 || model->cache_batch < shape->batch) return fail(-2, "no layers, or a cache of fewer sequences than the call");
     if (rows_covers(*shape)) return rows_forward(*shape, *model, ids, positions, h, workspace, out_ids, (hipStream_t)stream);
     if (tiles_cover(*shape)) return tiles_forward(*shape, *model, ids, positions, h, workspace, out_ids, (hipStream_t)stream);
     return fail(-2, "%d x %d rows of %d, %d: not a call that the whole forward takes", shape->batch, shape->seq, shape->hidden_size, shape->intermediate_size);
@@ -662,13 +670,13 @@ int mk_prefill_padded_seq(int seq) { return padded_seq(seq); }
 
 int mk_prefill_embed(const mk_prefill_shape *shape, const int64_t *ids, const int64_t *positions, const uint16_t *embed,
                      const uint16_t *norm_weight, uint16_t *h, uint16_t *x, void *stream) {
-    if (int rc = check_shape(shape)) return rc;
+    if (int rc = check(shape, ids, positions, embed, norm_weight, h, x)) return rc;
     norm_kernel<kNormEmbed><<<shape->batch * shape->seq, kNormThreads, 0, (hipStream_t)stream>>>(*shape, ids, positions, embed, norm_weight, h, x);
     return launched("embed");
 }
 
 int mk_prefill_add_norm(const mk_prefill_shape *shape, const uint16_t *y, const uint16_t *norm_weight, uint16_t *h, uint16_t *x, void *stream) {
-    if (int rc = check_shape(shape)) return rc;
+    if (int rc = check(shape, y, norm_weight, h, x)) return rc;
     norm_kernel<kNormAdd><<<shape->batch * shape->seq, kNormThreads, 0, (hipStream_t)stream>>>(*shape, nullptr, nullptr, y, norm_weight, h, x);
     return launched("add_norm");
 }
@@ -676,7 +684,7 @@ int mk_prefill_add_norm(const mk_prefill_shape *shape, const uint16_t *y, const 
 int mk_prefill_rope(const mk_prefill_shape *shape, const uint16_t *qkv, const int64_t *positions, const float *rope_cos,
                     const float *rope_sin, uint16_t *k_cache, uint16_t *v_cache, uint16_t *q, uint16_t *keys,
                     uint16_t *values_t, void *stream) {
-    if (int rc = check_shape(shape)) return rc;
+    if (int rc = check(shape, qkv, positions, rope_cos, rope_sin, k_cache, v_cache, q, keys, values_t)) return rc;
     const int padded = padded_seq(shape->seq);
     const dim3 grid(padded / kPosTile, shape->num_attention_heads + 2 * shape->num_kv_heads, shape->batch);
     auto *kernel = shape->head_dim == 64 ? rope_kernel<64> : rope_kernel<128>;
@@ -686,20 +694,20 @@ int mk_prefill_rope(const mk_prefill_shape *shape, const uint16_t *qkv, const in
 
 int mk_prefill_attention(const mk_prefill_shape *shape, const uint16_t *q, const uint16_t *keys, const uint16_t *values_t,
                          uint16_t *out, void *stream) {
-    if (int rc = check_shape(shape)) return rc;
+    if (int rc = check(shape, q, keys, values_t, out)) return rc;
     return shape->head_dim == 64 ? launch_attention<64>(*shape, q, keys, values_t, out, (hipStream_t)stream)
                                  : launch_attention<128>(*shape, q, keys, values_t, out, (hipStream_t)stream);
 }
 
 int mk_prefill_silu_mul(const mk_prefill_shape *shape, const uint16_t *gate, const uint16_t *up, uint16_t *out, void *stream) {
-    if (int rc = check_shape(shape)) return rc;
+    if (int rc = check(shape, gate, up, out)) return rc;
     const size_t pieces = (size_t)shape->batch * shape->seq * shape->intermediate_size / 8;
     silu_mul_kernel<<<(unsigned)((pieces + 255) / 256), 256, 0, (hipStream_t)stream>>>(pieces, gate, up, out);
     return launched("silu_mul");
 }
 
 int mk_prefill_argmax(const mk_prefill_shape *shape, const uint16_t *logits, int64_t *ids, void *stream) {
-    if (int rc = check_shape(shape)) return rc;
+    if (int rc = check(shape, logits, ids)) return rc;
     argmax_kernel<<<shape->batch * shape->seq, 1024, 0, (hipStream_t)stream>>>(shape->vocab_size, logits, ids);
     return launched("argmax");
 }

@@ -1,6 +1,6 @@
-"""The C ABI of libmk_llama.so as far as it can be checked without a GPU: the
-library loads, exports every function include/mk_llama.h declares, sizes its
-workspace sensibly and refuses malformed launches with a message; and the
+"""The C ABI of libmk_llama.so and libmk_prefill.so as far as it can be checked without a GPU: the
+libraries load, export every function their headers declare, size their
+workspaces sensibly and refuse malformed launches with a message; and the
 kernel's scalar math header, compiled for the host, agrees bit for bit with the
 checker's own copy (two files, one specification)."""
 
@@ -153,3 +153,60 @@ def test_kernel_math_header_equals_checker_math(tmp_path):
         x = np.float32(x)
         want = np.float32(x / np.float32(np.float32(1.0) + np.float32(orc.mk_oracle_expf(float(-x)))))
         assert as_bits(shim.p_silu(float(x))) == as_bits(want)
+
+
+PREFILL_HEADER = ROOT / "include" / "mk_prefill.h"
+
+
+def prefill_functions():
+    text = re.sub(r"/\*.*?\*/", "", PREFILL_HEADER.read_text(), flags=re.S)
+    return sorted(set(re.findall(r"\b(mk_prefill_\w+)\s*\(", text)))
+
+
+def load_prefill():
+    from megakernels_amd import prefill
+    if not prefill.LIBRARY.exists():
+        from megakernels_amd.csrc import build
+        build.build()
+    return prefill, prefill.load_library()
+
+
+def test_prefill_library_exports_every_declared_symbol():
+    _, lib = load_prefill()
+    assert {"mk_prefill_forward", "mk_prefill_workspace_bytes", "mk_prefill_attention"} < set(prefill_functions())
+    for name in prefill_functions():
+        assert getattr(lib, name) is not None
+
+
+def test_prefill_structs_match_the_header():
+    prefill, _ = load_prefill()
+    text = re.sub(r"/\*.*?\*/", "", PREFILL_HEADER.read_text(), flags=re.S)
+    for struct, mirror, size in (("mk_prefill_shape", prefill.Shape, 12 * 4), ("mk_prefill_model", prefill.Model, 14 * 8 + 2 * 4)):
+        body = text[text.index(f"typedef struct {struct} {{"):text.index(f"}} {struct};")].split("{")[1]
+        names = [re.findall(r"(\w+)\s*$", part.strip())[0] for decl in body.split(";") if decl.strip() for part in decl.split(",")]
+        assert names == [f[0] for f in mirror._fields_] and ctypes.sizeof(mirror) == size
+
+
+def test_prefill_refuses_null_pointers_without_touching_a_gpu():
+    prefill, lib = load_prefill()
+    shape = prefill.Shape(1, 5, 8, 2, 64, 512, 1024, 1024, 8, 8, 1, 1e-5)
+    somewhere = ctypes.c_void_p(4096)
+    for name, count in prefill._POINTERS.items():
+        function = getattr(lib, f"mk_prefill_{name}")
+        for missing in range(count):
+            assert function(ctypes.byref(shape), *[None if i == missing else somewhere for i in range(count)], None) == -2
+            assert b"null device pointer" in lib.mk_prefill_last_error()
+        assert function(None, *[somewhere] * count, None) == -1
+    pointers = [f[0] for f in prefill.Model._fields_ if f[1] is ctypes.c_void_p]
+    assert len(pointers) == 14
+    for missing in pointers:
+        model = prefill.Model(**{name: 4096 for name in pointers if name != missing}, num_layers=1, cache_batch=1)
+        assert lib.mk_prefill_forward(ctypes.byref(shape), ctypes.byref(model), *[somewhere] * 5, None) == -2
+        assert b"null device pointer" in lib.mk_prefill_last_error()
+    model = prefill.Model(**{name: 4096 for name in pointers}, num_layers=1, cache_batch=1)
+    for missing in range(5):
+        assert lib.mk_prefill_forward(ctypes.byref(shape), ctypes.byref(model), *[None if i == missing else somewhere for i in range(5)], None) == -2
+    assert lib.mk_prefill_forward(ctypes.byref(shape), None, *[somewhere] * 5, None) == -1
+    for layers, cache_batch in ((0, 1), (1, 0)):
+        model.num_layers, model.cache_batch = layers, cache_batch
+        assert lib.mk_prefill_forward(ctypes.byref(shape), ctypes.byref(model), *[somewhere] * 5, None) == -2
