@@ -72,6 +72,11 @@ int64_t mk_prefill_workspace_bytes(const mk_prefill_shape *shape);
 int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids,
                             const int64_t *positions, uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream);
 
+/* How the whole forward of more than 64 rows tiles a product (0 qkv, 1 O, 2 gate and up, 3 down, 4 LM head): plan = index of
+ * the kernel's shape, rows and columns of a tile, parts of K.  Host arithmetic only; what tests need to know that they reach
+ * every kernel. */
+int mk_prefill_tile_plan(const mk_prefill_shape *shape, int product, int32_t plan[4]);
+
 const char *mk_prefill_last_error(void);
 
 #ifdef __cplusplus

@@ -666,6 +666,24 @@ int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *mo
     return fail(-2, "%d x %d rows of %d, %d: not a call that the whole forward takes", shape->batch, shape->seq, shape->hidden_size, shape->intermediate_size);
 }
 
+int mk_prefill_tile_plan(const mk_prefill_shape *shape, int product, int32_t plan[4]) {
+    if (int rc = check(shape, plan)) return rc;
+    const mk_prefill_shape &s = *shape;
+    if (rows_covers(s) || !tiles_cover(s)) return fail(-2, "%d x %d rows of %d: not tiled", s.batch, s.seq, s.hidden_size);
+    const int rows = s.batch * s.seq, heads = s.num_attention_heads * s.head_dim;
+    TilePlan p;
+    switch (product) {
+    case 0: p = tile_plan(kTileRope, rows, heads + 2 * s.num_kv_heads * s.head_dim, s.hidden_size); break;
+    case 1: p = tile_plan(kTileResidual, rows, s.hidden_size, heads); break;
+    case 2: p = tile_plan(kTileSilu, rows, s.intermediate_size, s.hidden_size); break;
+    case 3: p = tile_plan(kTileResidual, rows, s.hidden_size, s.intermediate_size); break;
+    case 4: p = tile_plan(kTileArgmax, rows, s.vocab_size, s.hidden_size); break;
+    default: return fail(-2, "product %d", product);
+    }
+    plan[0] = p.shape, plan[1] = kTileShapes[p.shape].rows, plan[2] = kTileShapes[p.shape].columns, plan[3] = p.split;
+    return 0;
+}
+
 int mk_prefill_padded_seq(int seq) { return padded_seq(seq); }
 
 int mk_prefill_embed(const mk_prefill_shape *shape, const int64_t *ids, const int64_t *positions, const uint16_t *embed,

@@ -54,6 +54,8 @@ def load_library():
         lib.mk_prefill_workspace_bytes.restype = ctypes.c_int64
         lib.mk_prefill_forward.argtypes = [ctypes.POINTER(Shape), ctypes.POINTER(Model)] + [_P] * 6
         lib.mk_prefill_forward.restype = ctypes.c_int
+        lib.mk_prefill_tile_plan.argtypes = [ctypes.POINTER(Shape), ctypes.c_int, ctypes.POINTER(_I)]
+        lib.mk_prefill_tile_plan.restype = ctypes.c_int
         lib.mk_prefill_last_error.restype = ctypes.c_char_p
         _lib = lib
     return _lib

@@ -21,6 +21,21 @@ def config_heads_of_128():
     return cfg
 
 
+def config_heads_wider_than_the_stream(hidden=2048):
+    """6144 columns of queries, keys and values from a narrower hidden state."""
+    cfg = config_1b_slice(layers=1, vocab=1024)
+    cfg.hidden_size, cfg.head_dim, cfg.intermediate_size = hidden, 128, 1024
+    return cfg
+
+
+# Sizes above 64 rows at which the forward uses, between them, every tiling that it has for the 1B layers from 65 to 1024
+# rows (test_prefill_dispatch.py holds these lists against the library's own plans), and every kernel instance.
+TILED_1B = [70, 150, 200, 300, 540, 777, 1020]
+TILED_HEAD = [(128256, 70), (128256, 200), (128200, 777)]                 # vocabulary, rows; 128200: a last tile of 200 columns
+TILED_WIDE_HEADS = [(2048, 700), (512, 1400)]                             # hidden size, rows
+TILED_ARGMAX = [(1048, 90), (10008, 300), (40008, 100), (40008, 200)]     # vocabulary, rows, of the tiny configuration
+
+
 def _model(cfg, max_len, batch=1, interleave=True, seed=3):
     model = LlamaForCausalLM.from_random(
         cfg, ExtraModelConfig(interleave_rope=interleave, max_len_override=max_len, max_batch_size=batch), seed=seed)
@@ -61,6 +76,13 @@ def _compare(cfg, seq, batch=1, interleave=True, positions=None, max_len=None):
                                       ("k", model_gpu.stacked_kv_cache[0], model.stacked_kv_cache[0]),
                                       ("v", model_gpu.stacked_kv_cache[1], model.stacked_kv_cache[1]))):
         a, b = a.cpu().double(), b.double()
+        # every single value, too: a dozen independent roundings a layer, each with a deviation of 2^-9 / sqrt(3), add up to
+        # something like a normal distribution, whose eighth deviation is not met among some millions of values (2.2 bounds
+        # at most, of 4.6, in these tests); a value's last rounding is relative to itself
+        near = exact[i] if exact else b
+        off = (a - near).abs() / torch.maximum(near.pow(2).mean(-1, keepdim=True).sqrt(), near.abs()).clamp_min(1e-30)
+        print(f"  {name}: largest difference {float(off.max()) / bound:.2f} of the norm's bound", flush=True)
+        assert float(off.max()) <= 8 / math.sqrt(3) * bound, name
         if exact:
             assert a.shape == b.shape and float((a - exact[i]).norm()) <= 1.25 * float((b - exact[i]).norm()), name
             continue
@@ -79,9 +101,25 @@ def test_prefill_tiny(seq):
     _compare(config_tiny(), seq)
 
 
-@pytest.mark.parametrize("seq", [5, 64, 193, 777])   # 777: the largest tiles, and a K of four parts
+@pytest.mark.parametrize("seq", [5, 64, 193, 777])   # 777: the largest tiles, and a K of two parts
 def test_prefill_1b_layers(seq):
     _compare(config_1b_slice(), seq)
+
+
+@pytest.mark.parametrize("seq", TILED_1B)
+def test_every_tiling_of_the_1b_layers(seq):
+    _compare(config_1b_slice(), seq)
+
+
+@pytest.mark.parametrize("vocab,seq", TILED_HEAD)
+def test_head_of_the_full_vocabulary(vocab, seq):
+    _compare(config_1b_slice(layers=1, vocab=vocab), seq)
+
+
+@pytest.mark.parametrize("seq", [7, 20, 50])
+def test_prefill_of_few_rows_with_heads_wider_than_the_stream(seq):
+    _compare(config_heads_wider_than_the_stream(), seq)
+    _compare(config_heads_wider_than_the_stream(), seq, interleave=False)
 
 
 @pytest.mark.parametrize("seq", [33, 192, 320])
@@ -94,7 +132,9 @@ def test_prefill_batch_and_both_rotary_layouts(interleave):
     _compare(config_tiny(), 70, batch=3, interleave=interleave)
     _compare(config_8b_slice(), 40, batch=2, interleave=interleave)
     _compare(config_heads_of_128(), 50, batch=3, interleave=interleave)
-    _compare(config_heads_of_128(), 500, batch=2, interleave=interleave)   # the largest tiles
+    _compare(config_heads_of_128(), 500, batch=2, interleave=interleave)
+    for hidden, rows in TILED_WIDE_HEADS:
+        _compare(config_heads_wider_than_the_stream(hidden), rows, interleave=interleave)   # qkv in the larger tiles
 
 
 @pytest.mark.parametrize("interleave", [True, False])
@@ -109,23 +149,35 @@ def test_prefill_of_few_rows_at_positions_out_of_order():
     _compare(config_tiny(), 37, positions=order, max_len=90)
 
 
-def test_prefill_of_few_rows_takes_the_first_of_equal_logits():
+def _first_of_equal_logits(vocab, seq):
+    print(f"equal logits: vocabulary {vocab} seq {seq}", flush=True)
     cfg = config_tiny()
-    cfg.vocab_size = 1048   # a last block of 24 columns
+    cfg.vocab_size = vocab
     cfg.tie_word_embeddings = False
-    model = _model(cfg, 40)
-    model.lm_head.lm_head.weight.zero_()
-    for first in (0, 17, 1047):
-        model.lm_head.lm_head.weight[first:] = model.model.embed_tokens.weight[5]   # equal logits from `first` on
+    model = _model(cfg, seq + 7)
+    head = model.lm_head.lm_head.weight
+    favoured = model.model.embed_tokens.weight[5]
+    ids = torch.randint(0, cfg.vocab_size, (1, seq), generator=torch.Generator().manual_seed(0))
+    hidden = model(BatchState(input_ids=ids, position_ids=torch.arange(seq))).hidden_states
+    logit = rms_norm(hidden, model.lm_head.input_norm.weight, cfg.rms_norm_eps).float() @ favoured.float()
+    # a logit's sign is sure beyond six of its rounding errors, the dozen roundings of each of two layers
+    sure = logit.abs() > 6 * math.sqrt(24) * 2.0**-9 * logit.std()
+    assert bool(sure.sum() > 20)
+    for first in (0, 17, vocab - 1):
+        head.zero_()
+        head[first:] = favoured   # equal logits from `first` on
         model_gpu = model.to("cuda:0")
-        ids = torch.randint(0, cfg.vocab_size, (1, 33), generator=torch.Generator().manual_seed(0))
-        out = model_gpu(BatchState(input_ids=ids.to("cuda:0"), position_ids=torch.arange(33, device="cuda:0"))).output_ids.cpu()
-        logit = rms_norm(model(BatchState(input_ids=ids, position_ids=torch.arange(33))).hidden_states,
-                         model.lm_head.input_norm.weight, cfg.rms_norm_eps).float() @ model.model.embed_tokens.weight[5].float()
-        # a logit's sign is sure beyond six of its rounding errors, the dozen roundings of each of two layers
-        sure = logit.abs() > 6 * math.sqrt(24) * 2.0**-9 * logit.std()
-        assert bool(sure.sum() > 20) and bool((out == torch.where(logit > 0, first, 0))[sure].all())
-        model.lm_head.lm_head.weight.zero_()
+        out = model_gpu(BatchState(input_ids=ids.to("cuda:0"), position_ids=torch.arange(seq, device="cuda:0"))).output_ids.cpu()
+        assert bool((out == torch.where(logit > 0, first, 0))[sure].all())
+
+
+def test_prefill_of_few_rows_takes_the_first_of_equal_logits():
+    _first_of_equal_logits(1048, 33)   # a last block of 24 columns
+
+
+@pytest.mark.parametrize("vocab,seq", TILED_ARGMAX)   # last tiles of 24, 24, 72 and 72 columns
+def test_tiles_take_the_first_of_equal_logits(vocab, seq):
+    _first_of_equal_logits(vocab, seq)
 
 
 def test_prefill_at_positions_out_of_order_and_from_the_end():
@@ -158,6 +210,22 @@ def test_index_tensors_of_other_kinds():
         model(BatchState(input_ids=ids.double(), position_ids=positions))
     model.stacked_params.gate_proj = model.stacked_params.gate_proj.transpose(1, 2).contiguous().transpose(1, 2)
     assert not prefill.covers(model, ids, positions)   # another layout: the plain forward
+
+
+def test_tensors_that_do_not_fit_and_recorded_calls_run_in_the_plain_forward():
+    cfg, seq = config_tiny(), 40
+    model = _model(cfg, seq).to("cuda:0")
+    batch = BatchState(input_ids=torch.randint(0, 1000, (1, seq), device="cuda:0"), position_ids=torch.arange(seq, device="cuda:0"))
+    hidden = model(batch).hidden_states
+    bound = math.sqrt(12 * cfg.num_hidden_layers) * 2.0**-9
+    compiled = torch.compile(lambda: model(batch).hidden_states, backend="eager", fullgraph=True)()
+    assert float((compiled.double() - hidden.double()).norm() / hidden.double().norm()) <= bound
+    model.config.vocab_size = 1016   # the plain forward goes by the tensors
+    out = model(batch)
+    assert float((out.hidden_states.double() - hidden.double()).norm() / hidden.double().norm()) <= bound
+    model.config.vocab_size, model.config.num_hidden_layers = 1024, 3
+    with pytest.raises(IndexError):
+        model(batch)
 
 
 @pytest.mark.parametrize("seq", [40, 90])

@@ -154,3 +154,33 @@ def test_prompts_beyond_the_measured_crossing_take_the_librarys_products(hidden,
     assert _workspace(most, hidden) > 0 and _workspace(most, hidden, batch=2) > 0
     assert _workspace(most + 1, hidden) == 0 and _workspace(8192, hidden, batch=4) == 0
     assert _workspace(40, 4096) == 0 and _workspace(40, hidden + 8) == 0
+
+
+def _plan(product, rows, hidden=2048, inter=8192, heads=32, kv_heads=8, head_dim=64, vocab=128256):
+    shape = prefill.Shape(1, rows, heads, kv_heads, head_dim, hidden, inter, vocab, rows, rows, 1, 1e-5)
+    plan = (ctypes.c_int32 * 4)()
+    assert prefill.load_library().mk_prefill_tile_plan(ctypes.byref(shape), product, plan) == 0
+    return product, plan[0], plan[3]
+
+
+def test_the_gpu_tests_reach_every_tiling_of_the_1b_layers_and_every_instance():
+    import test_gpu_prefill as gpu
+
+    layers, head = range(4), 4
+    reached = {_plan(product, rows, vocab=8192) for rows in gpu.TILED_1B for product in layers}
+    reached |= {_plan(head, rows, vocab=vocab) for vocab, rows in gpu.TILED_HEAD}
+    assert {_plan(product, rows) for rows in range(65, 1025) for product in range(5)} <= reached
+    reached |= {_plan(product, rows, hidden, 1024, head_dim=128) for hidden, rows in gpu.TILED_WIDE_HEADS for product in layers}
+    reached |= {_plan(head, rows, 512, 1024, 8, 2, vocab=vocab) for vocab, rows in gpu.TILED_ARGMAX}
+    epilogue = {0: "rope", 1: "residual", 2: "silu", 3: "residual", 4: "argmax"}
+    instances = {(epilogue[product], shape) for product, shape, _ in reached}
+    assert instances == {(e, shape) for e in epilogue.values() for shape in range(4)} - {("residual", 3)}
+    assert {_plan(head, rows, 512, 1024, 8, 2, vocab=vocab)[1] for vocab, rows in gpu.TILED_ARGMAX} == {0, 1, 2, 3}
+
+
+def test_tile_plans_are_refused_where_nothing_is_tiled():
+    lib = prefill.load_library()
+    plan = (ctypes.c_int32 * 4)()
+    for rows, hidden, product in ((64, 2048, 0), (1025, 2048, 0), (100, 4096, 0), (100, 2048, 5), (100, 2048, -1)):
+        shape = prefill.Shape(1, rows, 32, 8, 64, hidden, 8192, 32768, rows, rows, 1, 1e-5)
+        assert lib.mk_prefill_tile_plan(ctypes.byref(shape), product, plan) < 0 and lib.mk_prefill_last_error()
