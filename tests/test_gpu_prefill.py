@@ -53,9 +53,13 @@ def _in_64_bits(model):
     return twin
 
 
-def _compare(cfg, seq, batch=1, interleave=True, positions=None, max_len=None):
-    print(f"prefill hidden={cfg.hidden_size} D={cfg.head_dim} seq={seq} batch={batch} interleave={interleave}", flush=True)
+def _compare(cfg, seq, batch=1, interleave=True, positions=None, max_len=None, norms=False):
+    print(f"prefill hidden={cfg.hidden_size} D={cfg.head_dim} seq={seq} batch={batch} interleave={interleave} norms={norms}", flush=True)
     model = _model(cfg, max_len or seq + 3, batch, interleave)
+    if norms:   # weights from a third to three, as trained ones are
+        gen = torch.Generator().manual_seed(9)
+        for weight in (model.stacked_params.attn_ln_weight, model.stacked_params.mlp_ln_weight, model.lm_head.input_norm.weight):
+            weight.copy_(torch.empty(weight.shape).uniform_(-1.1, 1.1, generator=gen).exp())
     model_gpu = model.to("cuda:0")
     ids = torch.randint(0, cfg.vocab_size, (batch, seq), generator=torch.Generator().manual_seed(seq))
     positions = torch.arange(seq) if positions is None else positions
@@ -114,6 +118,11 @@ def test_every_tiling_of_the_1b_layers(seq):
 @pytest.mark.parametrize("vocab,seq", TILED_HEAD)
 def test_head_of_the_full_vocabulary(vocab, seq):
     _compare(config_1b_slice(layers=1, vocab=vocab), seq)
+
+
+@pytest.mark.parametrize("seq", [7, 20, 50, 130, 1100])   # few rows in 16, 32, 64; tiles; the library's products
+def test_norm_weights_of_every_size(seq):
+    _compare(config_1b_slice(vocab=1024), seq, norms=True)
 
 
 @pytest.mark.parametrize("seq", [7, 20, 50])
