@@ -13,7 +13,7 @@ Weights, KV cache and instruction tensor are resident in HBM before the timed
 region starts.
 
 Workloads (random bf16 weights N(0, 0.02) from seed 0, RMSNorm weights 1):
-  c1  Llama-3.2-1B architecture, 32-token prompt prefilled by the plain PyTorch forward, decode from position 32
+  c1  Llama-3.2-1B architecture, 32-token prompt prefilled by the model's forward (libmk_prefill.so), decode from position 32
   c2  1B, KV cache pre-filled to 4096 positions with seeded N(0,1), decode from position 4096  (default)
   c3  1B, KV cache pre-filled to 16384 positions
   c4  Llama-3.1-8B architecture (untied LM head), 32-token prompt, decode from position 32
@@ -113,7 +113,7 @@ def run_workload(name: str, args, steps: int, warmup: int, cpu_steps: int, torch
     prompt_gen = torch.Generator().manual_seed(1)
     prompt = torch.randint(0, cfg.vocab_size, (1, 32), generator=prompt_gen)
     if work["kv"] == "prompt":
-        # prefill once with the plain forward on the GPU (reference scripts/generate.py:125-137); the
+        # prefill once with the model's forward on the GPU (libmk_prefill.so; reference scripts/generate.py:125-137); the
         # megakernel and the checker both start from its cache
         out = model(BatchState(input_ids=prompt.to(device), position_ids=torch.arange(32, device=device)))
         first_token = int(out.output_ids[0, -1])

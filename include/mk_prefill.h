@@ -67,7 +67,8 @@ typedef struct mk_prefill_model {
 
 /* The whole forward where batch * seq is not too large: matrix products included, all in kernels of this library.
  * h [rows, hidden_size] becomes the hidden states, out_ids [rows] the greedy ids.  The workspace's size is
- * mk_prefill_workspace_bytes (0: too many rows, or widths that are no multiple of 64; negative: an error). */
+ * mk_prefill_workspace_bytes.  0: not such a call - a hidden size above 2048 or no multiple of 64, an intermediate size that is
+ * no multiple of 64, more than 64 rows that are above 4096 or above 2^21 / hidden_size.  Negative: an error. */
 int64_t mk_prefill_workspace_bytes(const mk_prefill_shape *shape);
 int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids,
                             const int64_t *positions, uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream);

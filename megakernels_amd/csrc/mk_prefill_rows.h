@@ -12,8 +12,8 @@
 // The norm needs no pass of its own: sum_k W[n,k] (h_k s w_k) = s sum_k W[n,k] (h_k w_k), and every block reads all of h
 // anyway, so it sums the squares on the way and scales the finished sums.  (One rounding, of h_k w_k, where the plain
 // forward has two.)
-// 32 rows of a 2.5 GB model: 2225 us as library products with Python launches, 916 here (weights over the copy rate of
-// 4.9 TB/s: 505).  64 rows: 1160.
+// 32 rows of a 2.5 GB model: 2225 us as library products with Python launches, 890 to 940 here, from run to run (its bytes at
+// the rate of a copy, 4.9 TB/s: 507; at that of reads alone, 7.0 TB/s: 353).  64 rows: 1160.
 // The blocks of a product read X again and again from L2 (M * K * 2 bytes each): the reason for the limit of kRowsMax.
 constexpr int kRowsMax = 64;
 

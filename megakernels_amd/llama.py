@@ -1,5 +1,6 @@
 """Llama weights, rotary tables and KV cache in the layout the instruction VM
-reads, plus a plain PyTorch forward used for prompt prefill.
+reads, plus the dense forward: on the GPU over a whole prompt the HIP kernels
+of ``prefill.py``, otherwise plain PyTorch.
 
 What the decode path needs from reference ``megakernels/llama.py``:
 
@@ -461,7 +462,7 @@ class LlamaForCausalLM:
         k_cache = torch.zeros(shape, device=self.device, dtype=self.dtype)
         self.stacked_kv_cache = (k_cache, torch.zeros_like(k_cache))
 
-    # ---- plain forward (prefill and the torch generator) ------------------
+    # ---- dense forward (prefill and the torch generator) ------------------
 
     @torch.inference_mode()
     def forward(self, batch_state: BatchState) -> BatchState:
@@ -469,7 +470,9 @@ class LlamaForCausalLM:
         writes the KV cache at those positions and returns greedy
         ``output_ids [B, S]`` (reference ``llama.py:232-296,328-348,384-403``).
         ``S > 1`` is a prefill from position 0 with a causal mask, ``S == 1``
-        a decode step attending to ``seq_len`` cached positions."""
+        a decode step attending to ``seq_len`` cached positions.  A prefill
+        that ``prefill.covers`` runs in the HIP kernels; what follows below it
+        is the plain PyTorch forward, for everything else."""
         c = self.config
         p = self.stacked_params
         ids = batch_state.input_ids

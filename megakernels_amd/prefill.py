@@ -1,9 +1,9 @@
 """The prompt forward on the GPU: the dense forward of ``llama.py`` over whole prompts (``csrc/mk_prefill.hip``).
 
-PyTorch owns the memory and the stream.  A prompt of up to some thousand positions runs as one call, its matrix products
-included.  For longer ones PyTorch computes the plain products, and everything between them - embedding, RMS norm,
-residual adds, rotary embedding, cache append, causal attention, SiLU, argmax - is this library's.  There is no
-fallback for a missing library: a GPU forward that it covers raises ``RuntimeError``.
+PyTorch owns the memory and the stream.  A prompt of up to some thousand positions of a model up to 2048 wide runs as one
+call, its matrix products included.  For longer prompts and wider models PyTorch computes the plain products, and everything
+between them - embedding, RMS norm, residual adds, rotary embedding, cache append, causal attention, SiLU, argmax - is this
+library's.  There is no fallback for a missing library: a GPU forward that it covers raises ``RuntimeError``.
 """
 
 from __future__ import annotations

@@ -8,7 +8,7 @@ Differences forced by the environment: nothing is downloaded, so ``model`` is ``
 (random-initialised architecture; the prompt is ``prompt_len`` seeded random token ids) or a local checkpoint
 directory; when that directory holds a tokenizer, ``prompt=...`` (``chat=true`` for the chat template) is
 tokenised and the output is printed as text too, as the reference does (``generate.py:98-112,186-202``).  Modes: ``mk`` (HIP megakernel) and ``torch`` (plain PyTorch forward).
-As in the reference (``generate.py:125-137``) the prompt is prefilled by the PyTorch model and the timed
+As in the reference (``generate.py:125-137``) the prompt is prefilled by the model's forward, once, and the timed
 region is ``ntok - 1`` decode steps, repeated ``num_warmup + num_iters`` times.
 """
 

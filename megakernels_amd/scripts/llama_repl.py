@@ -4,7 +4,7 @@
         [max_tokens_per_turn=1024] [sched=rr] [num_attention_partitions=1] [print_prompt_len=true]
 
 Every turn renders the whole conversation through the tokenizer's chat template, prefills it with the
-plain PyTorch forward, then decodes greedily until an end-of-sequence id (looked for on the host every 16
+model's forward, then decodes greedily until an end-of-sequence id (looked for on the host every 16
 tokens, which is also how many decode steps go into one launch) or ``max_tokens_per_turn``.  The directory
 must hold ``config.json``, ``*.safetensors`` and the tokenizer; nothing is downloaded.
 """

@@ -110,7 +110,7 @@ def test_decode_8b_slice_all_steps_in_one_launch():
 
 
 def test_prefill_on_the_gpu_hands_its_cache_to_the_megakernel():
-    """The reference's flow (scripts/generate.py:125-137): the prompt goes through the plain PyTorch
+    """The reference's flow (scripts/generate.py:125-137): the prompt goes through the model's
     forward on the GPU, which fills the KV cache and yields the first token; the megakernel decodes
     from there.  The checker starts from a copy of the cache the GPU prefill left, and must see the
     same tokens and the same appended KV rows."""
