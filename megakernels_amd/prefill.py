@@ -68,21 +68,31 @@ def _tensors(model) -> list[Tensor]:
             p.down_proj, model.lm_head.input_norm.weight, model.lm_head.lm_head.weight, *model.stacked_kv_cache]
 
 
-def _shapes_match(model) -> bool:
-    """Whether every tensor has the shape that the configuration says.  The kernels take sizes from the configuration and
-    addresses from the tensors, which are public attributes: a shorter one would be read, or the cache written, past its end.
-    More layers than the configuration counts are only more memory."""
+def _fits(model, device: int) -> bool:
+    """Whether every tensor is what the kernels take it for: bf16 (the rotary tables fp32) on that device, contiguous, in
+    16-byte pieces, and of the shape that the configuration says.  The kernels take sizes from the configuration and addresses
+    from the tensors, which are public attributes: a shorter one would be read, or the cache written, past its end.  More
+    layers than the configuration counts are only more memory."""
     c = model.config
     L, hid, inter, vocab, D = c.num_hidden_layers, c.hidden_size, c.intermediate_size, c.vocab_size, c.head_dim
     q_rows, kv_rows = c.num_attention_heads * D, c.num_key_value_heads * D
-    embed, attn_norm, qkv, o, mlp_norm, gate, up, down, final_norm, head, k_cache, v_cache = (t.shape for t in _tensors(model))
-    cos, sin = model.model.rope_cos.shape, model.model.rope_sin.shape
-    stacked = ((attn_norm, (hid,)), (qkv, (q_rows + 2 * kv_rows, hid)), (o, (hid, q_rows)), (mlp_norm, (hid,)), (gate, (inter, hid)),
-               (up, (inter, hid)), (down, (hid, inter)))
-    return (L > 0 and all(len(shape) > 0 and shape[0] >= L and shape[1:] == rest for shape, rest in stacked)
-            and embed == head == (vocab, hid) and final_norm == (hid,)
-            and k_cache == v_cache and len(k_cache) == 5 and k_cache[0] >= L and k_cache[3:] == (c.num_key_value_heads, D)
-            and cos == sin and len(cos) == 2 and cos[1] == D)
+    tensors = _tensors(model)
+    embed, attn_norm, qkv, o, mlp_norm, gate, up, down, final_norm, head, k_cache, v_cache = [t.shape for t in tensors]
+    for shape, expected in ((attn_norm, (L, hid)), (qkv, (L, q_rows + 2 * kv_rows, hid)), (o, (L, hid, q_rows)), (mlp_norm, (L, hid)),
+                            (gate, (L, inter, hid)), (up, (L, inter, hid)), (down, (L, hid, inter))):
+        if shape != expected and (shape[1:] != expected[1:] or shape[0] < L):
+            return False
+    rope = (model.model.rope_cos, model.model.rope_sin)
+    cos, sin = [t.shape for t in rope]
+    if (L < 1 or embed != (vocab, hid) or head != embed or final_norm != (hid,)
+            or k_cache != v_cache or len(k_cache) != 5 or k_cache[0] < L or k_cache[3] != c.num_key_value_heads or k_cache[4] != D
+            or cos != sin or len(cos) != 2 or cos[1] != D):
+        return False
+    for dtype, group in ((torch.bfloat16, tensors), (torch.float32, rope)):
+        for t in group:
+            if t.dtype is not dtype or t.get_device() != device or not t.is_contiguous() or t.data_ptr() % 16:
+                return False
+    return True
 
 
 def _recorded() -> bool:
@@ -102,15 +112,12 @@ def covers(model, ids: Tensor, positions: Tensor) -> bool:
         return False
     c = model.config
     index = (torch.int64, torch.int32)
-    rope = (model.model.rope_cos, model.model.rope_sin)
     return (ids.is_cuda and ids.shape[-1] > 1 and ids.device == model.device and ids.dtype in index and positions.dtype in index
-            and positions.shape == ids.shape[1:] and _shapes_match(model) and 0 < ids.shape[0] <= model.stacked_kv_cache[0].shape[1]
+            and positions.shape == ids.shape[1:] and 0 < ids.shape[0] <= model.stacked_kv_cache[0].shape[1]
             and ids.shape[0] <= 65535 and ids.numel() <= 1 << 22
             and c.head_dim in (64, 128) and c.num_attention_heads == 4 * c.num_key_value_heads
             and c.hidden_size % 8 == 0 and c.hidden_size <= 8192 and c.intermediate_size % 8 == 0 and c.vocab_size % 8 == 0
-            and all(t.dtype == torch.bfloat16 and t.device == ids.device and t.is_contiguous() and t.data_ptr() % 16 == 0
-                    for t in _tensors(model))
-            and all(t.dtype == torch.float32 and t.device == ids.device and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in rope))
+            and _fits(model, ids.get_device()))
 
 
 def forward(model, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:

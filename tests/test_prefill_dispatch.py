@@ -23,6 +23,9 @@ class _OnGpu:
     def numel(self):
         return self.shape.numel()
 
+    def get_device(self):
+        return -1
+
 
 def _model(cfg=None, batch=1):
     return LlamaForCausalLM.from_random(cfg or config_tiny(), ExtraModelConfig(max_len_override=32, max_batch_size=batch))
@@ -87,6 +90,7 @@ MISFITS = {
     "a sine table shorter than the cosine's": lambda m: setattr(m.model, "rope_sin", m.model.rope_sin[:100].contiguous()),
     "rotary tables of half the width": lambda m: vars(m.model).update(rope_cos=m.model.rope_cos[:, :32].contiguous(),
                                                                       rope_sin=m.model.rope_sin[:, :32].contiguous()),
+    "stacked weights without dimensions": lambda m: vars(m.stacked_params).update({k: torch.ones((), dtype=torch.bfloat16) for k in vars(m.stacked_params)}),
     "a norm weight of another rank": lambda m: setattr(m.stacked_params, "attn_ln_weight", m.stacked_params.attn_ln_weight[0, 0].clone()),
 }
 
