@@ -831,7 +831,7 @@ int tiles_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const in
     a.n = s.vocab_size, a.k = hid, a.x = x, a.w0 = w.head;
     if (int rc = launch_tiles<kTileArgmax>(a, "head", stream)) return rc;
     const TilePlan plan = tile_plan(kTileArgmax, rows, s.vocab_size, hid);
-    tile_best_kernel<<<(rows + 63) / 64, 1024, 0, stream>>>(rows, plan.n_tiles * (kTileShapes[plan.shape].columns / 64), best, out_ids);
+    tile_best_kernel<<<(rows + 15) / 16, 1024, 0, stream>>>(rows, plan.n_tiles * (kTileShapes[plan.shape].columns / 64), best, out_ids);
     return launched("best");
 }
 
