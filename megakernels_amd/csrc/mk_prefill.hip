@@ -3,8 +3,9 @@
 // A prompt of a few thousand positions is bound by its matrix products; what a framework adds to them is traffic - the
 // same activations read and written once per small operation - and launches.  In this file every stage between two
 // products is one kernel: residual add + RMS norm, rotary embedding + cache append + the layouts attention reads, attention
-// itself, SiLU * up, argmax.  Shorter prompts of models up to 2048 wide have their products here, too, with these stages
-// inside them: mk_prefill_rows.h for up to 64 rows, mk_prefill_tiles.h above; the host side below chooses.  Values are
+// itself, SiLU * up, argmax.  Prompts of up to some thousand positions have their products here, too, with these stages
+// inside them: mk_prefill_rows.h for up to 64 rows of models up to 2048 wide, mk_prefill_tiles.h above, mk_prefill_wide.h for
+// longer prompts and wider models; the host side below chooses.  Values are
 // narrowed to bf16 exactly where the plain forward narrows them (megakernels/llama.py:38-47 for the norm, :136-174 for the
 // rotation), but for the norm of few rows.
 #include <hip/hip_runtime.h>
@@ -414,6 +415,7 @@ __global__ __launch_bounds__(1024) void argmax_kernel(int vocab, const uint16_t 
 
 #include "mk_prefill_rows.h"
 #include "mk_prefill_tiles.h"
+#include "mk_prefill_wide.h"
 
 // ---------------------------------------------------------------------------------------------
 // host side
@@ -554,8 +556,20 @@ bool tiles_cover(const mk_prefill_shape &s) {
     const int64_t rows = (int64_t)s.batch * s.seq;
     return whole_covers(s) && rows <= 4096 && rows * s.hidden_size <= 1 << 21;
 }
+// Wide tiles (mk_prefill_wide.h) beside the narrower ones.  Whole forwards, us, narrow tiles or the library's products, and wide:
+//   1B architecture: 253 rows 1749 and 1747, 320 rows 2117 and 2028, 777 rows 2971 and 2885, 1024 rows 3325 and 3191 (tiles);
+//     1100 rows 4343 and 4100, 1500 rows 4782 and 4601, 2048 rows 5879 and 5329, 4096 rows 10876 and 9999 (library)
+//   8B architecture: 520 rows 11766 and 11541, 640 rows 12443 and 12949, 700 rows 13312 and 13027, 777 rows 14972 and 13715,
+//     2048 rows 28628 and 27299, 3000 rows 40426 and 43355, 4096 rows 52510 and 53104 (library)
+// Prompts of up to 512 rows of wide models are the library's for the reason above, those up to 704 for want of a gain.
+bool wide_covers(const mk_prefill_shape &s) {
+    const int64_t rows = (int64_t)s.batch * s.seq;
+    const bool narrow = s.hidden_size <= 2048;
+    return s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0 && s.hidden_size >= 256 && rows > (narrow ? 256 : 704) && rows <= (narrow ? 4096 : 2048)
+        && (int64_t)s.batch * s.kv_max_len < INT32_MAX;
+}
 
-// ---- more rows: tiles ----
+// ---- more rows: tiles, narrow and wide ----
 
 // The shapes a product can be tiled in, with what a stage of 64 elements of K takes (us, measured with as many blocks as
 // there are slots) and how many blocks the chip holds at once.
@@ -567,8 +581,10 @@ constexpr TileShape kTileShapes[] = {
     {64, 128, 256, 0.42f},   // four stages in LDS: the least time for one tile
     {128, 128, 256, 0.62f},  // four stages
     {128, 128, 512, 1.05f},  // two stages, two blocks a CU
-    {256, 256, 256, 1.72f},  // the most work per byte of LDS: 1.23 PFLOP/s over whole rounds
+    {256, 256, 256, 1.40f},  // square_kernel: the most work per byte of LDS
+    {128, 256, 256, 0.84f},  // flat_kernel
 };
+constexpr int kSquare = 3, kFlat = 4, kSquareLeastK = 4 * kTileK;
 struct TilePlan {
     int shape, split, m_tiles, n_tiles;
     float us;
@@ -576,17 +592,20 @@ struct TilePlan {
 // The plan with the least estimated time: rounds of blocks, 3 us to start and end, and for a split of K the blocks' meeting
 // and their sums' way through memory.  (rows 253: 2048 x 8192 estimated 25, measured 24.3 in 64 x 128 x 4 parts against
 // 52.9 whole; rows 777: 16384 x 2048 58 and 56.8 in 256 x 256 against 70.4 in 128 x 128.)  The residual epilogue has no
-// 256 x 256: with at most 2^21 outputs (tiles_cover) there are at most two rounds of 64 x 128, 0.84 us a stage.
-TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k) {
-    const int columns = epilogue == kTileSilu ? 2 * n : n, shapes = epilogue == kTileResidual ? 3 : 4;
+// 256 x 256: its products are narrow, and 128 x 256 fills the chip twice as soon.
+TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k, bool wide) {
+    const int columns = epilogue == kTileSilu ? 2 * n : n;
     const bool whole = epilogue == kTileSilu || epilogue == kTileArgmax;  // no split of K
     TilePlan best{};
-    for (int shape = 0; shape < shapes; shape++) {
+    for (int shape = 0; shape <= (wide ? kFlat : kSquare); shape++) {
         const TileShape &t = kTileShapes[shape];
+        if (shape == kSquare && (epilogue == kTileResidual || k < kSquareLeastK)) continue;
         const int m_tiles = (rows + t.rows - 1) / t.rows, n_tiles = (columns + t.columns - 1) / t.columns, stages = k / kTileK;
         for (int split = 1; split <= 8; split *= 2) {
-            if (split > 1 && (whole || stages / split < 8 || t.rows == 256)) break;
+            if (split > 1 && (whole || stages / split < 8 || shape == kSquare)) break;
             const int64_t rounds = ((int64_t)m_tiles * n_tiles * split + t.slots - 1) / t.slots;
+            // more sums than fit one round of blocks cost more than the estimate (3000 rows of an 8B model's layers)
+            if (wide && split > 1 && rounds > 1) break;
             const float meeting = split > 1 ? 3.0f + (float)split * rows * columns * 8 / 3e6f : 0.0f;
             const float us = (float)rounds * ((stages + split - 1) / split) * t.stage_us + 3.0f + meeting;
             if (best.split == 0 || us < best.us) best = {shape, split, m_tiles, n_tiles, us};
@@ -594,32 +613,53 @@ TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k) {
     }
     return best;
 }
+// the five products of a layer and of the head
+struct Plans {
+    TilePlan qkv, o, up, down, head;
+    Plans(const mk_prefill_shape &s, bool wide) {
+        const int rows = s.batch * s.seq, heads = s.num_attention_heads * s.head_dim, kv = s.num_kv_heads * s.head_dim;
+        qkv = tile_plan(kTileRope, rows, heads + 2 * kv, s.hidden_size, wide);
+        o = tile_plan(kTileResidual, rows, s.hidden_size, heads, wide);
+        up = tile_plan(kTileSilu, rows, s.intermediate_size, s.hidden_size, wide);
+        down = tile_plan(kTileResidual, rows, s.hidden_size, s.intermediate_size, wide);
+        head = tile_plan(kTileArgmax, rows, s.vocab_size, s.hidden_size, wide);
+    }
+    int get(int product, int32_t plan[4]) const {
+        if (product < 0 || product > 4) return fail(-2, "product %d", product);
+        const TilePlan &p = (&qkv)[product];
+        plan[0] = p.shape, plan[1] = kTileShapes[p.shape].rows, plan[2] = kTileShapes[p.shape].columns, plan[3] = p.split;
+        return 0;
+    }
+};
 
-template <int WN, int MT, int STAGES, int EPI>
-int launch_tiles(const TileArgs &a, const TilePlan &plan, const char *what, hipStream_t stream) {
-    constexpr int bytes = STAGES * (MT * 64 + WN * 64) * kTileK * 2;
-    auto *kernel = tile_kernel<WN, MT, 2, STAGES, EPI>;
+template <typename Kernel>
+int launch_lds(Kernel *kernel, dim3 grid, int threads, int bytes, const TileArgs &a, const char *what, hipStream_t stream) {
     const hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return fail(-5, "%s: %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
-    kernel<<<dim3(8 * ((plan.n_tiles + 7) / 8) * plan.m_tiles, plan.split), WN * 128, bytes, stream>>>(a);
+    kernel<<<grid, threads, bytes, stream>>>(a);
     return launched(what);
 }
+template <int WN, int MT, int STAGES, int EPI>
+int launch_tiles(const TileArgs &a, dim3 grid, const char *what, hipStream_t stream) {
+    return launch_lds(tile_kernel<WN, MT, 2, STAGES, EPI>, grid, WN * 128, STAGES * (MT * 64 + WN * 64) * kTileK * 2, a, what, stream);
+}
 template <int EPI>
-int launch_tiles(const TileArgs &a, const char *what, hipStream_t stream) {
-    const TilePlan plan = tile_plan((TileEpilogue)EPI, a.rows, a.n, a.k);
+int launch_tiles(const TileArgs &a, const TilePlan &plan, const char *what, hipStream_t stream) {
+    const dim3 grid(8 * ((plan.n_tiles + 7) / 8) * plan.m_tiles, plan.split);
     switch (plan.shape) {
-    case 0: return launch_tiles<2, 1, 4, EPI>(a, plan, what, stream);
-    case 1: return launch_tiles<2, 2, 4, EPI>(a, plan, what, stream);
-    case 2: return launch_tiles<2, 2, 2, EPI>(a, plan, what, stream);
+    case 0: return launch_tiles<2, 1, 4, EPI>(a, grid, what, stream);
+    case 1: return launch_tiles<2, 2, 4, EPI>(a, grid, what, stream);
+    case 2: return launch_tiles<2, 2, 2, EPI>(a, grid, what, stream);
+    case kFlat: return launch_lds(flat_kernel<EPI>, grid, 512, kFlatBytes, a, what, stream);
     }
-    if constexpr (EPI != kTileResidual) return launch_tiles<4, 4, 2, EPI>(a, plan, what, stream);
+    if constexpr (EPI != kTileResidual) return launch_lds(square_kernel<EPI>, dim3(256), 512, kSquareBytes, a, what, stream);
     else return fail(-2, "%s: no such tiles", what);
 }
 
 // The workspace, in elements of 2 bytes, as in RowsWorkspace.
 struct TilesWorkspace {
     size_t x, q, attn, prod, keys, values_t, arrived, best, partial, total;
-    explicit TilesWorkspace(const mk_prefill_shape &s) {
+    TilesWorkspace(const mk_prefill_shape &s, const Plans &plans) {
         const size_t rows = (size_t)s.batch * s.seq, heads = rows * s.num_attention_heads * s.head_dim;
         const size_t kv = (size_t)s.batch * s.num_kv_heads * s.head_dim * padded_seq(s.seq);
         x = 0;
@@ -630,9 +670,7 @@ struct TilesWorkspace {
         values_t = keys + kv;
         arrived = values_t + kv;
         size_t counters = 0, sums = 0;
-        for (const TilePlan &plan : {tile_plan(kTileRope, (int)rows, (s.num_attention_heads + 2 * s.num_kv_heads) * s.head_dim, s.hidden_size),
-                                     tile_plan(kTileResidual, (int)rows, s.hidden_size, s.num_attention_heads * s.head_dim),
-                                     tile_plan(kTileResidual, (int)rows, s.hidden_size, s.intermediate_size)}) {
+        for (const TilePlan &plan : {plans.qkv, plans.o, plans.down}) {
             if (plan.split == 1) continue;
             const size_t tiles = (size_t)plan.m_tiles * plan.n_tiles;
             counters = max(counters, tiles);
@@ -650,8 +688,18 @@ __global__ __launch_bounds__(256) void zero_kernel(u32x4 *dst, int pieces) {
 
 int rows_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const int64_t *ids, const int64_t *positions, uint16_t *h,
                  uint16_t *workspace, int64_t *out_ids, hipStream_t stream);
-int tiles_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const int64_t *ids, const int64_t *positions, uint16_t *h,
-                  uint16_t *workspace, int64_t *out_ids, hipStream_t stream);
+int tiles_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const Plans &plans, const int64_t *ids, const int64_t *positions,
+                  uint16_t *h, uint16_t *workspace, int64_t *out_ids, hipStream_t stream);
+
+int check_model(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids, const int64_t *positions, const uint16_t *h,
+                const uint16_t *workspace, const int64_t *out_ids) {
+    if (int rc = check(shape, ids, positions, h, workspace, out_ids)) return rc;
+    if (!model) return fail(-1, "no model");
+    const mk_prefill_model &m = *model;
+    if (int rc = check(shape, m.embed, m.attn_norm, m.qkv, m.o, m.mlp_norm, m.gate, m.up, m.down, m.final_norm, m.head, m.rope_cos, m.rope_sin, m.k_cache, m.v_cache)) return rc;
+    if (m.num_layers < 1 || m.cache_batch < shape->batch) return fail(-2, "no layers, or a cache of fewer sequences than the call");
+    return 0;
+}
 
 }  // namespace
 
@@ -660,37 +708,39 @@ extern "C" {
 int64_t mk_prefill_workspace_bytes(const mk_prefill_shape *shape) {
     if (int rc = check_shape(shape)) return rc;
     if (rows_covers(*shape)) return (int64_t)RowsWorkspace(*shape).total * 2;
-    return tiles_cover(*shape) ? (int64_t)TilesWorkspace(*shape).total * 2 : 0;
+    return tiles_cover(*shape) ? (int64_t)TilesWorkspace(*shape, Plans(*shape, false)).total * 2 : 0;
 }
 
 int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids, const int64_t *positions,
                        uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream) {
-    if (int rc = check(shape, ids, positions, h, workspace, out_ids)) return rc;
-    if (!model) return fail(-1, "no model");
-    const mk_prefill_model &m = *model;
-    if (int rc = check(shape, m.embed, m.attn_norm, m.qkv, m.o, m.mlp_norm, m.gate, m.up, m.down, m.final_norm, m.head, m.rope_cos, m.rope_sin, m.k_cache, m.v_cache)) return rc;
-    if (model->num_layers < 1 || model->cache_batch < shape->batch) return fail(-2, "no layers, or a cache of fewer sequences than the call");
+    if (int rc = check_model(shape, model, ids, positions, h, workspace, out_ids)) return rc;
     if (rows_covers(*shape)) return rows_forward(*shape, *model, ids, positions, h, workspace, out_ids, (hipStream_t)stream);
-    if (tiles_cover(*shape)) return tiles_forward(*shape, *model, ids, positions, h, workspace, out_ids, (hipStream_t)stream);
+    if (tiles_cover(*shape)) return tiles_forward(*shape, *model, Plans(*shape, false), ids, positions, h, workspace, out_ids, (hipStream_t)stream);
     return fail(-2, "%d x %d rows of %d, %d: not a call that the whole forward takes", shape->batch, shape->seq, shape->hidden_size, shape->intermediate_size);
 }
 
 int mk_prefill_tile_plan(const mk_prefill_shape *shape, int product, int32_t plan[4]) {
     if (int rc = check(shape, plan)) return rc;
-    const mk_prefill_shape &s = *shape;
-    if (rows_covers(s) || !tiles_cover(s)) return fail(-2, "%d x %d rows of %d: not tiled", s.batch, s.seq, s.hidden_size);
-    const int rows = s.batch * s.seq, heads = s.num_attention_heads * s.head_dim;
-    TilePlan p;
-    switch (product) {
-    case 0: p = tile_plan(kTileRope, rows, heads + 2 * s.num_kv_heads * s.head_dim, s.hidden_size); break;
-    case 1: p = tile_plan(kTileResidual, rows, s.hidden_size, heads); break;
-    case 2: p = tile_plan(kTileSilu, rows, s.intermediate_size, s.hidden_size); break;
-    case 3: p = tile_plan(kTileResidual, rows, s.hidden_size, s.intermediate_size); break;
-    case 4: p = tile_plan(kTileArgmax, rows, s.vocab_size, s.hidden_size); break;
-    default: return fail(-2, "product %d", product);
-    }
-    plan[0] = p.shape, plan[1] = kTileShapes[p.shape].rows, plan[2] = kTileShapes[p.shape].columns, plan[3] = p.split;
-    return 0;
+    if (rows_covers(*shape) || !tiles_cover(*shape)) return fail(-2, "%d x %d rows of %d: not tiled", shape->batch, shape->seq, shape->hidden_size);
+    return Plans(*shape, false).get(product, plan);
+}
+
+int64_t mk_prefill_wide_workspace_bytes(const mk_prefill_shape *shape) {
+    if (int rc = check_shape(shape)) return rc;
+    return wide_covers(*shape) ? (int64_t)TilesWorkspace(*shape, Plans(*shape, true)).total * 2 : 0;
+}
+
+int mk_prefill_wide_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids, const int64_t *positions,
+                            uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream) {
+    if (int rc = check_model(shape, model, ids, positions, h, workspace, out_ids)) return rc;
+    if (!wide_covers(*shape)) return fail(-2, "%d x %d rows of %d, %d: not a call of wide tiles", shape->batch, shape->seq, shape->hidden_size, shape->intermediate_size);
+    return tiles_forward(*shape, *model, Plans(*shape, true), ids, positions, h, workspace, out_ids, (hipStream_t)stream);
+}
+
+int mk_prefill_wide_plan(const mk_prefill_shape *shape, int product, int32_t plan[4]) {
+    if (int rc = check(shape, plan)) return rc;
+    if (!wide_covers(*shape)) return fail(-2, "%d x %d rows of %d: no wide tiles", shape->batch, shape->seq, shape->hidden_size);
+    return Plans(*shape, true).get(product, plan);
 }
 
 int mk_prefill_padded_seq(int seq) { return padded_seq(seq); }
@@ -786,9 +836,9 @@ int rows_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const int
     return launched("best");
 }
 
-int tiles_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const int64_t *ids, const int64_t *positions, uint16_t *h,
-                  uint16_t *workspace, int64_t *out_ids, hipStream_t stream) {
-    const TilesWorkspace at(s);
+int tiles_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const Plans &plans, const int64_t *ids, const int64_t *positions,
+                  uint16_t *h, uint16_t *workspace, int64_t *out_ids, hipStream_t stream) {
+    const TilesWorkspace at(s, plans);
     const int rows = s.batch * s.seq, H = s.num_attention_heads, KVH = s.num_kv_heads, D = s.head_dim, hid = s.hidden_size, inter = s.intermediate_size;
     uint16_t *const x = workspace + at.x, *const q = workspace + at.q, *const attn = workspace + at.attn, *const prod = workspace + at.prod;
     uint16_t *const keys = workspace + at.keys, *const values_t = workspace + at.values_t;
@@ -812,26 +862,25 @@ int tiles_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const in
         TileArgs a = base;
         a.n = (int)qkv_rows, a.k = hid, a.x = x, a.w0 = w.qkv + layer * qkv_rows * hid, a.out = q;
         a.k_cache = w.k_cache + layer * cache_layer, a.v_cache = w.v_cache + layer * cache_layer;
-        if (int rc = launch_tiles<kTileRope>(a, "qkv", stream)) return rc;
+        if (int rc = launch_tiles<kTileRope>(a, plans.qkv, "qkv", stream)) return rc;
         if (int rc = mk_prefill_attention(&s, q, keys, values_t, attn, stream)) return rc;
         a = base;
         a.n = hid, a.k = H * D, a.x = attn, a.w0 = w.o + (size_t)layer * hid * H * D, a.out = h;
-        if (int rc = launch_tiles<kTileResidual>(a, "o", stream)) return rc;
+        if (int rc = launch_tiles<kTileResidual>(a, plans.o, "o", stream)) return rc;
         if (int rc = norm(w.mlp_norm + (size_t)layer * hid)) return rc;
         a = base;
         a.n = inter, a.k = hid, a.x = x, a.out = prod;
         a.w0 = w.gate + (size_t)layer * inter * hid, a.w1 = w.up + (size_t)layer * inter * hid;
-        if (int rc = launch_tiles<kTileSilu>(a, "gate and up", stream)) return rc;
+        if (int rc = launch_tiles<kTileSilu>(a, plans.up, "gate and up", stream)) return rc;
         a = base;
         a.n = hid, a.k = inter, a.x = prod, a.w0 = w.down + (size_t)layer * hid * inter, a.out = h;
-        if (int rc = launch_tiles<kTileResidual>(a, "down", stream)) return rc;
+        if (int rc = launch_tiles<kTileResidual>(a, plans.down, "down", stream)) return rc;
         if (int rc = norm(layer + 1 == w.num_layers ? w.final_norm : w.attn_norm + (size_t)(layer + 1) * hid)) return rc;
     }
     TileArgs a = base;
     a.n = s.vocab_size, a.k = hid, a.x = x, a.w0 = w.head;
-    if (int rc = launch_tiles<kTileArgmax>(a, "head", stream)) return rc;
-    const TilePlan plan = tile_plan(kTileArgmax, rows, s.vocab_size, hid);
-    tile_best_kernel<<<(rows + 15) / 16, 1024, 0, stream>>>(rows, plan.n_tiles * (kTileShapes[plan.shape].columns / 64), best, out_ids);
+    if (int rc = launch_tiles<kTileArgmax>(a, plans.head, "head", stream)) return rc;
+    tile_best_kernel<<<(rows + 15) / 16, 1024, 0, stream>>>(rows, plans.head.n_tiles * (kTileShapes[plans.head.shape].columns / 64), best, out_ids);
     return launched("best");
 }
 

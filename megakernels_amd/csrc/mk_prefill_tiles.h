@@ -159,73 +159,40 @@ __global__ __launch_bounds__(WN * 128, 2) void tile_kernel(TileArgs a) {
         asm volatile("" ::: "memory");
     };
     int i = 0;
-    if constexpr (MT * NT <= 4) {
-        // few products per operand: read a whole stage ahead
-        bf16x8 w[2][4][NT], x[2][4][MT];
-        auto stage = [&](int at, auto odd_, auto steady) {
-            constexpr int odd = decltype(odd_)::value;
-            if constexpr (steady) {
-                steady_arrive();  // every wave has read stage `at`, too
-                request(at + STAGES);
-            } else if (at + 1 < steps) {
-                arrive(at + 1);
-                if (at + STAGES < steps) request(at + STAGES);
-            }
-            if (steady || at + 1 < steps)
-#pragma unroll
-                for (int step = 0; step < 4; step++) read(at + 1, step, w[1 - odd][step], x[1 - odd][step]);
-#pragma unroll
-            for (int step = 0; step < 4; step++) multiply(w[odd][step], x[odd][step]);
-            if constexpr (steady) {
-#pragma unroll
-                for (int p = 0; p < 2 * MT * NT; p++) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);                // MFMA
-                    __builtin_amdgcn_sched_group_barrier(0x100, MT * NT == 2 ? 3 : 2, 0);  // LDS read
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            }
-        };
-#pragma unroll
-        for (int step = 0; step < 4; step++) read(0, step, w[0][step], x[0][step]);
-        for (; i + 1 + STAGES < steps; i += 2) {
-            stage(i, std::integral_constant<int, 0>{}, std::true_type{});
-            stage(i + 1, std::integral_constant<int, 1>{}, std::true_type{});
+    // few products per operand: read a whole stage ahead
+    bf16x8 w[2][4][NT], x[2][4][MT];
+    auto stage = [&](int at, auto odd_, auto steady) {
+        constexpr int odd = decltype(odd_)::value;
+        if constexpr (steady) {
+            steady_arrive();  // every wave has read stage `at`, too
+            request(at + STAGES);
+        } else if (at + 1 < steps) {
+            arrive(at + 1);
+            if (at + STAGES < steps) request(at + STAGES);
         }
-        for (; i < steps; i += 2) {
-            stage(i, std::integral_constant<int, 0>{}, std::false_type{});
-            if (i + 1 < steps) stage(i + 1, std::integral_constant<int, 1>{}, std::false_type{});
-        }
-    } else {
-        bf16x8 w[2][NT], x[2][MT];
-        auto stage = [&](int at, auto steady) {
+        if (steady || at + 1 < steps)
 #pragma unroll
-            for (int step = 0; step < 4; step++) {
-                if (step < 3) {
-                    read(at, step + 1, w[(step + 1) % 2], x[(step + 1) % 2]);
-                } else if constexpr (steady) {
-                    steady_arrive();  // every wave has read the last of stage `at`, too
-                    request(at + STAGES);
-                    read(at + 1, 0, w[0], x[0]);
-                } else if (at + 1 < steps) {
-                    arrive(at + 1);
-                    if (at + STAGES < steps) request(at + STAGES);
-                    read(at + 1, 0, w[0], x[0]);
-                }
-                multiply(w[step % 2], x[step % 2]);
-                if constexpr (steady) {
+            for (int step = 0; step < 4; step++) read(at + 1, step, w[1 - odd][step], x[1 - odd][step]);
 #pragma unroll
-                    for (int p = 0; p < MT + NT; p++) {
-                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // MFMA
-                        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // LDS read
-                    }
-                    __builtin_amdgcn_sched_group_barrier(0x008, MT * NT - MT - NT, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+        for (int step = 0; step < 4; step++) multiply(w[odd][step], x[odd][step]);
+        if constexpr (steady) {
+#pragma unroll
+            for (int p = 0; p < 2 * MT * NT; p++) {
+                __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);                // MFMA
+                __builtin_amdgcn_sched_group_barrier(0x100, MT * NT == 2 ? 3 : 2, 0);  // LDS read
             }
-        };
-        read(0, 0, w[0], x[0]);
-        for (; i + STAGES < steps; i++) stage(i, std::true_type{});
-        for (; i < steps; i++) stage(i, std::false_type{});
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#pragma unroll
+    for (int step = 0; step < 4; step++) read(0, step, w[0][step], x[0][step]);
+    for (; i + 1 + STAGES < steps; i += 2) {
+        stage(i, std::integral_constant<int, 0>{}, std::true_type{});
+        stage(i + 1, std::integral_constant<int, 1>{}, std::true_type{});
+    }
+    for (; i < steps; i += 2) {
+        stage(i, std::integral_constant<int, 0>{}, std::false_type{});
+        if (i + 1 < steps) stage(i + 1, std::integral_constant<int, 1>{}, std::false_type{});
     }
     __syncthreads();
 

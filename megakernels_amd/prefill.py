@@ -1,9 +1,9 @@
 """The prompt forward on the GPU: the dense forward of ``llama.py`` over whole prompts (``csrc/mk_prefill.hip``).
 
-PyTorch owns the memory and the stream.  A prompt of up to some thousand positions of a model up to 2048 wide runs as one
-call, its matrix products included.  For longer prompts and wider models PyTorch computes the plain products, and everything
-between them - embedding, RMS norm, residual adds, rotary embedding, cache append, causal attention, SiLU, argmax - is this
-library's.  There is no fallback for a missing library: a GPU forward that it covers raises ``RuntimeError``.
+PyTorch owns the memory and the stream.  A prompt of up to some thousand positions (of a model wider than 2048: of some
+hundred to two thousand) runs as one call, its matrix products included.  For the others PyTorch computes the plain products,
+and everything between them - embedding, RMS norm, residual adds, rotary embedding, cache append, causal attention, SiLU,
+argmax - is this library's.  There is no fallback for a missing library: a GPU forward that it covers raises ``RuntimeError``.
 """
 
 from __future__ import annotations
@@ -50,12 +50,11 @@ def load_library():
             function = getattr(lib, f"mk_prefill_{name}")
             function.argtypes = [ctypes.POINTER(Shape)] + [_P] * (count + 1)  # ... and the stream
             function.restype = ctypes.c_int
-        lib.mk_prefill_workspace_bytes.argtypes = [ctypes.POINTER(Shape)]
-        lib.mk_prefill_workspace_bytes.restype = ctypes.c_int64
-        lib.mk_prefill_forward.argtypes = [ctypes.POINTER(Shape), ctypes.POINTER(Model)] + [_P] * 6
-        lib.mk_prefill_forward.restype = ctypes.c_int
-        lib.mk_prefill_tile_plan.argtypes = [ctypes.POINTER(Shape), ctypes.c_int, ctypes.POINTER(_I)]
-        lib.mk_prefill_tile_plan.restype = ctypes.c_int
+        for kind, plan in (("", "tile"), ("wide_", "wide")):
+            workspace_bytes, forward, tiling = (getattr(lib, f"mk_prefill_{n}") for n in (f"{kind}workspace_bytes", f"{kind}forward", f"{plan}_plan"))
+            workspace_bytes.argtypes, workspace_bytes.restype = [ctypes.POINTER(Shape)], ctypes.c_int64
+            forward.argtypes, forward.restype = [ctypes.POINTER(Shape), ctypes.POINTER(Model)] + [_P] * 6, ctypes.c_int
+            tiling.argtypes, tiling.restype = [ctypes.POINTER(Shape), ctypes.c_int, ctypes.POINTER(_I)], ctypes.c_int
         lib.mk_prefill_last_error.restype = ctypes.c_char_p
         _lib = lib
     return _lib
@@ -133,11 +132,12 @@ def forward(model, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
     positions = positions.to(device=device, dtype=torch.int64).contiguous()
     shape = Shape(B, S, H, KVH, D, c.hidden_size, c.intermediate_size, c.vocab_size, k_cache.shape[2],
                   model.model.rope_cos.shape[0], int(bool(model.extra_config.interleave_rope)), c.rms_norm_eps)
-    workspace_bytes = lib.mk_prefill_workspace_bytes(ctypes.byref(shape))
-    if workspace_bytes < 0:
-        raise RuntimeError(f"mk_prefill_workspace_bytes: {lib.mk_prefill_last_error().decode()}")
-    if workspace_bytes:
-        return _forward_whole(lib, model, shape, workspace_bytes, ids, positions)
+    for whole in ("wide_", ""):
+        workspace_bytes = getattr(lib, f"mk_prefill_{whole}workspace_bytes")(ctypes.byref(shape))
+        if workspace_bytes < 0:
+            raise RuntimeError(f"mk_prefill_{whole}workspace_bytes: {lib.mk_prefill_last_error().decode()}")
+        if workspace_bytes:
+            return _forward_whole(lib, f"mk_prefill_{whole}forward", model, shape, workspace_bytes, ids, positions)
     padded = lib.mk_prefill_padded_seq(S)
 
     def rows(width):
@@ -168,7 +168,7 @@ def forward(model, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
     return h, out_ids
 
 
-def _forward_whole(lib, model, shape, workspace_bytes: int, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
+def _forward_whole(lib, entry: str, model, shape, workspace_bytes: int, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
     """A prompt that is not too long: one call launches the whole forward, matrix products included.  Issued one by one from
     Python, the launches of a short prompt took longer than the GPU needs for them."""
     c, device = model.config, ids.device
@@ -180,7 +180,7 @@ def _forward_whole(lib, model, shape, workspace_bytes: int, ids: Tensor, positio
     out_ids = torch.empty(ids.shape, dtype=torch.int64, device=device)
     with torch.cuda.device(device):
         stream = torch.cuda.current_stream(device).cuda_stream
-        if lib.mk_prefill_forward(ctypes.byref(shape), ctypes.byref(pointers), ids.data_ptr(), positions.data_ptr(), h.data_ptr(),
-                                       workspace.data_ptr(), out_ids.data_ptr(), stream) != 0:
-            raise RuntimeError(f"mk_prefill_forward: {lib.mk_prefill_last_error().decode()}")
+        if getattr(lib, entry)(ctypes.byref(shape), ctypes.byref(pointers), ids.data_ptr(), positions.data_ptr(), h.data_ptr(),
+                               workspace.data_ptr(), out_ids.data_ptr(), stream) != 0:
+            raise RuntimeError(f"{entry}: {lib.mk_prefill_last_error().decode()}")
     return h, out_ids

@@ -34,6 +34,11 @@ TILED_1B = [70, 150, 200, 300, 540, 777, 1020]
 TILED_HEAD = [(128256, 70), (128256, 200), (128200, 777)]                 # vocabulary, rows; 128200: a last tile of 200 columns
 TILED_WIDE_HEADS = [(2048, 700), (512, 1400)]                             # hidden size, rows
 TILED_ARGMAX = [(1048, 90), (10008, 300), (40008, 100), (40008, 200)]     # vocabulary, rows, of the tiny configuration
+# The same for the forward of wide tiles: layers of the 1B and of the 8B architecture, vocabularies for its last product, and
+# heads of 128 from a narrower hidden state.
+WIDE_1B = [257, 300, 400, 600, 1100, 1500, 2700, 4096]
+WIDE_8B = [705, 1100, 1300, 1700]
+WIDE_HEAD = [(8200, 300), (40008, 700)]                                   # vocabulary, rows; last tiles of 8 and 72 columns
 
 
 def _model(cfg, max_len, batch=1, interleave=True, seed=3):
@@ -178,6 +183,58 @@ def _first_of_equal_logits(vocab, seq):
         model_gpu = model.to("cuda:0")
         out = model_gpu(BatchState(input_ids=ids.to("cuda:0"), position_ids=torch.arange(seq, device="cuda:0"))).output_ids.cpu()
         assert bool((out == torch.where(logit > 0, first, 0))[sure].all())
+
+
+@pytest.mark.parametrize("seq", WIDE_1B)
+def test_every_wide_tiling_of_the_1b_layers(seq):
+    _compare(config_1b_slice(layers=1, vocab=1024), seq)
+
+
+@pytest.mark.parametrize("seq", WIDE_8B)
+def test_every_wide_tiling_of_the_8b_layers(seq):
+    _compare(config_8b_slice(inter=14336), seq, interleave=seq % 200 != 100)
+
+
+@pytest.mark.parametrize("interleave", [True, False])
+def test_wide_tiles_of_several_sequences_and_wide_heads(interleave):
+    _compare(config_1b_slice(layers=1, vocab=1024), 531, batch=3, interleave=interleave)
+    _compare(config_heads_wider_than_the_stream(1024), 1500, interleave=interleave)
+    _compare(config_heads_wider_than_the_stream(), 1900, interleave=interleave)
+    order = torch.randperm(900, generator=torch.Generator().manual_seed(1))[:777]
+    _compare(config_1b_slice(layers=1, vocab=1024), 777, positions=order, max_len=900, interleave=interleave)
+
+
+@pytest.mark.parametrize("vocab,seq", WIDE_HEAD)
+def test_wide_tiles_take_the_first_of_equal_logits(vocab, seq):
+    _first_of_equal_logits(vocab, seq)
+
+
+@pytest.mark.parametrize("vocab,seq", WIDE_HEAD)
+def test_argmax_of_wide_tiles_with_no_positive_logit_and_with_nan(vocab, seq):
+    cfg = config_tiny()
+    cfg.vocab_size, cfg.tie_word_embeddings = vocab, False
+    model = _model(cfg, seq)
+    head = model.lm_head.lm_head.weight
+    norm = model.lm_head.input_norm.weight
+    ids = torch.randint(0, cfg.vocab_size, (1, seq), generator=torch.Generator().manual_seed(0))
+    batch = BatchState(input_ids=ids.to("cuda:0"), position_ids=torch.arange(seq, device="cuda:0"))
+    norm.zero_()   # logits are zeros of both signs
+    assert bool((model.to("cuda:0")(batch).output_ids == 0).all())
+    norm.fill_(1.0)
+    head[4100], head[vocab - 1] = float("nan"), float("nan")   # above everything, the first of them
+    assert bool((model.to("cuda:0")(batch).output_ids == 4100).all())
+
+
+@pytest.mark.parametrize("seq", [300, 540, 777, 1020])
+def test_narrow_tiles_where_wide_ones_are_preferred(seq, monkeypatch):
+    lib = prefill.load_library()
+
+    class OnlyNarrow:
+        def __getattr__(self, name):
+            return (lambda shape: 0) if name == "mk_prefill_wide_workspace_bytes" else getattr(lib, name)
+
+    monkeypatch.setattr(prefill, "_lib", OnlyNarrow())
+    _compare(config_1b_slice(layers=1), seq)
 
 
 def test_prefill_of_few_rows_takes_the_first_of_equal_logits():
