@@ -478,17 +478,25 @@ int rows_split(int k) { return k >= 6144 ? 4 : 1; }
 
 template <int MT, int NT, int WAVES, int STAGES, int EPI, bool NORM>
 int launch_rows(const RowsArgs &a, int split, const char *what, hipStream_t stream) {
-    const int width = EPI == kRowsSilu ? 16 : NT * 16, bytes = RowsLds<MT, NT, WAVES, STAGES, NORM>::bytes(a.k);
+    const int width = EPI == kRowsSilu ? NT * 8 : NT * 16, bytes = RowsLds<MT, NT, WAVES, STAGES, NORM>::bytes(a.k);
     auto *kernel = rows_kernel<MT, NT, WAVES, STAGES, EPI, NORM>;
     const hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return fail(-5, "%s: %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
     kernel<<<dim3((a.n + width - 1) / width, split), WAVES * 64, bytes, stream>>>(a);
     return launched(what);
 }
-// Two tiles a block: two or three blocks of four waves fit a CU, and one's meeting is hidden by the others' loads.
+// Two tiles a block of four waves.  (One stage for more than 32 rows: 60 rows 1043 us, 1023 with two.)
 template <int MT, int EPI, bool NORM>
 int launch_rows_wide(const RowsArgs &a, int split, const char *what, hipStream_t stream) {
-    return launch_rows<MT, 2, 4, MT == 4 ? 1 : 2, EPI, NORM>(a, split, what, stream);
+    return launch_rows<MT, 2, 4, 2, EPI, NORM>(a, split, what, stream);
+}
+// Four tiles a block where there are enough columns (gate and up, LM head): a block reads X once, and with two tiles X's
+// bytes from L2 are as many as W's from memory.  Whole forwards of the 1B layers, us, two and four tiles: 12 rows 860 and
+// 843, 32 rows 925 and 898, 60 rows 1146 and 1073.
+constexpr int kRowsFar = 4;
+template <int MT, int EPI>
+int launch_rows_far(const RowsArgs &a, const char *what, hipStream_t stream) {
+    return launch_rows<MT, kRowsFar, 4, 1, EPI, true>(a, 1, what, stream);
 }
 // One tile a block: where there is at most one block per CU it has eight waves, so that the CU has enough loads in flight.
 // More blocks than CUs only queries, keys and values can have (above 4096 columns: heads wider than the hidden state).
@@ -507,9 +515,9 @@ int launch_rows(const RowsArgs &a, const char *what, hipStream_t stream) {
         if (a.rows <= 32) return launch_rows_narrow<2, EPI, NORM>(a, what, stream);
         return launch_rows_narrow<4, EPI, NORM>(a, what, stream);
     } else {
-        if (a.rows <= 16) return launch_rows_wide<1, EPI, NORM>(a, 1, what, stream);
-        if (a.rows <= 32) return launch_rows_wide<2, EPI, NORM>(a, 1, what, stream);
-        return launch_rows_wide<4, EPI, NORM>(a, 1, what, stream);
+        if (a.rows <= 16) return launch_rows_far<1, EPI>(a, what, stream);
+        if (a.rows <= 32) return launch_rows_far<2, EPI>(a, what, stream);
+        return launch_rows_far<4, EPI>(a, what, stream);
     }
 }
 
@@ -526,7 +534,7 @@ struct RowsWorkspace {
         values_t = keys + kv;
         arrived = values_t + kv;
         best = arrived + (s.hidden_size / 32 + 3) / 4 * 4 * 2;
-        partial = best + rows * ((s.vocab_size + 31) / 32 + 1) / 2 * 2 * 4;
+        partial = best + (rows * ((s.vocab_size + kRowsFar * 16 - 1) / (kRowsFar * 16)) + 1) / 2 * 2 * 4;
         const size_t sums = (rows <= 16 ? 16 : rows <= 32 ? 32 : 64) * (size_t)s.hidden_size;  // of one part of K
         const int split = max(rows_split(s.intermediate_size), rows_split(s.num_attention_heads * s.head_dim));
         total = partial + (split > 1 ? split * sums * 2 : 0);
@@ -824,15 +832,15 @@ int rows_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const int
         a = base;
         a.n = inter, a.k = hid, a.x = h, a.norm_weight = w.mlp_norm + (size_t)layer * hid, a.out = prod;
         a.w0 = w.gate + (size_t)layer * inter * hid, a.w1 = w.up + (size_t)layer * inter * hid;
-        if (int rc = launch_rows<2, kRowsSilu, true>(a, "gate and up", stream)) return rc;
+        if (int rc = launch_rows<kRowsFar, kRowsSilu, true>(a, "gate and up", stream)) return rc;
         a = base;
         a.n = hid, a.k = inter, a.x = prod, a.w0 = w.down + (size_t)layer * hid * inter, a.out = h;
         if (int rc = launch_rows<1, kRowsResidual, false>(a, "down", stream)) return rc;
     }
     RowsArgs a = base;
     a.n = s.vocab_size, a.k = hid, a.x = h, a.norm_weight = w.final_norm, a.w0 = w.head;
-    if (int rc = launch_rows<2, kRowsArgmax, true>(a, "head", stream)) return rc;
-    rows_best_kernel<<<rows, 256, 0, stream>>>((s.vocab_size + 31) / 32, best, out_ids);
+    if (int rc = launch_rows<kRowsFar, kRowsArgmax, true>(a, "head", stream)) return rc;
+    rows_best_kernel<<<rows, 256, 0, stream>>>((s.vocab_size + kRowsFar * 16 - 1) / (kRowsFar * 16), best, out_ids);
     return launched("best");
 }
 

@@ -2,7 +2,7 @@
 //
 // With M rows a weight element is used M times, so up to some hundred rows the time is the weights' bytes over the
 // memory rate plus what each launch adds.  Both ends shape the kernel below:
-//   * a block owns 16 (or 32) output columns and its waves split K, so that even a 2048-wide product has 128 blocks with
+//   * a block owns 16 to 64 output columns and its waves split K, so that even a 2048-wide product has 128 blocks with
 //     every wave's loads in flight at once.  Both operands go from memory straight into LDS in whole lines (a wave: eight
 //     rows of 128 bytes), each wave into a ring of its own, so the loop has no barrier; the partial sums meet in LDS.
 //     Loaded into registers in the order of v_mfma_f32_16x16x32_bf16 instead, every 16 lanes touch 16 lines and the L1
@@ -12,8 +12,9 @@
 // The norm needs no pass of its own: sum_k W[n,k] (h_k s w_k) = s sum_k W[n,k] (h_k w_k), and every block reads all of h
 // anyway, so it sums the squares on the way and scales the finished sums.  (One rounding, of h_k w_k, where the plain
 // forward has two.)
-// 32 rows of a 2.5 GB model: 2225 us as library products with Python launches, 890 to 940 here, from run to run (its bytes at
-// the rate of a copy, 4.9 TB/s: 507; at that of reads alone, 7.0 TB/s: 353).  64 rows: 1160.
+// 32 rows of a 2.5 GB model: 2225 us as library products with Python launches, 860 to 870 here (its bytes at the rate of a
+// copy, 4.9 TB/s: 507; at that of reads alone, 7.0 TB/s: 353).  60 rows: 1023.  More loads in flight (three or four stages,
+// twice the waves) change none of it: what is left is five launches a layer, each with its start from cold.
 // The blocks of a product read X again and again from L2 (M * K * 2 bytes each): the reason for the limit of kRowsMax.
 constexpr int kRowsMax = 64;
 
@@ -37,42 +38,43 @@ struct RowsArgs {
 __device__ __forceinline__ uint32_t order_bits(uint32_t bf16);
 __device__ __forceinline__ float silu(float g);
 
-// W row that lane `r` of the block's tile `t` holds
+// W row that lane `r` of the block's tile `t` holds (SiLU: the first half of the tiles are gate's, the others up's)
 template <int NT, int EPI>
 __device__ __forceinline__ int rows_weight_row(const RowsArgs &a, int t, int r) {
-    if constexpr (EPI == kRowsArgmax) return min((int)(blockIdx.x * NT + t) * 16 + r, a.n - 1);
-    const int first = EPI == kRowsSilu ? blockIdx.x * 16 : (blockIdx.x * NT + t) * 16, D = a.s.head_dim;
+    const int first = EPI == kRowsSilu ? (blockIdx.x * (NT / 2) + t % (NT / 2)) * 16 : (blockIdx.x * NT + t) * 16, D = a.s.head_dim;
     if (EPI == kRowsRope && !a.s.interleaved && first < (a.s.num_attention_heads + a.s.num_kv_heads) * D) {
         // the two members of a rotary pair are half a head apart: eight columns of each half
         return first / D * D + first % D / 2 + (r & 7) + (r >> 3) * (D / 2);
     }
-    return first + r;
+    return EPI == kRowsArgmax || EPI == kRowsSilu ? min(first + r, a.n - 1) : first + r;
 }
 
 // The fragments of COUNT tiles, 2048 bytes apart, read and waited for in one block of assembly: before an ordinary read of
 // LDS the compiler waits for every load into LDS that is still in flight.
 template <int COUNT>
 __device__ __forceinline__ void rows_read(u32x4 (&v)[COUNT], uint32_t at) {
-    static_assert(COUNT >= 2 && COUNT <= 6);
+    static_assert(COUNT >= 2 && COUNT <= 8);
+#define MK_READ(n, from, offset) "ds_read_b128 %" #n ", %" #from " offset:" #offset "\n\t"
     if constexpr (COUNT == 2)
-        asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:2048\n\ts_waitcnt lgkmcnt(0)"
-                     : "=&v"(v[0]), "=&v"(v[1]) : "v"(at) : "memory");
+        asm volatile(MK_READ(0, 2, 0) MK_READ(1, 2, 2048) "s_waitcnt lgkmcnt(0)" : "=&v"(v[0]), "=&v"(v[1]) : "v"(at) : "memory");
     else if constexpr (COUNT == 3)
-        asm volatile("ds_read_b128 %0, %3\n\tds_read_b128 %1, %3 offset:2048\n\tds_read_b128 %2, %3 offset:4096\n\ts_waitcnt lgkmcnt(0)"
+        asm volatile(MK_READ(0, 3, 0) MK_READ(1, 3, 2048) MK_READ(2, 3, 4096) "s_waitcnt lgkmcnt(0)"
                      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]) : "v"(at) : "memory");
     else if constexpr (COUNT == 4)
-        asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:2048\n\tds_read_b128 %2, %4 offset:4096\n\t"
-                     "ds_read_b128 %3, %4 offset:6144\n\ts_waitcnt lgkmcnt(0)"
+        asm volatile(MK_READ(0, 4, 0) MK_READ(1, 4, 2048) MK_READ(2, 4, 4096) MK_READ(3, 4, 6144) "s_waitcnt lgkmcnt(0)"
                      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]) : "v"(at) : "memory");
     else if constexpr (COUNT == 5)
-        asm volatile("ds_read_b128 %0, %5\n\tds_read_b128 %1, %5 offset:2048\n\tds_read_b128 %2, %5 offset:4096\n\t"
-                     "ds_read_b128 %3, %5 offset:6144\n\tds_read_b128 %4, %5 offset:8192\n\ts_waitcnt lgkmcnt(0)"
+        asm volatile(MK_READ(0, 5, 0) MK_READ(1, 5, 2048) MK_READ(2, 5, 4096) MK_READ(3, 5, 6144) MK_READ(4, 5, 8192) "s_waitcnt lgkmcnt(0)"
                      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]) : "v"(at) : "memory");
-    else
-        asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %6 offset:2048\n\tds_read_b128 %2, %6 offset:4096\n\t"
-                     "ds_read_b128 %3, %6 offset:6144\n\tds_read_b128 %4, %6 offset:8192\n\tds_read_b128 %5, %6 offset:10240\n\t"
+    else if constexpr (COUNT == 6)
+        asm volatile(MK_READ(0, 6, 0) MK_READ(1, 6, 2048) MK_READ(2, 6, 4096) MK_READ(3, 6, 6144) MK_READ(4, 6, 8192) MK_READ(5, 6, 10240)
                      "s_waitcnt lgkmcnt(0)"
                      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]) : "v"(at) : "memory");
+    else
+        asm volatile(MK_READ(0, 8, 0) MK_READ(1, 8, 2048) MK_READ(2, 8, 4096) MK_READ(3, 8, 6144) MK_READ(4, 8, 8192) MK_READ(5, 8, 10240)
+                     MK_READ(6, 8, 12288) MK_READ(7, 8, 14336) "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]), "=&v"(v[6]), "=&v"(v[7]) : "v"(at) : "memory");
+#undef MK_READ
 }
 // ... and the norm weights of the two halves of a step
 __device__ __forceinline__ void rows_read_norm(u32x4 (&v)[2], uint32_t at) {
@@ -176,13 +178,20 @@ __global__ __launch_bounds__(WAVES * 64) void rows_kernel(RowsArgs a) {
         for (int j = 0; j < kLoads; j++) {
             const int row = j % 2 * 8 + load_row, piece = (lane % 8) ^ ((row >> 1) & 7), t = j / 2;
             const uint16_t *const base = t >= NT ? a.x + (size_t)min((t - NT) * 16 + row, a.rows - 1) * a.k
-                                                 : (EPI == kRowsSilu && t == 1 ? a.w1 : a.w0) + (size_t)rows_weight_row<NT, EPI>(a, t, row) * a.k;
+                                                 : (EPI == kRowsSilu && t >= NT / 2 ? a.w1 : a.w0) + (size_t)rows_weight_row<NT, EPI>(a, t, row) * a.k;
             src[j] = base + (first_step + wave) * 64 + piece * 8;
         }
         auto request = [&](int i) {
             unsigned char *const slot = ring + i % STAGES * Lds::kStep;
 #pragma unroll
-            for (int j = 0; j < kLoads; j++) load_to_lds(src[j] + (size_t)i * (WAVES * 64), (MK_LDS void *)(slot + j * 1024));
+            for (int j = 0; j < kLoads; j++) {
+                // the weights past the caches: they are used once (32 rows of the 1B architecture 899 us without, 868)
+                constexpr int kPast = 2;
+                const MK_GLOBAL void *const from = (const MK_GLOBAL void *)(src[j] + (size_t)i * (WAVES * 64));
+                MK_LDS void *const to = (MK_LDS void *)(slot + j * 1024);
+                if (j < 2 * NT) __builtin_amdgcn_global_load_lds(from, to, 16, 0, kPast);
+                else __builtin_amdgcn_global_load_lds(from, to, 16, 0, 0);
+            }
         };
         const uint32_t read_at = (uint32_t)(uintptr_t)(MK_LDS unsigned char *)ring + r * 128, swizzle = (r >> 1) & 7;
         const uint32_t norm_at = (uint32_t)(uintptr_t)(MK_LDS unsigned char *)norm_lds + g * 16;
@@ -309,12 +318,17 @@ __global__ __launch_bounds__(WAVES * 64) void rows_kernel(RowsArgs a) {
         }
     } else if constexpr (EPI == kRowsSilu) {
         if (!valid) return;
-        u32x2 next;
 #pragma unroll
-        for (int j = 0; j < 2; j++)
-            next[j] = pack_bf16(round_bf16(silu(round_bf16(sum[0][2 * j]))) * round_bf16(sum[1][2 * j]),
-                                round_bf16(silu(round_bf16(sum[0][2 * j + 1]))) * round_bf16(sum[1][2 * j + 1]));
-        *(u32x2 *)(a.out + (size_t)row * a.n + (size_t)blockIdx.x * 16 + 4 * g) = next;
+        for (int t = 0; t < NT / 2; t++) {
+            const int column = (blockIdx.x * (NT / 2) + t) * 16 + 4 * g;
+            if (column >= a.n) continue;
+            u32x2 next;
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                next[j] = pack_bf16(round_bf16(silu(round_bf16(sum[t][2 * j]))) * round_bf16(sum[NT / 2 + t][2 * j]),
+                                    round_bf16(silu(round_bf16(sum[t][2 * j + 1]))) * round_bf16(sum[NT / 2 + t][2 * j + 1]));
+            *(u32x2 *)(a.out + (size_t)row * a.n + column) = next;
+        }
     } else if constexpr (EPI == kRowsArgmax) {
         uint64_t best = 0;
 #pragma unroll
