@@ -615,7 +615,9 @@ TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k, bool wide) {
             // more sums than fit one round of blocks cost more than the estimate (3000 rows of an 8B model's layers)
             if (wide && split > 1 && rounds > 1) break;
             const float meeting = split > 1 ? 3.0f + (float)split * rows * columns * 8 / 3e6f : 0.0f;
-            const float us = (float)rounds * ((stages + split - 1) / split) * t.stage_us + 3.0f + meeting;
+            float full = (float)rounds;
+            if (wide && shape == kSquare && (int64_t)m_tiles * n_tiles % t.slots && (int64_t)m_tiles * n_tiles % t.slots <= t.slots / 2) full -= 0.35f;  // halves
+            const float us = full * ((stages + split - 1) / split) * t.stage_us + 3.0f + meeting;
             if (best.split == 0 || us < best.us) best = {shape, split, m_tiles, n_tiles, us};
         }
     }

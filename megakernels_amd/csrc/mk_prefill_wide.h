@@ -253,13 +253,34 @@ __device__ __forceinline__ void wide_best(const TileArgs &a, int first, int g, R
 
 // ---- 256 x 256: waves of 128 rows x 64 columns, in quarters of 64 x 32; as many blocks as CUs, each with its list of tiles ----
 //
-// A tile of 64 elements of K is four pieces of 16 KB (columns 0-31 of every wave, rows 0-63, columns 32-63, rows 64-127) and
-// four phases.  The ring holds nine: seven ahead, one being read, one that the group behind may still be reading; and it runs
-// on across tiles, so that a tile's first operands arrive while the one before is finished.  At least four tiles of K.
+// A tile of 64 elements of K is four pieces of 16 KB (columns 0-31 of every wave, the tile's upper 128 rows, columns 32-63, the
+// lower 128 rows) and four phases.  The ring holds nine: seven ahead, one being read, one that the group behind may still be
+// reading; and it runs on across tiles, so that a tile's first operands arrive while the one before is finished.  At least four
+// tiles of K.
 // Products alone, output in bf16: 4096 x 16384 x 2048 198 us (the library 188), 176 without the stores, 1.56 PFLOP/s; 8192^3
 // 721 us (the library 681).  With what follows, 4096 rows: gate, up and SiLU 201 us (the library's products and a pass over
 // them 225), queries, keys and values with their rotation 64 (62), LM head with argmax 1467 (1817).
+//
+// Half a tile (128 rows) is two of the four phases and takes 0.65 of its time.  Where no more than half of an XCD's blocks
+// would have a tile in the last round, every block has half of one; and a tile whose lower rows are past the end is its upper
+// half.  Whole forwards, us: 8B architecture 2048 rows (gate and up: 3.5 rounds) 27180 -> 26750, 1B 1300 rows 4546 -> 4418.
 constexpr int kSquarePieces = 9, kSquareBytes = kSquarePieces * 16384;
+enum SquareRows { kAllRows, kUpperRows, kLowerRows };
+struct SquareItem {
+    int m, n;  // n < 0: there is none
+    SquareRows rows;
+};
+// item `local` of the list of XCD `xcd`, which `blocks` blocks work on (a product that is narrower than the chip has halves on
+// the XCDs with fewer tiles while the others work on whole ones, which is no gain: 4096 x 3072 64 -> 66 us, so rotation has none)
+template <int EPI>
+__device__ __forceinline__ SquareItem square_item(int local, int xcd, int m_tiles, int n_tiles, int blocks, int rows) {
+    const int tiles = (n_tiles - xcd + 7) / 8 * m_tiles, whole = tiles / blocks * blocks, left = tiles - whole;
+    const bool halves = EPI != kTileRope && local >= whole && 2 * left <= blocks;
+    const WideTile t = wide_tile(halves ? whole + (local - whole) / 2 : local, xcd, m_tiles, n_tiles);
+    const bool upper_only = rows - t.m * 256 <= 128;
+    if (halves && (local - whole) % 2) return {t.m, upper_only ? -1 : t.n, kLowerRows};
+    return {t.m, t.n, halves || upper_only ? kUpperRows : kAllRows};
+}
 
 template <int EPI>
 __global__ __launch_bounds__(512, 2) void square_kernel(TileArgs a) {
@@ -269,23 +290,24 @@ __global__ __launch_bounds__(512, 2) void square_kernel(TileArgs a) {
     extern __shared__ __align__(16) unsigned char lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / 64), lane = (int)threadIdx.x % 64;
     const int wave_m = wave / 4, wave_n = wave % 4, r16 = lane % 16, g = lane / 16;
-    const int m_tiles = (a.rows + 255) / 256, n_tiles = (a.n + kColumns - 1) / kColumns, xcd = blockIdx.x % 8, k_tiles = a.k / kTileK;
+    const int m_tiles = (a.rows + 255) / 256, n_tiles = (a.n + kColumns - 1) / kColumns, k_tiles = a.k / kTileK;
+    const int xcd = blockIdx.x % 8, blocks = gridDim.x / 8;
     const uint32_t k_bytes = (uint32_t)a.k * 2;
     int local = blockIdx.x / 8;
-    WideTile tile = wide_tile(local, xcd, m_tiles, n_tiles);
-    if (tile.n < 0) return;
+    SquareItem item = square_item<EPI>(local, xcd, m_tiles, n_tiles, blocks, a.rows);
+    if (item.n < 0) return;
 
     // a request of a wave moves eight rows of 128 bytes; two requests a piece
     uint32_t x_off[2][2], w_off[2][2];
     __amdgpu_buffer_rsrc_t x_buffer, w_buffer[2];
-    int k_at = 0;
+    int k_at = 0, put = 0, get = 0;
 #pragma unroll
     for (int j = 0; j < 2; j++) {
         const int row = wave * 16 + j * 8 + lane / 8, piece = (lane % 8) ^ ((row >> 1) & 7);
 #pragma unroll
-        for (int half = 0; half < 2; half++) x_off[half][j] = (uint32_t)(row / 64 * 128 + half * 64 + row % 64) * k_bytes + piece * 16;
+        for (int half = 0; half < 2; half++) x_off[half][j] = (uint32_t)(half * 128 + row) * k_bytes + piece * 16;
     }
-    auto point = [&](const WideTile &t) {
+    auto point = [&](const SquareItem &t) {
         x_buffer = buffer_of(a.x + (size_t)t.m * 256 * a.k, (uint32_t)min(256, a.rows - t.m * 256) * k_bytes);
         const size_t first = (size_t)t.n * kColumns;
         const uint32_t bytes = (uint32_t)min(kColumns, a.n - t.n * kColumns) * k_bytes;
@@ -301,17 +323,18 @@ __global__ __launch_bounds__(512, 2) void square_kernel(TileArgs a) {
             }
         k_at = 0;
     };
-    int put = 0, get = 0;
-    auto request = [&](auto piece_) {  // columns, rows, columns, rows
-        constexpr int piece = decltype(piece_)::value;
+    auto request_x = [&](const uint32_t (&off)[2], int at) {
         MK_LDS unsigned char *const dst = (MK_LDS unsigned char *)lds + put + wave * 2048;
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            if constexpr (piece % 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(x_buffer, (MK_LDS void *)(dst + j * 1024), 16, x_off[piece / 2][j], k_at, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(w_buffer[piece / 2], (MK_LDS void *)(dst + j * 1024), 16, w_off[piece / 2][j], k_at, 0, 0);
-        }
+        for (int j = 0; j < 2; j++) __builtin_amdgcn_raw_ptr_buffer_load_lds(x_buffer, (MK_LDS void *)(dst + j * 1024), 16, off[j], at, 0, 0);
         put = put + 16384 == kSquareBytes ? 0 : put + 16384;
-        if constexpr (piece == 3) k_at += 128;
+    };
+    auto request_w = [&](auto run_, int at) {
+        constexpr int run = decltype(run_)::value;
+        MK_LDS unsigned char *const dst = (MK_LDS unsigned char *)lds + put + wave * 2048;
+#pragma unroll
+        for (int j = 0; j < 2; j++) __builtin_amdgcn_raw_ptr_buffer_load_lds(w_buffer[run], (MK_LDS void *)(dst + j * 1024), 16, w_off[run][j], at, 0, 0);
+        put = put + 16384 == kSquareBytes ? 0 : put + 16384;
     };
     f32x4 acc[2][4][2][2];  // [half of the rows][16 rows][run][four columns]
     bf16x8 x[4][2], w[2][2][2];
@@ -349,75 +372,106 @@ __global__ __launch_bounds__(512, 2) void square_kernel(TileArgs a) {
     };
     constexpr std::integral_constant<int, 0> c0{};
     constexpr std::integral_constant<int, 1> c1{};
-    constexpr std::integral_constant<int, 2> c2{};
-    constexpr std::integral_constant<int, 3> c3{};
     auto k_tile = [&](auto newer_) {
         constexpr int newer = decltype(newer_)::value;
-        read_x(), request(c0), wide_operands<newer>(), multiply(c0, c0);
-        read_w(c1), request(c1), wide_operands<newer>(), multiply(c0, c1);
-        read_x(), request(c2), wide_operands<newer>(), multiply(c1, c0);
-        read_w(c0), request(c3), wide_operands<newer>(), multiply(c1, c1);
+        read_x(), request_w(c0, k_at), wide_operands<newer>(), multiply(c0, c0);
+        read_w(c1), request_x(x_off[0], k_at), wide_operands<newer>(), multiply(c0, c1);
+        read_x(), request_w(c1, k_at), wide_operands<newer>(), multiply(c1, c0);
+        read_w(c0), request_x(x_off[1], k_at), wide_operands<newer>(), multiply(c1, c1);
+        k_at += 128;
     };
-    auto start = [&]() {
-        point(tile);
-        put = get = 0;
-#pragma unroll
-        for (int t = 0; t < 2; t++) request(c0), request(c1), request(c2), request(c3);
+    // the ring is filled and its first piece read: the second group a barrier behind
+    auto begin = [&]() {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         wide_meet();
         if (wave_m) wide_meet();
         read_w(c0);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // its place is requested again in the next phase but one of the other group
     };
-    start();
-    while (true) {
-#pragma unroll
-        for (int i = 0; i < 32; i++) ((f32x4 *)acc)[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        // the stores of the tile before are newer than what this tile's first phases need
-        k_tile(std::integral_constant<int, kAhead + kStores>{});
-        for (int k = 1; k < k_tiles - 2; k++) k_tile(std::integral_constant<int, kAhead>{});
-        // the last two request the next tile's first; after the last tile this one's again, which nobody reads
-        const WideTile next = wide_tile(local += gridDim.x / 8, xcd, m_tiles, n_tiles);
-        point(EPI != kTileRope && next.n >= 0 ? next : tile);
-        k_tile(std::integral_constant<int, kAhead>{});
-        k_tile(std::integral_constant<int, kAhead>{});
-
+    auto end = [&]() {  // the groups side by side again, nothing on its way to LDS
+        if (!wave_m) wide_meet();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+    };
+    // HALVES halves of the item's rows from half `at` on, to where they belong
+    auto finish = [&](auto halves_, int at) {
+        constexpr int HALVES = decltype(halves_)::value;
         const int lane_of = here_of_lane(lane), g = lane_of / 16, r16 = lane_of % 16;
-        const int first = tile.n * 256 + wave_n * 64;
-        auto row_of = [&](int i) { return tile.m * 256 + wave_m * 128 + i * 16 + r16; };
+        const int first = item.n * 256 + wave_n * 64, top = item.m * 256 + at * 128;
+        auto row_of = [&](int i) { return top + i / 4 * 128 + wave_m * 64 + i % 4 * 16 + r16; };
         auto values = [&](int i) -> const f32x4(&)[2][2] { return acc[i / 4][i % 4]; };
         if constexpr (EPI == kTileRope) {
-            // the tables take the ring's place, 64 rows of each group at a time; few blocks have another tile after this one
-            if (!wave_m) wide_meet();
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            __syncthreads();
+            // the tables take the ring's place, 128 rows at a time
 #pragma unroll
-            for (int half = 0; half < 2; half++) {
-                wide_tables(a, lds, wave, lane_of, [&](int line) { return tile.m * 256 + line / 64 * 128 + half * 64 + line % 64; });
+            for (int half = 0; half < HALVES; half++) {
+                wide_tables(a, lds, wave, lane_of, [&](int line) { return top + half * 128 + line; });
                 wide_rope(a, lds, first, g, wave_m * 64 + r16, [&](int i) { return row_of(half * 4 + i); },
                           [&](int i) -> const f32x4(&)[2][2] { return acc[half][i]; });
                 __syncthreads();
             }
-            if (next.n < 0) return;
-            tile = next;
-            start();
-            continue;
-        }
-        if constexpr (EPI == kTileSilu) {
+        } else if constexpr (EPI == kTileSilu) {
             // a lane without a row or column stores outside the buffer: the count of stores is the same
-            const __amdgpu_buffer_rsrc_t out = buffer_of(a.out + (size_t)tile.m * 256 * a.n, (uint32_t)min(256, a.rows - tile.m * 256) * a.n * 2);
+            const __amdgpu_buffer_rsrc_t out = buffer_of(a.out + (size_t)item.m * 256 * a.n, (uint32_t)min(256, a.rows - item.m * 256) * a.n * 2);
             const int column = first / 2 + g * 8;
 #pragma unroll
-            for (int i = 0; i < 8; i++)
-                __builtin_amdgcn_raw_buffer_store_b128(wide_silu(values(i)), out, column < a.n ? ((uint32_t)(row_of(i) - tile.m * 256) * a.n + column) * 2 : kOutside, 0, 2);
-        } else if constexpr (EPI == kTileArgmax) {
-            wide_best<8>(a, first, g, row_of, values);
+            for (int i = 0; i < HALVES * 4; i++)
+                __builtin_amdgcn_raw_buffer_store_b128(wide_silu(values(i)), out, column < a.n ? ((uint32_t)(row_of(i) - item.m * 256) * a.n + column) * 2 : kOutside, 0, 2);
+        } else {
+            wide_best<HALVES * 4>(a, first, g, row_of, values);
         }
-        if (next.n < 0) break;
-        tile = next;
+    };
+    bool begun = false;
+    while (true) {
+#pragma unroll
+        for (int i = 0; i < 32; i++) ((f32x4 *)acc)[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        // (the compiler is told that these are the same for the whole wave, and the buffers are made anew for every item: once it
+        // took them for the lanes' own, every request became a loop over the lanes' addresses)
+        item = {__builtin_amdgcn_readfirstlane(item.m), __builtin_amdgcn_readfirstlane(item.n), (SquareRows)__builtin_amdgcn_readfirstlane(item.rows)};
+        put = __builtin_amdgcn_readfirstlane(put), get = __builtin_amdgcn_readfirstlane(get);
+        local = __builtin_amdgcn_readfirstlane(local) + blocks;
+        const SquareItem next = square_item<EPI>(local, xcd, m_tiles, n_tiles, blocks, a.rows);
+        // rotation needs LDS, and half a tile uses the ring in another order: the ring does not run on across those
+        const bool goes_on = EPI != kTileRope && item.rows == kAllRows && next.n >= 0 && next.rows == kAllRows;
+        if (item.rows == kAllRows) {
+            point(item);
+            if (!begun) {
+                put = get = 0;
+#pragma unroll
+                for (int t = 0; t < 2; t++) request_w(c0, t * 128), request_x(x_off[0], t * 128), request_w(c1, t * 128), request_x(x_off[1], t * 128);
+                begin();
+            }
+            k_at = 256;
+            // the stores of the tile before are newer than what this tile's first phases need
+            k_tile(std::integral_constant<int, kAhead + kStores>{});
+            for (int k = 1; k < k_tiles - 2; k++) k_tile(std::integral_constant<int, kAhead>{});
+            // the last two request the next tile's first; where there is none, this one's again, which nobody reads
+            point(goes_on ? next : item);
+            k_tile(std::integral_constant<int, kAhead>{});
+            k_tile(std::integral_constant<int, kAhead>{});
+            if (!goes_on) end();
+            finish(std::integral_constant<int, 2>{}, 0);
+        } else {
+            // per tile of K: one piece of rows, then both of columns, the second already the next tile's; three tiles ahead, past
+            // the end of K too, where nobody reads what arrives
+            uint32_t off[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) off[j] = item.rows == kLowerRows ? x_off[1][j] : x_off[0][j];
+            point(item);
+            put = get = 0;
+            request_w(c0, 0), request_x(off, 0), request_w(c1, 0), request_w(c0, 128), request_x(off, 128), request_w(c1, 128), request_w(c0, 256);
+            begin();
+            for (int k = 0; k < k_tiles; k++) {
+                read_x(), request_x(off, k_at + 256), wide_operands<8>(), multiply(c0, c0);
+                read_w(c1), read_w(c0), request_w(c1, k_at + 256), request_w(c0, k_at + 384), wide_operands<10>(), multiply(c0, c1);
+                k_at += 128;
+            }
+            end();
+            finish(std::integral_constant<int, 1>{}, item.rows == kLowerRows);
+        }
+        if (next.n < 0) return;
+        begun = goes_on;
+        item = next;
     }
-    if (!wave_m) wide_meet();
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last requests write to LDS
 }
 
 // ---- 128 x 256: a tile's K is split between the two groups, which add their sums at the end ----
