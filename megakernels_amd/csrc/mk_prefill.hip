@@ -592,7 +592,7 @@ constexpr TileShape kTileShapes[] = {
     {256, 256, 256, 1.40f},  // square_kernel: the most work per byte of LDS
     {128, 256, 256, 0.84f},  // flat_kernel
 };
-constexpr int kSquare = 3, kFlat = 4, kSquareLeastK = 4 * kTileK;
+constexpr int kSquare = 3, kFlat = 4, kWideLeastK = 4 * kTileK;
 struct TilePlan {
     int shape, split, m_tiles, n_tiles;
     float us;
@@ -607,7 +607,7 @@ TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k, bool wide) {
     TilePlan best{};
     for (int shape = 0; shape <= (wide ? kFlat : kSquare); shape++) {
         const TileShape &t = kTileShapes[shape];
-        if (shape == kSquare && (epilogue == kTileResidual || k < kSquareLeastK)) continue;
+        if ((shape == kSquare && epilogue == kTileResidual) || (shape >= kSquare && k < kWideLeastK)) continue;
         const int m_tiles = (rows + t.rows - 1) / t.rows, n_tiles = (columns + t.columns - 1) / t.columns, stages = k / kTileK;
         for (int split = 1; split <= 8; split *= 2) {
             if (split > 1 && (whole || stages / split < 8 || shape == kSquare)) break;

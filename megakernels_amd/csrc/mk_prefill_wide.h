@@ -478,8 +478,9 @@ __global__ __launch_bounds__(512, 2) void square_kernel(TileArgs a) {
 //
 // Each group takes 32 of every 64 elements of K, with waves of 128 rows x 64 columns as above: tiles half as large for as few
 // reads of LDS per product.  (Waves of 64 x 64 would need a third more than LDS delivers beside the matrix cores.)  The
-// ring holds three tiles of 64 elements of K.  Products alone: 4096 x 2048 x 8192 113 us, 1.22 PFLOP/s (the library 110),
-// 4096 x 2048 x 2048 35 (33), 2048 x 4096 x 14336 201 (206).  777 x 2048 x 8192 with K in four parts: 43 us, 46 as 128 x 128
+// ring holds three tiles of 64 elements of K, requested three phases ahead; a block's share is at least three.  Products alone, when a phase read eight fragments
+// and the next four: 4096 x 2048 x 8192 113 us, 1.22 PFLOP/s (the library 110), 4096 x 2048 x 2048 35 (33), 2048 x 4096 x
+// 14336 201 (206); with six and six the whole forward of 4096 tokens of the 1B architecture went from 9890 to 9730 us.  777 x 2048 x 8192 with K in four parts: 43 us, 46 as 128 x 128
 // in two.
 // K may also be split over gridDim.y blocks, whose sums meet in memory as in tile_kernel.
 constexpr int kFlatStage = 49152, kFlatBytes = 3 * kFlatStage;
@@ -512,72 +513,86 @@ __global__ __launch_bounds__(512, 2) void flat_kernel(TileArgs a) {
         const int row = wave / 2 * 64 + j * 16 + wave % 2 * 8 + lane / 8;
         w_off[j] = (uint32_t)wide_weight_row<EPI>(a, tile.n, row) * k_bytes + ((lane % 8) ^ ((row >> 1) & 7)) * 16;
     }
-    int put = 0, get = 0;
-    auto request_first = [&](int t) {  // rows 0-63 and the columns
-        MK_LDS unsigned char *const dst = (MK_LDS unsigned char *)lds + put;
-        const int k_at = (first_step + t) * 128;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(x_buffer, (MK_LDS void *)(dst + wave * 1024), 16, x_off[0], k_at, 0, 0);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            MK_LDS void *const at = (MK_LDS void *)(dst + 16384 + wave / 2 * 8192 + j * 2048 + wave % 2 * 1024);
-            if (j < 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(w0_buffer, at, 16, w_off[j], k_at, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(w1_buffer, at, 16, w_off[j], k_at, 0, 0);
-        }
+    // places in the ring of tile t, t + 1 and t + 2 of K (that of t is t + 3's, too), and requests to them
+    int place = 0, next_place = kFlatStage, far_place = 2 * kFlatStage;
+    auto request_rows = [&](int t, int to, int half) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(x_buffer, (MK_LDS void *)((MK_LDS unsigned char *)lds + to + half * 8192 + wave * 1024), 16, x_off[half],
+                                                 (first_step + t) * 128, 0, 0);
     };
-    auto request_second = [&](int t) {  // rows 64-127
-        MK_LDS unsigned char *const dst = (MK_LDS unsigned char *)lds + put;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(x_buffer, (MK_LDS void *)(dst + 8192 + wave * 1024), 16, x_off[1], (first_step + t) * 128, 0, 0);
-        put = put + kFlatStage == kFlatBytes ? 0 : put + kFlatStage;
+    auto request_columns = [&](int t, int to, auto run_) {
+        constexpr int run = decltype(run_)::value;
+#pragma unroll
+        for (int j = run * 2; j < run * 2 + 2; j++)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(run ? w1_buffer : w0_buffer,
+                                                     (MK_LDS void *)((MK_LDS unsigned char *)lds + to + 16384 + wave / 2 * 8192 + j * 2048 + wave % 2 * 1024), 16,
+                                                     w_off[j], (first_step + t) * 128, 0, 0);
     };
     f32x4 acc[2][4][2][2];
 #pragma unroll
     for (int i = 0; i < 32; i++) ((f32x4 *)acc)[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    bf16x8 x[4], w[4];
+    bf16x8 x[4], first_run[2][2], second_run[2];  // first run of columns: of even and odd tiles of K
     const uint32_t at = r16 * 128 + ((group * 4 + g) ^ ((r16 >> 1) & 7)) * 16;
     auto read_x = [&](int half) {
-        const unsigned char *const base = lds + get + half * 8192 + at;
+        const unsigned char *const base = lds + place + half * 8192 + at;
 #pragma unroll
         for (int i = 0; i < 4; i++) x[i] = *(const bf16x8 *)(base + i * 2048);
-        if (half) get = get + kFlatStage == kFlatBytes ? 0 : get + kFlatStage;
     };
-    auto read_w = [&]() {
-        const unsigned char *const base = lds + get + 16384 + wave_n * 8192 + at;
+    auto read_w = [&](int from, int run, bf16x8 (&to)[2]) {
+        const unsigned char *const base = lds + from + 16384 + wave_n * 8192 + run * 4096 + at;
 #pragma unroll
-        for (int j = 0; j < 4; j++) w[j] = *(const bf16x8 *)(base + j * 2048);
+        for (int j = 0; j < 2; j++) to[j] = *(const bf16x8 *)(base + j * 2048);
     };
-    auto multiply = [&](auto half_) {
-        constexpr int half = decltype(half_)::value;
+    auto multiply = [&](auto half_, auto odd_) {
+        constexpr int half = decltype(half_)::value, odd = decltype(odd_)::value;
         __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                acc[half][i][j / 2][j % 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j], x[i], acc[half][i][j / 2][j % 2], 0, 0, 0);
+                acc[half][i][j / 2][j % 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(j < 2 ? first_run[odd][j] : second_run[j - 2], x[i], acc[half][i][j / 2][j % 2], 0, 0, 0);
         __builtin_amdgcn_s_setprio(0);
         wide_meet();
     };
     constexpr std::integral_constant<int, 0> c0{};
     constexpr std::integral_constant<int, 1> c1{};
-    request_first(0), request_second(0);
-    if (steps > 1) {
-        request_first(1), request_second(1);
-        asm volatile("s_waitcnt vmcnt(7)" ::: "memory");
-    } else {
-        asm volatile("s_waitcnt vmcnt(1)" ::: "memory");
-    }
+    // The first run of a tile's columns is read a phase early, so that both phases of a tile read six fragments.  LEFT: tiles
+    // of K that follow, where they are few.
+    request_columns(0, place, c0);
+    request_rows(0, place, 0), request_columns(0, place, c1);
+    request_rows(0, place, 1), request_columns(1, next_place, c0);
+    request_rows(1, next_place, 0), request_columns(1, next_place, c1);
+    request_rows(1, next_place, 1), request_columns(2, far_place, c0);
+    asm volatile("s_waitcnt vmcnt(9)" ::: "memory");
     wide_meet();
     if (group) wide_meet();
+    auto k_tile = [&](int t, auto odd_, auto left_) {
+        constexpr int odd = decltype(odd_)::value, left = decltype(left_)::value;
+        constexpr std::integral_constant<int, odd> parity{};
+        read_x(0), read_w(place, 1, second_run);
+        if constexpr (left >= 2) request_rows(t + 2, far_place, 0), request_columns(t + 2, far_place, c1);
+        wide_operands<left >= 2 ? 9 : left == 1 ? 4 : 0>(), multiply(c0, parity);
+        read_x(1);
+        if constexpr (left >= 1) read_w(next_place, 0, first_run[1 - odd]);
+        if constexpr (left >= 2) request_rows(t + 2, far_place, 1);
+        if constexpr (left >= 3) request_columns(t + 3, place, c0);
+        wide_operands<left >= 3 ? 9 : left == 2 ? 7 : left == 1 ? 1 : 0>(), multiply(c1, parity);
+        const int passed = place;
+        place = next_place, next_place = far_place, far_place = passed;
+    };
+    constexpr std::integral_constant<int, 3> many{};
     int t = 0;
-    for (; t + 2 < steps; t++) {
-        read_w(), read_x(0), request_first(t + 2), wide_operands<11>(), multiply(c0);
-        read_x(1), request_second(t + 2), wide_operands<7>(), multiply(c1);
+    if (steps % 2 == 0) {  // an odd number before the last three
+        read_w(place, 0, first_run[1]);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        k_tile(t++, c1, many);
+    } else {
+        read_w(place, 0, first_run[0]);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     }
-    if (t + 1 < steps) {
-        read_w(), read_x(0), wide_operands<6>(), multiply(c0);
-        read_x(1), wide_operands<1>(), multiply(c1);
-    }
-    read_w(), read_x(0), wide_operands<0>(), multiply(c0);
-    read_x(1), wide_operands<0>(), multiply(c1);
+    for (; t + 3 < steps; t += 2) k_tile(t, c0, many), k_tile(t + 1, c1, many);
+    k_tile(t, c0, std::integral_constant<int, 2>{});
+    k_tile(t + 1, c1, c1);
+    k_tile(t + 2, c0, c0);
     if (!group) wide_meet();
 
     const int first = tile.n * 256 + wave_n * 64;
