@@ -79,7 +79,7 @@ int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *mo
 int mk_prefill_tile_plan(const mk_prefill_shape *shape, int product, int32_t plan[4]);
 
 /* The whole forward of longer prompts and wider models, from wide tiles; arguments as above.  Workspace 0: not such a call -
- * up to 256 or more than 4096 rows (of a model wider than 2048: up to 704 or more than 2048), a hidden size below 256 or no
+ * up to 256 or more than 4096 rows (of a model wider than 2048: up to 512 or more than 2048), a hidden size below 256 or no
  * multiple of 64, an intermediate size that is no multiple of 64, a cache of 2^31 rows. */
 int64_t mk_prefill_wide_workspace_bytes(const mk_prefill_shape *shape);
 int mk_prefill_wide_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids,

@@ -565,15 +565,15 @@ bool tiles_cover(const mk_prefill_shape &s) {
     return whole_covers(s) && rows <= 4096 && rows * s.hidden_size <= 1 << 21;
 }
 // Wide tiles (mk_prefill_wide.h) beside the narrower ones.  Whole forwards, us, narrow tiles or the library's products, and wide:
-//   1B architecture: 253 rows 1749 and 1747, 320 rows 2117 and 2028, 777 rows 2971 and 2885, 1024 rows 3325 and 3191 (tiles);
-//     1100 rows 4343 and 4100, 1500 rows 4782 and 4601, 2048 rows 5879 and 5329, 4096 rows 10876 and 9999 (library)
-//   8B architecture: 520 rows 11766 and 11541, 640 rows 12443 and 12949, 700 rows 13312 and 13027, 777 rows 14972 and 13715,
-//     2048 rows 28628 and 27299, 3000 rows 40426 and 43355, 4096 rows 52510 and 53104 (library)
-// Prompts of up to 512 rows of wide models are the library's for the reason above, those up to 704 for want of a gain.
+//   1B architecture: 253 rows 1752 and 1752, 320 rows 2132 and 2034, 777 rows 2971 and 2829, 1024 rows 3325 and 3191 (tiles);
+//     1100 rows 4343 and 4100, 1500 rows 4782 and 4601, 2048 rows 5879 and 5329, 4096 rows 10982 and 10181 (library)
+//   8B architecture: 520 rows 11889 and 11437, 640 rows 12608 and 12239, 777 rows 15119 and 13540, 2048 rows 28328 and 26686,
+//     2300 rows 31529 and 34397, 2600 rows 44288 and 38257, 3000 rows 41329 and 43537, 4096 rows 53581 and 54067 (library)
+// Prompts of up to 512 rows of wide models are the library's for the reason above.
 bool wide_covers(const mk_prefill_shape &s) {
     const int64_t rows = (int64_t)s.batch * s.seq;
     const bool narrow = s.hidden_size <= 2048;
-    return s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0 && s.hidden_size >= 256 && rows > (narrow ? 256 : 704) && rows <= (narrow ? 4096 : 2048)
+    return s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0 && s.hidden_size >= 256 && rows > (narrow ? 256 : 512) && rows <= (narrow ? 4096 : 2048)
         && (int64_t)s.batch * s.kv_max_len < INT32_MAX;
 }
 

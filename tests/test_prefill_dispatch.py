@@ -187,7 +187,7 @@ def _wide_workspace(rows, hidden, batch=1, inter=None, max_len=8192):
     return prefill.load_library().mk_prefill_wide_workspace_bytes(ctypes.byref(shape))
 
 
-@pytest.mark.parametrize("hidden,least,most", [(256, 257, 4096), (1024, 257, 4096), (2048, 257, 4096), (2112, 705, 2048), (4096, 705, 2048), (8192, 705, 2048)])
+@pytest.mark.parametrize("hidden,least,most", [(256, 257, 4096), (1024, 257, 4096), (2048, 257, 4096), (2112, 513, 2048), (4096, 513, 2048), (8192, 513, 2048)])
 def test_prompts_that_wide_tiles_take(hidden, least, most):
     assert _wide_workspace(least, hidden) > 0 and _wide_workspace(most, hidden) > 0 and _wide_workspace(most, hidden, batch=2) > 0
     assert _wide_workspace(least - 1, hidden) == 0 and _wide_workspace(most + 1, hidden) == 0
@@ -210,7 +210,7 @@ def test_the_gpu_tests_reach_every_wide_tiling_of_the_1b_and_8b_layers():
     reached = {_wide_plan(product, rows, vocab=1024) for rows in gpu.WIDE_1B for product in range(5)}
     assert {_wide_plan(product, rows) for rows in range(257, 4097) for product in range(4)} <= reached
     reached |= {_wide_plan(product, rows, vocab=4096, **of_8b) for rows in gpu.WIDE_8B for product in range(5)}
-    assert {_wide_plan(product, rows, **of_8b) for rows in range(705, 2049) for product in range(4)} <= reached
+    assert {_wide_plan(product, rows, **of_8b) for rows in range(513, 2049) for product in range(4)} <= reached
     reached |= {_wide_plan(head, rows, 512, 1024, 8, 2, vocab=vocab) for vocab, rows in gpu.WIDE_HEAD}
     assert {_wide_plan(head, rows) for rows in range(257, 4097)} <= reached
     # products that K is not split for run in 128 x 256 and 256 x 256, the residual ones in 128 x 256
@@ -230,7 +230,7 @@ def test_tile_plans_are_refused_where_nothing_is_tiled():
 def test_wide_plans_and_forwards_are_refused_where_there_are_none():
     lib = prefill.load_library()
     plan = (ctypes.c_int32 * 4)()
-    for rows, hidden, product in ((256, 2048, 0), (4097, 2048, 0), (704, 4096, 0), (2049, 4096, 0), (1000, 2048, 5), (1000, 2048, -1)):
+    for rows, hidden, product in ((256, 2048, 0), (4097, 2048, 0), (512, 4096, 0), (2049, 4096, 0), (1000, 2048, 5), (1000, 2048, -1)):
         shape = prefill.Shape(1, rows, 32, 8, 64, hidden, 8192, 32768, rows, rows, 1, 1e-5)
         assert lib.mk_prefill_wide_plan(ctypes.byref(shape), product, plan) < 0 and lib.mk_prefill_last_error()
     shape = prefill.Shape(1, 1000, 32, 8, 64, 2048, 8192, 32768, 1000, 1000, 1, 1e-5)
