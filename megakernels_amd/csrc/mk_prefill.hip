@@ -574,7 +574,9 @@ bool wide_covers(const mk_prefill_shape &s) {
     const int64_t rows = (int64_t)s.batch * s.seq;
     const bool narrow = s.hidden_size <= 2048;
     return s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0 && s.hidden_size >= 256 && rows > (narrow ? 256 : 512) && rows <= (narrow ? 4096 : 2048)
-        && (int64_t)s.batch * s.kv_max_len < INT32_MAX;
+        && (int64_t)s.batch * s.kv_max_len < INT32_MAX
+        // (offsets of 32 bits within a tile's rows)
+        && s.intermediate_size <= 1 << 20 && s.num_kv_heads <= 1 << 10;
 }
 
 // ---- more rows: tiles, narrow and wide ----

@@ -4,8 +4,8 @@
 // K goes through a ring of LDS stages of 64 elements, filled by loads that go from memory straight into LDS (eight rows of
 // 128 bytes a wave; 16-byte pieces swizzled so that a wave's reads spread over all banks) and stay in flight across the one
 // barrier of a stage: each wave waits for its own loads of the next stage, then meets the others.  A wave reads the operands
-// of its next 16 elements of K before it multiplies the current ones, also across that barrier.  Operands are swapped (w first), so that a lane holds four neighbouring columns
-// of one row: rotary pairs and gate and up of one output lie in one lane.
+// of its next stage before it multiplies the current one's, also across that barrier.  Operands are swapped (w first), so that
+// a lane holds four neighbouring columns of one row: rotary pairs and gate and up of one output lie in one lane.
 constexpr int kTileK = 64;
 
 enum TileEpilogue { kTileRope, kTileResidual, kTileSilu, kTileArgmax };

@@ -477,11 +477,11 @@ __global__ __launch_bounds__(512, 2) void square_kernel(TileArgs a) {
 // ---- 128 x 256: a tile's K is split between the two groups, which add their sums at the end ----
 //
 // Each group takes 32 of every 64 elements of K, with waves of 128 rows x 64 columns as above: tiles half as large for as few
-// reads of LDS per product.  (Waves of 64 x 64 would need a third more than LDS delivers beside the matrix cores.)  The
-// ring holds three tiles of 64 elements of K, requested three phases ahead; a block's share is at least three.  Products alone, when a phase read eight fragments
-// and the next four: 4096 x 2048 x 8192 113 us, 1.22 PFLOP/s (the library 110), 4096 x 2048 x 2048 35 (33), 2048 x 4096 x
-// 14336 201 (206); with six and six the whole forward of 4096 tokens of the 1B architecture went from 9890 to 9730 us.  777 x 2048 x 8192 with K in four parts: 43 us, 46 as 128 x 128
-// in two.
+// reads of LDS per product.  (Waves of 64 x 64 would need a third more than LDS delivers beside the matrix cores.)  The ring
+// holds three tiles of 64 elements of K, requested three phases ahead; a block's share is at least three.
+// Products alone, when a phase read eight fragments and the next four: 4096 x 2048 x 8192 113 us, 1.22 PFLOP/s (the library
+// 110), 4096 x 2048 x 2048 35 (33), 2048 x 4096 x 14336 201 (206).  With six and six the whole forward of 4096 tokens of the 1B
+// architecture went from 9890 to 9732 us.  777 x 2048 x 8192 with K in four parts: 43 us, 46 as 128 x 128 in two.
 // K may also be split over gridDim.y blocks, whose sums meet in memory as in tile_kernel.
 constexpr int kFlatStage = 49152, kFlatBytes = 3 * kFlatStage;
 

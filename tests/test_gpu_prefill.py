@@ -313,6 +313,27 @@ def test_whole_forward_in_a_captured_graph(seq):
         assert torch.equal(out.hidden_states, expected) and bool(model.stacked_kv_cache[0].any())
 
 
+@pytest.mark.parametrize("seq", [300, 1100])
+def test_wide_forward_in_a_captured_graph(seq):
+    cfg = config_1b_slice(layers=1, vocab=1024)
+    model = _model(cfg, seq).to("cuda:0")
+    batch = BatchState(input_ids=torch.randint(0, cfg.vocab_size, (1, seq), device="cuda:0"), position_ids=torch.arange(seq, device="cuda:0"))
+    expected = model(batch)
+    hidden, ids = expected.hidden_states.clone(), expected.output_ids.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = model(batch)
+    for _ in range(3):
+        model.stacked_kv_cache[0].zero_()
+        with torch.inference_mode():
+            out.hidden_states.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.hidden_states, hidden) and torch.equal(out.output_ids, ids) and bool(model.stacked_kv_cache[0].any())
+        assert torch.equal(model(batch).hidden_states, hidden)
+
+
 def test_argmax_takes_the_first_maximum_and_nan_above_all():
     lib = prefill.load_library()
     import ctypes
