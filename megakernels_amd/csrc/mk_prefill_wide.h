@@ -257,7 +257,7 @@ __device__ __forceinline__ void wide_best(const TileArgs &a, int first, int g, R
 // lower 128 rows) and four phases.  The ring holds nine: seven ahead, one being read, one that the group behind may still be
 // reading; and it runs on across tiles, so that a tile's first operands arrive while the one before is finished.  At least four
 // tiles of K.
-// Products alone, output in bf16: 4096 x 16384 x 2048 198 us (the library 188), 176 without the stores, 1.56 PFLOP/s; 8192^3
+// Products alone, output in bf16: 4096 x 16384 x 2048 198 us past the caches (the library 188), 176 without the stores, 1.56 PFLOP/s; 8192^3
 // 721 us (the library 681).  With what follows, 4096 rows: gate, up and SiLU 201 us (the library's products and a pass over
 // them 225), queries, keys and values with their rotation 64 (62), LM head with argmax 1467 (1817).
 //
@@ -410,12 +410,14 @@ __global__ __launch_bounds__(512, 2) void square_kernel(TileArgs a) {
                 __syncthreads();
             }
         } else if constexpr (EPI == kTileSilu) {
-            // a lane without a row or column stores outside the buffer: the count of stores is the same
+            // a lane without a row or column stores outside the buffer: the count of stores is the same.  (Past the caches these
+            // stores are over sooner, but the next product reads what they wrote: whole forwards of 1300 rows of the 1B
+            // architecture 4127 us, 4082 through them, 4096 rows 9705 and 9593, 2048 rows of the 8B one 26340 and 25830.)
             const __amdgpu_buffer_rsrc_t out = buffer_of(a.out + (size_t)item.m * 256 * a.n, (uint32_t)min(256, a.rows - item.m * 256) * a.n * 2);
             const int column = first / 2 + g * 8;
 #pragma unroll
             for (int i = 0; i < HALVES * 4; i++)
-                __builtin_amdgcn_raw_buffer_store_b128(wide_silu(values(i)), out, column < a.n ? ((uint32_t)(row_of(i) - item.m * 256) * a.n + column) * 2 : kOutside, 0, 2);
+                __builtin_amdgcn_raw_buffer_store_b128(wide_silu(values(i)), out, column < a.n ? ((uint32_t)(row_of(i) - item.m * 256) * a.n + column) * 2 : kOutside, 0, 0);
         } else {
             wide_best<HALVES * 4>(a, first, g, row_of, values);
         }
