@@ -575,8 +575,8 @@ bool wide_covers(const mk_prefill_shape &s) {
     const bool narrow = s.hidden_size <= 2048;
     return s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0 && s.hidden_size >= 256 && rows > (narrow ? 256 : 512) && rows <= (narrow ? 4096 : 2048)
         && (int64_t)s.batch * s.kv_max_len < INT32_MAX
-        // (offsets of 32 bits within a tile's rows)
-        && s.intermediate_size <= 1 << 20 && s.num_kv_heads <= 1 << 10;
+        // (offsets of 32 bits within a tile's rows, of K as of the columns)
+        && s.intermediate_size <= kWideMostColumns && s.num_kv_heads <= 1 << 10;
 }
 
 // ---- more rows: tiles, narrow and wide ----
@@ -610,6 +610,8 @@ TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k, bool wide) {
     for (int shape = 0; shape <= (wide ? kFlat : kSquare); shape++) {
         const TileShape &t = kTileShapes[shape];
         if ((shape == kSquare && epilogue == kTileResidual) || (shape >= kSquare && k < kWideLeastK)) continue;
+        // (a product of more columns reaches this without wide_covers, too)
+        if (shape == kSquare && epilogue == kTileSilu && n > kWideMostColumns) continue;
         const int m_tiles = (rows + t.rows - 1) / t.rows, n_tiles = (columns + t.columns - 1) / t.columns, stages = k / kTileK;
         for (int split = 1; split <= 8; split *= 2) {
             if (split > 1 && (whole || stages / split < 8 || shape == kSquare)) break;

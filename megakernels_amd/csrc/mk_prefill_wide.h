@@ -34,7 +34,11 @@ __device__ __forceinline__ int wide_weight_row(const TileArgs &a, int n_tile, in
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void *base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, (int)bytes, 0x00020000);
 }
-constexpr uint32_t kOutside = 0x80000000u;  // an offset beyond every buffer: nothing is stored
+// Offsets have 32 bits, and kOutside, where nothing is stored, is one beyond every buffer that is written: 256 rows of at most
+// this many columns of two bytes.
+constexpr int kWideMostColumns = 1 << 20;
+constexpr uint32_t kOutside = 0x80000000u;
+static_assert(256ll * kWideMostColumns * 2 <= kOutside);
 
 // a phase of the other group lies between two of these
 __device__ __forceinline__ void wide_meet() {

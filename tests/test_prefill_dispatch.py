@@ -148,8 +148,8 @@ def test_calls_that_are_recorded_are_not_taken():
     assert torch.equal(torch.compile(lambda x: x + int(_covers(model)), backend="eager", fullgraph=True)(torch.zeros(2)), torch.zeros(2))
 
 
-def _workspace(rows, hidden, batch=1):
-    shape = prefill.Shape(batch, rows // batch, 32, 8, 64, hidden, 4 * hidden, 32768, rows, rows, 1, 1e-5)
+def _workspace(rows, hidden, batch=1, inter=None):
+    shape = prefill.Shape(batch, rows // batch, 32, 8, 64, hidden, inter or 4 * hidden, 32768, rows, rows, 1, 1e-5)
     return prefill.load_library().mk_prefill_workspace_bytes(ctypes.byref(shape))
 
 
@@ -236,3 +236,14 @@ def test_wide_plans_and_forwards_are_refused_where_there_are_none():
     shape = prefill.Shape(1, 1000, 32, 8, 64, 2048, 8192, 32768, 1000, 1000, 1, 1e-5)
     assert lib.mk_prefill_wide_plan(ctypes.byref(shape), 0, None) < 0
     assert lib.mk_prefill_wide_forward(ctypes.byref(shape), None, None, None, None, None, None, None) < 0 and lib.mk_prefill_last_error()
+
+
+@pytest.mark.parametrize("rows,hidden", [(256, 256), (129, 256), (1000, 256), (200, 2048)])
+def test_gate_and_up_of_more_columns_than_32_bits_address_run_in_narrow_tiles(rows, hidden):
+    """256 x 256 tiles address gate and up's output, 256 rows of it, with 32 bits: the forward that takes intermediate sizes
+    beyond 2^20 must not run it in them."""
+    square, up = 3, 2
+    assert _plan(up, rows, hidden, 1 << 20)[1] == square
+    for inter in ((1 << 20) + 64, 4194368, 8388672, (1 << 25) + 64):   # 8388672: 256 rows are 2^32 bytes and a little
+        assert _workspace(rows, hidden, inter=inter) > 0 and _wide_workspace(rows, hidden, inter=inter) == 0
+        assert _plan(up, rows, hidden, inter)[1] < square
