@@ -1,6 +1,7 @@
 """The prompt forward's HIP kernels against the plain PyTorch forward on the CPU: hidden states, cache rows and greedy
 ids, at the sizes where tiles, waves and position groups begin and end."""
 
+import ctypes
 import math
 
 import pytest
@@ -225,6 +226,51 @@ def test_argmax_of_wide_tiles_with_no_positive_logit_and_with_nan(vocab, seq):
     assert bool((model.to("cuda:0")(batch).output_ids == 4100).all())
 
 
+@pytest.mark.parametrize("seq,tiles", [(300, 4), (700, 3)])
+def test_silu_of_every_gate_in_wide_tiles(seq, tiles):
+    """Every bf16 gate through the two kernels' own exponential and division, against the kernel that has the library's: gate
+    `n` is weight `n` of the gate projection times one, up is one, and the down projection leaves it in column `n`."""
+    lib = prefill.load_library()
+    cfg = config_1b_slice(layers=1, vocab=1024)
+    hid, inter = cfg.hidden_size, cfg.intermediate_size
+    model = _model(cfg, seq).to("cuda:0")
+    p, embed = model.stacked_params, model.model.embed_tokens.weight
+    shape = prefill.Shape(1, seq, cfg.num_attention_heads, cfg.num_key_value_heads, cfg.head_dim, hid, inter, cfg.vocab_size, seq,
+                          model.model.rope_cos.shape[0], 1, cfg.rms_norm_eps)
+    plan = (ctypes.c_int32 * 4)()
+    assert lib.mk_prefill_wide_plan(ctypes.byref(shape), 2, plan) == 0 and plan[0] == tiles
+    for t in (p.qkv_proj, p.o_proj, p.gate_proj, p.up_proj, p.down_proj, embed):
+        t.zero_()
+    embed[:, 0] = 64.0
+    p.mlp_ln_weight[0, 0] = 1 / hid**0.5   # normed, column 0 is one
+    p.up_proj[0, :hid, 0] = 1.0
+    p.down_proj[0, :, :hid] = torch.eye(hid)
+    batch = BatchState(input_ids=torch.zeros(1, seq, dtype=torch.int64, device="cuda:0"), position_ids=torch.arange(seq, device="cuda:0"))
+
+    def through(gates):   # of columns 1 and up
+        p.gate_proj[0, 1:hid, 0] = gates
+        return model(batch).hidden_states[0, :, 1:]
+
+    every = torch.arange(65536, dtype=torch.int32).to(torch.int16).view(torch.bfloat16).cuda()
+    least = 2.0**-126   # smaller ones the matrix cores may flush, on the way in or out
+    gates = every[every.isfinite() & (every.abs() >= least)]
+    gates = torch.nn.functional.pad(gates, (0, -len(gates) % 8))
+    ones, expected = torch.ones_like(gates), torch.empty_like(gates)
+    one_row = prefill.Shape(1, 1, 4, 1, 64, 64, len(gates), 8, 1, 1, 1, 1e-5)
+    assert lib.mk_prefill_silu_mul(ctypes.byref(one_row), gates.data_ptr(), ones.data_ptr(), expected.data_ptr(), None) == 0
+    torch.cuda.synchronize()
+    for first in range(0, len(gates), hid - 1):
+        part, want = gates[first:first + hid - 1], expected[first:first + hid - 1]
+        got = through(torch.nn.functional.pad(part, (0, hid - 1 - len(part))))[:, :len(part)]
+        want = want.expand_as(got)
+        sure = want.abs() >= least
+        assert torch.equal(got[sure], want[sure]) and bool((got[~sure].abs() <= least).all()), first
+    for special, want in ((math.inf, math.inf), (-math.inf, math.nan), (math.nan, math.nan)):
+        gate = torch.zeros(hid - 1)
+        gate[9] = special
+        assert torch.allclose(through(gate)[:, 9].float(), torch.tensor(want, device="cuda:0"), equal_nan=True)
+
+
 @pytest.mark.parametrize("seq", [300, 540, 777, 1020])
 def test_narrow_tiles_where_wide_ones_are_preferred(seq, monkeypatch):
     lib = prefill.load_library()
@@ -336,8 +382,6 @@ def test_wide_forward_in_a_captured_graph(seq):
 
 def test_argmax_takes_the_first_maximum_and_nan_above_all():
     lib = prefill.load_library()
-    import ctypes
-
     vocab = 1024
     logits = torch.randn(5, vocab).to(torch.bfloat16)
     logits[0] = -3.0
@@ -354,8 +398,6 @@ def test_argmax_takes_the_first_maximum_and_nan_above_all():
 
 
 def test_shapes_outside_the_kernels_are_refused():
-    import ctypes
-
     lib = prefill.load_library()
     for field, value in (("head_dim", 96), ("num_attention_heads", 16), ("hidden_size", 516), ("seq", 0), ("vocab_size", 1001)):
         shape = prefill.Shape(1, 5, 8, 2, 64, 512, 1024, 1024, 8, 8, 1, 1e-5)
