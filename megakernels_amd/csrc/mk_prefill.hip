@@ -620,7 +620,9 @@ TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k, bool wide) {
             if (wide && split > 1 && rounds > 1) break;
             const float meeting = split > 1 ? 3.0f + (float)split * rows * columns * 8 / 3e6f : 0.0f;
             float full = (float)rounds;
-            if (wide && shape == kSquare && (int64_t)m_tiles * n_tiles % t.slots && (int64_t)m_tiles * n_tiles % t.slots <= t.slots / 2) full -= 0.35f;  // halves
+            // halves of tiles in a last round that they fit, which square_kernel has but for rotation
+            const int64_t last = (int64_t)m_tiles * n_tiles % t.slots;
+            if (wide && shape == kSquare && epilogue != kTileRope && last && last <= t.slots / 2) full -= 0.35f;
             const float us = full * ((stages + split - 1) / split) * t.stage_us + 3.0f + meeting;
             if (best.split == 0 || us < best.us) best = {shape, split, m_tiles, n_tiles, us};
         }

@@ -247,3 +247,12 @@ def test_gate_and_up_of_more_columns_than_32_bits_address_run_in_narrow_tiles(ro
     for inter in ((1 << 20) + 64, 4194368, 8388672, (1 << 25) + 64):   # 8388672: 256 rows are 2^32 bytes and a little
         assert _workspace(rows, hidden, inter=inter) > 0 and _wide_workspace(rows, hidden, inter=inter) == 0
         assert _plan(up, rows, hidden, inter)[1] < square
+
+
+def test_rotation_is_not_planned_for_halves_of_tiles_that_it_does_not_have():
+    """Two whole rounds of 256 x 256 tiles take longer than two of 128 x 256, which one and a half would not."""
+    flat, qkv = 4, 0
+    for hidden, rows, inter in ((2048, range(2689, 4097), 1024), (8192, range(1281, 2049), 28672)):
+        heads = 32 if hidden == 2048 else 64
+        plans = {_wide_plan(qkv, r, hidden, inter, heads, heads // 4, 128)[1] for r in rows}
+        assert plans == {flat}, (hidden, plans)
