@@ -601,8 +601,11 @@ struct TilePlan {
 };
 // The plan with the least estimated time: rounds of blocks, 3 us to start and end, and for a split of K the blocks' meeting
 // and their sums' way through memory.  (rows 253: 2048 x 8192 estimated 25, measured 24.3 in 64 x 128 x 4 parts against
-// 52.9 whole; rows 777: 16384 x 2048 58 and 56.8 in 256 x 256 against 70.4 in 128 x 128.)  The residual epilogue has no
-// 256 x 256: its products are narrow, and 128 x 256 fills the chip twice as soon.
+// 52.9 whole; rows 777: 16384 x 2048 estimated 48, measured 51.4 in 256 x 256.)  Rounds are those of the XCD with the most
+// column tiles, as column tile n is XCD n % 8's: 12 of them are two for four XCDs and one for the others.  (Counted over the
+// whole chip, plans were chosen that took a round more: whole forwards of eight layers, us, 1536 wide 2300 rows 2763 -> 2442,
+// 2304 wide 560 rows 1744 -> 1521, 2048 wide 2300 rows 3317 -> 3220.)  The residual epilogue has no 256 x 256: its products are
+// narrow, and 128 x 256 fills the chip twice as soon.
 TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k, bool wide) {
     const int columns = epilogue == kTileSilu ? 2 * n : n;
     const bool whole = epilogue == kTileSilu || epilogue == kTileArgmax;  // no split of K
@@ -615,14 +618,14 @@ TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k, bool wide) {
         const int m_tiles = (rows + t.rows - 1) / t.rows, n_tiles = (columns + t.columns - 1) / t.columns, stages = k / kTileK;
         for (int split = 1; split <= 8; split *= 2) {
             if (split > 1 && (whole || stages / split < 8 || shape == kSquare)) break;
-            const int64_t rounds = ((int64_t)m_tiles * n_tiles * split + t.slots - 1) / t.slots;
+            const int64_t tiles = (int64_t)((n_tiles + 7) / 8) * m_tiles * split, slots = t.slots / 8;  // of the fullest XCD
+            const int64_t rounds = (tiles + slots - 1) / slots;
             // more sums than fit one round of blocks cost more than the estimate (3000 rows of an 8B model's layers)
             if (wide && split > 1 && rounds > 1) break;
             const float meeting = split > 1 ? 3.0f + (float)split * rows * columns * 8 / 3e6f : 0.0f;
             float full = (float)rounds;
             // halves of tiles in a last round that they fit, which square_kernel has but for rotation
-            const int64_t last = (int64_t)m_tiles * n_tiles % t.slots;
-            if (wide && shape == kSquare && epilogue != kTileRope && last && last <= t.slots / 2) full -= 0.35f;
+            if (wide && shape == kSquare && epilogue != kTileRope && tiles % slots && tiles % slots <= slots / 2) full -= 0.35f;
             const float us = full * ((stages + split - 1) / split) * t.stage_us + 3.0f + meeting;
             if (best.split == 0 || us < best.us) best = {shape, split, m_tiles, n_tiles, us};
         }

@@ -37,7 +37,7 @@ TILED_WIDE_HEADS = [(2048, 700), (512, 1400)]                             # hidd
 TILED_ARGMAX = [(1048, 90), (10008, 300), (40008, 100), (40008, 200)]     # vocabulary, rows, of the tiny configuration
 # The same for the forward of wide tiles: layers of the 1B and of the 8B architecture, vocabularies for its last product, and
 # heads of 128 from a narrower hidden state.
-WIDE_1B = [257, 300, 400, 600, 1100, 1300, 1500, 2700, 4096]   # 600, 1300, 4096: halves of 256 x 256 tiles
+WIDE_1B = [257, 300, 400, 600, 1100, 1300, 1500, 2300, 2700, 4096]   # 600, 1300, 4096: halves of 256 x 256 tiles
 WIDE_8B = [513, 705, 1100, 1300, 1700]
 WIDE_HEAD = [(8200, 300), (24584, 700)]                                   # vocabulary, rows; last tiles of 8 columns, halves
 

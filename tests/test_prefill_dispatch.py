@@ -256,3 +256,17 @@ def test_rotation_is_not_planned_for_halves_of_tiles_that_it_does_not_have():
         heads = 32 if hidden == 2048 else 64
         plans = {_wide_plan(qkv, r, hidden, inter, heads, heads // 4, 128)[1] for r in rows}
         assert plans == {flat}, (hidden, plans)
+
+
+def test_plans_count_the_rounds_of_the_xcd_with_the_most_column_tiles():
+    """Column tile n is XCD n % 8's, of 32 CUs with one block of these shapes each: a plan must not need a second round there
+    while another shape needs one that is less than twice as long."""
+    qkv, o, down, medium, two_a_cu, flat = 0, 1, 3, 1, 2, 4
+    # 12 tiles of 128 columns and 20 row tiles: two rounds of 40 tiles a XCD, where 128 x 256 has one of 20
+    for rows in (2049, 2300, 2500):
+        shape = dict(hidden=1536, inter=6144, heads=24, kv_heads=6)
+        assert _wide_plan(o, rows, **shape)[1:] == (flat, 1) and _wide_plan(down, rows, **shape)[1:] == (flat, 1)
+        # 12 tiles of 256 columns of the 1B architecture, 17 to 20 row tiles
+        assert _wide_plan(qkv, rows)[1:] == (two_a_cu, 1)
+    # K in four parts only where all of them are in one round
+    assert _wide_plan(down, 560, hidden=2304, inter=9216, heads=20, kv_heads=5, head_dim=128)[1:] == (medium, 2)
