@@ -79,9 +79,9 @@ int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *mo
 int mk_prefill_tile_plan(const mk_prefill_shape *shape, int product, int32_t plan[4]);
 
 /* The whole forward of longer prompts and wider models, from wide tiles; arguments as above.  Workspace 0: not such a call -
- * up to 256 or more than 4096 rows (of a model wider than 2048: up to 512 or more than 2048), a hidden size below 256 or no
- * multiple of 64, an intermediate size that is no multiple of 64 or above 2^20, a cache of 2^31 rows.  mk_prefill_wide_plan: as
- * mk_prefill_tile_plan. */
+ * fewer than 257 or more than 4096 rows (of a model wider than 2048 fewer than 513, wider than 6144 fewer than 641, and more than
+ * 1024, 3072 to 4096 wide more than 2048), a hidden size below 256 or no multiple of 64, an intermediate size that is no multiple
+ * of 64 or above 2^20, a cache of 2^31 rows.  mk_prefill_wide_plan: as mk_prefill_tile_plan. */
 int64_t mk_prefill_wide_workspace_bytes(const mk_prefill_shape *shape);
 int mk_prefill_wide_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids,
                             const int64_t *positions, uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream);

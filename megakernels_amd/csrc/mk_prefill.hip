@@ -570,10 +570,23 @@ bool tiles_cover(const mk_prefill_shape &s) {
 //   8B architecture: 520 rows 11889 and 11437, 640 rows 12608 and 12239, 777 rows 15119 and 13540, 2048 rows 28328 and 26686,
 //     2300 rows 31529 and 34397, 2600 rows 44288 and 38257, 3000 rows 41329 and 43537, 4096 rows 53581 and 54067 (library)
 // Prompts of up to 512 rows of wide models are the library's for the reason above.
+// The lines for other widths, from whole forwards of four or eight layers with vocabularies of 32768, us, library's products (or
+// narrow tiles, up to 2^21 values of a narrow model) and wide.  Which one wins depends on how the rounds of both fit:
+//   up to 2048 wide: 512 wide 4096 rows 1528 and 1386, 1024 wide 2049 rows 1624 and 1444, 1536 wide 2300 rows 2405 and 2442, 4096
+//     rows 3866 and 3444.  Beyond 4096 rows 2048 wide 5000 rows 6572 and 6392, 8192 rows 10414 and 10181: not crossed, but not
+//     looked at for narrower models or the whole architecture.
+//   2049 to 3071 wide: 2304 wide 560 rows 1751 and 1521, 1024 rows 2445 and 2311, but 1300 rows 2591 and 2811, 1536 rows 2922 and
+//     3110; 2560 wide 700 rows 2124 and 2021, but 1100 rows 2599 and 2876
+//   3072 to 4096 wide: 3072 wide 513 rows 1842 and 1648, 1300 rows 3113 and 3073, 2048 rows 3969 and 3855; 3584 wide 513 rows 1635 and
+//     1578, 2048 rows 5236 and 3773; the worst of 60 sizes 3840 wide, 1100 rows, 1.07 times the library's
+//   wider: 5120 wide 650 rows 2152 and 2006, 1024 rows 2802 and 2681, but 1650 rows 4275 and 4717; 6144 wide 560 rows 3521 and 3040,
+//     but 2048 rows 8005 and 8422; 7168 wide 560 rows 3237 and 3509 (five row tiles fill five eighths of the chip), 777 rows 4660 and
+//     3984, but 1400 rows 5965 and 6993; 8192 wide 560 rows 4447 and 4574, 777 rows 6070 and 5707, but 1536 rows 9203 and 10004
 bool wide_covers(const mk_prefill_shape &s) {
     const int64_t rows = (int64_t)s.batch * s.seq;
-    const bool narrow = s.hidden_size <= 2048;
-    return s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0 && s.hidden_size >= 256 && rows > (narrow ? 256 : 512) && rows <= (narrow ? 4096 : 2048)
+    const int hid = s.hidden_size;
+    const int least = hid <= 2048 ? 257 : hid <= 6144 ? 513 : 641, most = hid <= 2048 ? 4096 : hid >= 3072 && hid <= 4096 ? 2048 : 1024;
+    return hid % 64 == 0 && s.intermediate_size % 64 == 0 && hid >= 256 && rows >= least && rows <= most
         && (int64_t)s.batch * s.kv_max_len < INT32_MAX
         // (offsets of 32 bits within a tile's rows, of K as of the columns)
         && s.intermediate_size <= kWideMostColumns && s.num_kv_heads <= 1 << 10;

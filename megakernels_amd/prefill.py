@@ -1,7 +1,7 @@
 """The prompt forward on the GPU: the dense forward of ``llama.py`` over whole prompts (``csrc/mk_prefill.hip``).
 
 PyTorch owns the memory and the stream.  A prompt of up to some thousand positions (of a model wider than 2048: of some
-hundred to two thousand) runs as one call, its matrix products included.  For the others PyTorch computes the plain products,
+hundred to one or two thousand) runs as one call, its matrix products included.  For the others PyTorch computes the plain products,
 and everything between them - embedding, RMS norm, residual adds, rotary embedding, cache append, causal attention, SiLU,
 argmax - is this library's.  There is no fallback for a missing library: a GPU forward that it covers raises ``RuntimeError``.
 """

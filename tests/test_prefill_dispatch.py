@@ -187,7 +187,9 @@ def _wide_workspace(rows, hidden, batch=1, inter=None, max_len=8192):
     return prefill.load_library().mk_prefill_wide_workspace_bytes(ctypes.byref(shape))
 
 
-@pytest.mark.parametrize("hidden,least,most", [(256, 257, 4096), (1024, 257, 4096), (2048, 257, 4096), (2112, 513, 2048), (4096, 513, 2048), (8192, 513, 2048)])
+@pytest.mark.parametrize("hidden,least,most", [
+    (256, 257, 4096), (1024, 257, 4096), (2048, 257, 4096), (2112, 513, 1024), (3008, 513, 1024), (3072, 513, 2048), (4096, 513, 2048),
+    (4160, 513, 1024), (6144, 513, 1024), (6208, 641, 1024), (8192, 641, 1024)])
 def test_prompts_that_wide_tiles_take(hidden, least, most):
     assert _wide_workspace(least, hidden) > 0 and _wide_workspace(most, hidden) > 0 and _wide_workspace(most, hidden, batch=2) > 0
     assert _wide_workspace(least - 1, hidden) == 0 and _wide_workspace(most + 1, hidden) == 0
@@ -252,10 +254,7 @@ def test_gate_and_up_of_more_columns_than_32_bits_address_run_in_narrow_tiles(ro
 def test_rotation_is_not_planned_for_halves_of_tiles_that_it_does_not_have():
     """Two whole rounds of 256 x 256 tiles take longer than two of 128 x 256, which one and a half would not."""
     flat, qkv = 4, 0
-    for hidden, rows, inter in ((2048, range(2689, 4097), 1024), (8192, range(1281, 2049), 28672)):
-        heads = 32 if hidden == 2048 else 64
-        plans = {_wide_plan(qkv, r, hidden, inter, heads, heads // 4, 128)[1] for r in rows}
-        assert plans == {flat}, (hidden, plans)
+    assert {_wide_plan(qkv, rows, head_dim=128)[1] for rows in range(2689, 4097)} == {flat}   # 6144 columns
 
 
 def test_plans_count_the_rounds_of_the_xcd_with_the_most_column_tiles():
