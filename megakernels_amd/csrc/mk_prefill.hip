@@ -490,12 +490,16 @@ template <int MT, int EPI, bool NORM>
 int launch_rows_wide(const RowsArgs &a, int split, const char *what, hipStream_t stream) {
     return launch_rows<MT, 2, 4, 2, EPI, NORM>(a, split, what, stream);
 }
-// Four tiles a block where there are enough columns (gate and up, LM head): a block reads X once, and with two tiles X's
+// Four tiles a block where there are enough columns (LM head, gate and up): a block reads X once, and with two tiles X's
 // bytes from L2 are as many as W's from memory.  Whole forwards of the 1B layers, us, two and four tiles: 12 rows 860 and
-// 843, 32 rows 925 and 898, 60 rows 1146 and 1073.
-constexpr int kRowsFar = 4;
+// 843, 32 rows 925 and 898, 60 rows 1146 and 1073.  Gate and up have two where blocks of four are no more than half the CUs: whole
+// forwards of eight layers, 32 rows, us, two and four tiles, 5120 columns (160 blocks of four) 342 and 331, 4096 columns 274 and
+// 284, 2048 columns 189 and 203; 64 rows 442 and 415, 340 and 341, 224 and 239.
+constexpr int kRowsFar = 4, kRowsFarBlocks = 129;
 template <int MT, int EPI>
 int launch_rows_far(const RowsArgs &a, const char *what, hipStream_t stream) {
+    if constexpr (EPI == kRowsSilu)
+        if ((a.n + kRowsFar * 8 - 1) / (kRowsFar * 8) < kRowsFarBlocks) return launch_rows<MT, 2, 4, MT == 4 ? 1 : 2, EPI, true>(a, 1, what, stream);
     return launch_rows<MT, kRowsFar, 4, 1, EPI, true>(a, 1, what, stream);
 }
 // One tile a block: where there is at most one block per CU it has eight waves, so that the CU has enough loads in flight.
