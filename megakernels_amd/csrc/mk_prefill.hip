@@ -479,7 +479,7 @@ int rows_split(int k) { return k >= 6144 ? 4 : 1; }
 template <int MT, int NT, int WAVES, int STAGES, int EPI, bool NORM>
 int launch_rows(const RowsArgs &a, int split, const char *what, hipStream_t stream) {
     const int width = EPI == kRowsSilu ? NT * 8 : NT * 16, bytes = RowsLds<MT, NT, WAVES, STAGES, NORM>::bytes(a.k);
-    auto *kernel = rows_kernel<MT, NT, WAVES, STAGES, EPI, NORM>;
+    auto *kernel = a.past ? rows_kernel<MT, NT, WAVES, STAGES, EPI, NORM, true> : rows_kernel<MT, NT, WAVES, STAGES, EPI, NORM, false>;
     const hipError_t e = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) return fail(-5, "%s: %d bytes of LDS: %s", what, bytes, hipGetErrorString(e));
     kernel<<<dim3((a.n + width - 1) / width, split), WAVES * 64, bytes, stream>>>(a);
@@ -523,6 +523,15 @@ int launch_rows(const RowsArgs &a, const char *what, hipStream_t stream) {
         if (a.rows <= 32) return launch_rows_far<2, EPI>(a, what, stream);
         return launch_rows_far<4, EPI>(a, what, stream);
     }
+}
+
+// Weights that one forward uses once go past the caches, unless the last-level cache (256 MiB) holds about all of the model's, for
+// the next forward.  Whole forwards, 32 rows, us, through the caches and past them: the 1B architecture (2.5 GB) 896 and 865, 1024
+// wide with ten layers (371 MB) 336 and 327, eight (310 MB) 279 and 272, seven (280 MB) 238 and 240, five (219 MB) 157 and 179.
+constexpr int64_t kRowsCached = 280 << 20;
+bool rows_past(const mk_prefill_shape &s, int layers) {
+    const int64_t heads = (int64_t)s.num_attention_heads * s.head_dim, kv = (int64_t)s.num_kv_heads * s.head_dim;
+    return 2 * s.hidden_size * (layers * (2 * heads + 2 * kv + 3ll * s.intermediate_size) + s.vocab_size) > kRowsCached;
 }
 
 // the workspace of the forward for few rows, in elements of 2 bytes; every part a multiple of 16 bytes
@@ -844,7 +853,7 @@ int rows_forward(const mk_prefill_shape &s, const mk_prefill_model &w, const int
     if (int rc = launched("embed")) return rc;
 
     RowsArgs base{};
-    base.s = s, base.rows = rows, base.padded = padded_seq(s.seq), base.positions = positions;
+    base.s = s, base.rows = rows, base.padded = padded_seq(s.seq), base.positions = positions, base.past = rows_past(s, w.num_layers);
     base.rope_cos = w.rope_cos, base.rope_sin = w.rope_sin, base.keys = keys, base.values_t = values_t, base.best = best;
     base.arrived = (int *)(workspace + at.arrived), base.partial = (float *)(workspace + at.partial);
     const size_t qkv_rows = (size_t)(H + 2 * KVH) * D, cache_layer = (size_t)w.cache_batch * s.kv_max_len * KVH * D;

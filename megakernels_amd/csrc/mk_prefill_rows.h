@@ -23,6 +23,7 @@ enum RowsEpilogue { kRowsRope, kRowsResidual, kRowsSilu, kRowsArgmax };
 struct RowsArgs {
     mk_prefill_shape s;
     int rows, n, k, padded;
+    bool past;                                  // whether the weights go past the caches
     const uint16_t *x, *norm_weight, *w0, *w1;  // x [rows, k]; w0 (and w1: up beside gate) [n, k]
     uint16_t *out;                              // residual: h, in place; SiLU: [rows, n]; rope: q [rows, H D]
     const int64_t *positions;
@@ -144,7 +145,7 @@ struct RowsLds {
     static constexpr int bytes(int k) { return kRing + (NORM ? (k / 64 + WAVES * 8 - 1) / (WAVES * 8) * WAVES * 1024 : 0); }
 };
 
-template <int MT, int NT, int WAVES, int STAGES, int EPI, bool NORM>
+template <int MT, int NT, int WAVES, int STAGES, int EPI, bool NORM, bool PAST>
 __global__ __launch_bounds__(WAVES * 64) void rows_kernel(RowsArgs a) {
     typedef RowsLds<MT, NT, WAVES, STAGES, NORM> Lds;
     constexpr int kLoads = (NT + MT) * 2;  // load instructions of a step
@@ -185,8 +186,7 @@ __global__ __launch_bounds__(WAVES * 64) void rows_kernel(RowsArgs a) {
             unsigned char *const slot = ring + i % STAGES * Lds::kStep;
 #pragma unroll
             for (int j = 0; j < kLoads; j++) {
-                // the weights past the caches: they are used once (32 rows of the 1B architecture 899 us without, 868)
-                constexpr int kPast = 2;
+                constexpr int kPast = PAST ? 2 : 0;
                 const MK_GLOBAL void *const from = (const MK_GLOBAL void *)(src[j] + (size_t)i * (WAVES * 64));
                 MK_LDS void *const to = (MK_LDS void *)(slot + j * 1024);
                 if (j < 2 * NT) __builtin_amdgcn_global_load_lds(from, to, 16, 0, kPast);

@@ -131,6 +131,13 @@ def test_norm_weights_of_every_size(seq):
     _compare(config_1b_slice(vocab=1024), seq, norms=True)
 
 
+@pytest.mark.parametrize("seq", [7, 20, 50])   # the other tests' models of few rows fit the last-level cache
+def test_prefill_of_few_rows_with_weights_past_the_caches(seq):
+    cfg = config_1b_slice(vocab=65536)
+    assert 2 * cfg.hidden_size * cfg.vocab_size + 2 * 3 * cfg.num_hidden_layers * cfg.hidden_size * cfg.intermediate_size > 300 << 20
+    _compare(cfg, seq)
+
+
 @pytest.mark.parametrize("seq", [7, 20, 50])
 def test_prefill_of_few_rows_with_heads_wider_than_the_stream(seq):
     _compare(config_heads_wider_than_the_stream(), seq)
