@@ -67,21 +67,21 @@ typedef struct mk_prefill_model {
 
 /* The whole forward where batch * seq is not too large: matrix products included, all in kernels of this library.
  * h [rows, hidden_size] becomes the hidden states, out_ids [rows] the greedy ids.  The workspace's size is
- * mk_prefill_workspace_bytes.  0: not such a call - a hidden size above 2048 or no multiple of 64, an intermediate size that is
- * no multiple of 64, more than 64 rows that are above 4096 or above 2^21 / hidden_size.  Negative: an error. */
+ * mk_prefill_workspace_bytes.  0: not such a call - more than 4096 rows of a model up to 2048 wide; of a wider one fewer than 513 or
+ * more than 1024 (3072 to 4096 wide: 2048, above 6144: fewer than 641); a hidden or intermediate size that is no multiple of 64.
+ * (Of a model with an intermediate size above 2^20, a cache of 2^31 rows or more than 1024 KV heads: more than
+ * 2^21 / hidden_size of more than 64 rows, or a hidden size above 2048.)  Negative: an error. */
 int64_t mk_prefill_workspace_bytes(const mk_prefill_shape *shape);
 int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids,
                             const int64_t *positions, uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream);
 
-/* How the whole forward of more than 64 rows tiles a product (0 qkv, 1 O, 2 gate and up, 3 down, 4 LM head): plan = index of
+/* How mk_prefill_forward of more than 64 rows tiles a product (0 qkv, 1 O, 2 gate and up, 3 down, 4 LM head): plan = index of
  * the kernel's shape, rows and columns of a tile, parts of K.  Host arithmetic only; what tests need to know that they reach
  * every kernel. */
 int mk_prefill_tile_plan(const mk_prefill_shape *shape, int product, int32_t plan[4]);
 
-/* The whole forward of longer prompts and wider models, from wide tiles; arguments as above.  Workspace 0: not such a call -
- * fewer than 257 or more than 4096 rows (of a model wider than 2048 fewer than 513, wider than 6144 fewer than 641, and more than
- * 1024, 3072 to 4096 wide more than 2048), a hidden size below 256 or no multiple of 64, an intermediate size that is no multiple
- * of 64 or above 2^20, a cache of 2^31 rows.  mk_prefill_wide_plan: as mk_prefill_tile_plan. */
+/* Those calls of the above that run in wide tiles, alone: mk_prefill_forward, and its workspace and plans, of longer prompts and
+ * wider models.  Workspace 0, or an error: not such a call - fewer than 257 rows, a hidden size below 256, or one in the brackets above. */
 int64_t mk_prefill_wide_workspace_bytes(const mk_prefill_shape *shape);
 int mk_prefill_wide_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids,
                             const int64_t *positions, uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream);

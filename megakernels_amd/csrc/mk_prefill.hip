@@ -661,7 +661,8 @@ TilePlan tile_plan(TileEpilogue epilogue, int rows, int n, int k, bool wide) {
 // the five products of a layer and of the head
 struct Plans {
     TilePlan qkv, o, up, down, head;
-    Plans(const mk_prefill_shape &s, bool wide) {
+    explicit Plans(const mk_prefill_shape &s) {
+        const bool wide = wide_covers(s);
         const int rows = s.batch * s.seq, heads = s.num_attention_heads * s.head_dim, kv = s.num_kv_heads * s.head_dim;
         qkv = tile_plan(kTileRope, rows, heads + 2 * kv, s.hidden_size, wide);
         o = tile_plan(kTileResidual, rows, s.hidden_size, heads, wide);
@@ -753,39 +754,40 @@ extern "C" {
 int64_t mk_prefill_workspace_bytes(const mk_prefill_shape *shape) {
     if (int rc = check_shape(shape)) return rc;
     if (rows_covers(*shape)) return (int64_t)RowsWorkspace(*shape).total * 2;
-    return tiles_cover(*shape) ? (int64_t)TilesWorkspace(*shape, Plans(*shape, false)).total * 2 : 0;
+    return wide_covers(*shape) || tiles_cover(*shape) ? (int64_t)TilesWorkspace(*shape, Plans(*shape)).total * 2 : 0;
 }
 
 int mk_prefill_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids, const int64_t *positions,
                        uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream) {
     if (int rc = check_model(shape, model, ids, positions, h, workspace, out_ids)) return rc;
     if (rows_covers(*shape)) return rows_forward(*shape, *model, ids, positions, h, workspace, out_ids, (hipStream_t)stream);
-    if (tiles_cover(*shape)) return tiles_forward(*shape, *model, Plans(*shape, false), ids, positions, h, workspace, out_ids, (hipStream_t)stream);
+    if (wide_covers(*shape) || tiles_cover(*shape)) return tiles_forward(*shape, *model, Plans(*shape), ids, positions, h, workspace, out_ids, (hipStream_t)stream);
     return fail(-2, "%d x %d rows of %d, %d: not a call that the whole forward takes", shape->batch, shape->seq, shape->hidden_size, shape->intermediate_size);
 }
 
 int mk_prefill_tile_plan(const mk_prefill_shape *shape, int product, int32_t plan[4]) {
     if (int rc = check(shape, plan)) return rc;
-    if (rows_covers(*shape) || !tiles_cover(*shape)) return fail(-2, "%d x %d rows of %d: not tiled", shape->batch, shape->seq, shape->hidden_size);
-    return Plans(*shape, false).get(product, plan);
+    if (rows_covers(*shape) || !(wide_covers(*shape) || tiles_cover(*shape)))
+        return fail(-2, "%d x %d rows of %d: not tiled", shape->batch, shape->seq, shape->hidden_size);
+    return Plans(*shape).get(product, plan);
 }
 
 int64_t mk_prefill_wide_workspace_bytes(const mk_prefill_shape *shape) {
     if (int rc = check_shape(shape)) return rc;
-    return wide_covers(*shape) ? (int64_t)TilesWorkspace(*shape, Plans(*shape, true)).total * 2 : 0;
+    return wide_covers(*shape) ? mk_prefill_workspace_bytes(shape) : 0;
 }
 
 int mk_prefill_wide_forward(const mk_prefill_shape *shape, const mk_prefill_model *model, const int64_t *ids, const int64_t *positions,
                             uint16_t *h, uint16_t *workspace, int64_t *out_ids, void *stream) {
-    if (int rc = check_model(shape, model, ids, positions, h, workspace, out_ids)) return rc;
+    if (int rc = check_shape(shape)) return rc;
     if (!wide_covers(*shape)) return fail(-2, "%d x %d rows of %d, %d: not a call of wide tiles", shape->batch, shape->seq, shape->hidden_size, shape->intermediate_size);
-    return tiles_forward(*shape, *model, Plans(*shape, true), ids, positions, h, workspace, out_ids, (hipStream_t)stream);
+    return mk_prefill_forward(shape, model, ids, positions, h, workspace, out_ids, stream);
 }
 
 int mk_prefill_wide_plan(const mk_prefill_shape *shape, int product, int32_t plan[4]) {
     if (int rc = check(shape, plan)) return rc;
     if (!wide_covers(*shape)) return fail(-2, "%d x %d rows of %d: no wide tiles", shape->batch, shape->seq, shape->hidden_size);
-    return Plans(*shape, true).get(product, plan);
+    return mk_prefill_tile_plan(shape, product, plan);
 }
 
 int mk_prefill_padded_seq(int seq) { return padded_seq(seq); }

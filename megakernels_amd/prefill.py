@@ -132,12 +132,11 @@ def forward(model, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
     positions = positions.to(device=device, dtype=torch.int64).contiguous()
     shape = Shape(B, S, H, KVH, D, c.hidden_size, c.intermediate_size, c.vocab_size, k_cache.shape[2],
                   model.model.rope_cos.shape[0], int(bool(model.extra_config.interleave_rope)), c.rms_norm_eps)
-    for whole in ("wide_", ""):
-        workspace_bytes = getattr(lib, f"mk_prefill_{whole}workspace_bytes")(ctypes.byref(shape))
-        if workspace_bytes < 0:
-            raise RuntimeError(f"mk_prefill_{whole}workspace_bytes: {lib.mk_prefill_last_error().decode()}")
-        if workspace_bytes:
-            return _forward_whole(lib, f"mk_prefill_{whole}forward", model, shape, workspace_bytes, ids, positions)
+    workspace_bytes = lib.mk_prefill_workspace_bytes(ctypes.byref(shape))
+    if workspace_bytes < 0:
+        raise RuntimeError(f"mk_prefill_workspace_bytes: {lib.mk_prefill_last_error().decode()}")
+    if workspace_bytes:
+        return _forward_whole(lib, model, shape, workspace_bytes, ids, positions)
     padded = lib.mk_prefill_padded_seq(S)
 
     def rows(width):
@@ -168,7 +167,7 @@ def forward(model, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
     return h, out_ids
 
 
-def _forward_whole(lib, entry: str, model, shape, workspace_bytes: int, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
+def _forward_whole(lib, model, shape, workspace_bytes: int, ids: Tensor, positions: Tensor) -> tuple[Tensor, Tensor]:
     """A prompt that is not too long: one call launches the whole forward, matrix products included.  Issued one by one from
     Python, the launches of a short prompt took longer than the GPU needs for them."""
     c, device = model.config, ids.device
@@ -180,7 +179,7 @@ def _forward_whole(lib, entry: str, model, shape, workspace_bytes: int, ids: Ten
     out_ids = torch.empty(ids.shape, dtype=torch.int64, device=device)
     with torch.cuda.device(device):
         stream = torch.cuda.current_stream(device).cuda_stream
-        if getattr(lib, entry)(ctypes.byref(shape), ctypes.byref(pointers), ids.data_ptr(), positions.data_ptr(), h.data_ptr(),
-                               workspace.data_ptr(), out_ids.data_ptr(), stream) != 0:
-            raise RuntimeError(f"{entry}: {lib.mk_prefill_last_error().decode()}")
+        if lib.mk_prefill_forward(ctypes.byref(shape), ctypes.byref(pointers), ids.data_ptr(), positions.data_ptr(), h.data_ptr(),
+                                  workspace.data_ptr(), out_ids.data_ptr(), stream) != 0:
+            raise RuntimeError(f"mk_prefill_forward: {lib.mk_prefill_last_error().decode()}")
     return h, out_ids

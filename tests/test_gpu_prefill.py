@@ -29,17 +29,18 @@ def config_heads_wider_than_the_stream(hidden=2048):
     return cfg
 
 
-# Sizes above 64 rows at which the forward uses, between them, every tiling that it has for the 1B layers from 65 to 1024
-# rows (test_prefill_dispatch.py holds these lists against the library's own plans), and every kernel instance.
-TILED_1B = [70, 150, 200, 300, 540, 777, 1020]
+# Sizes above 64 rows at which the forward uses, between them, every tiling that it has for the 1B layers (test_prefill_dispatch.py
+# holds these lists, with those below, against the library's own plans), and every kernel instance.
+TILED_1B = [70, 150, 200, 253, 300, 540, 777, 1020]
 TILED_HEAD = [(128256, 70), (128256, 200), (128200, 777)]                 # vocabulary, rows; 128200: a last tile of 200 columns
 TILED_WIDE_HEADS = [(2048, 700), (512, 1400)]                             # hidden size, rows
+TILED_NARROW = [(192, 700), (192, 2100)]                                  # hidden sizes that wide tiles do not take
 TILED_ARGMAX = [(1048, 90), (10008, 300), (40008, 100), (40008, 200)]     # vocabulary, rows, of the tiny configuration
-# The same for the forward of wide tiles: layers of the 1B and of the 8B architecture, vocabularies for its last product, and
+# The same where wide tiles are among the shapes: layers of the 1B and of the 8B architecture, vocabularies for its last product, and
 # heads of 128 from a narrower hidden state.
 WIDE_1B = [257, 300, 400, 600, 1100, 1300, 1500, 2300, 2700, 4096]   # 600, 1300, 4096: halves of 256 x 256 tiles
 WIDE_8B = [513, 705, 1100, 1300, 1700]
-WIDE_HEAD = [(8200, 300), (24584, 700)]                                   # vocabulary, rows; last tiles of 8 columns, halves
+WIDE_HEAD = [(8200, 300), (8200, 700), (24584, 700)]                      # vocabulary, rows; last tiles of 8 columns, halves
 
 
 def _model(cfg, max_len, batch=1, interleave=True, seed=3):
@@ -278,16 +279,10 @@ def test_silu_of_every_gate_in_wide_tiles(seq, tiles):
         assert torch.allclose(through(gate)[:, 9].float(), torch.tensor(want, device="cuda:0"), equal_nan=True)
 
 
-@pytest.mark.parametrize("seq", [300, 540, 777, 1020])
-def test_narrow_tiles_where_wide_ones_are_preferred(seq, monkeypatch):
-    lib = prefill.load_library()
-
-    class OnlyNarrow:
-        def __getattr__(self, name):
-            return (lambda shape: 0) if name == "mk_prefill_wide_workspace_bytes" else getattr(lib, name)
-
-    monkeypatch.setattr(prefill, "_lib", OnlyNarrow())
-    _compare(config_1b_slice(layers=1), seq)
+@pytest.mark.parametrize("hidden,seq", TILED_NARROW)
+def test_narrow_tiles_of_long_prompts_of_narrow_models(hidden, seq):
+    _compare(config_heads_wider_than_the_stream(hidden), seq)
+    _compare(config_heads_wider_than_the_stream(hidden), seq, interleave=False)
 
 
 def test_prefill_of_few_rows_takes_the_first_of_equal_logits():

@@ -153,11 +153,21 @@ def _workspace(rows, hidden, batch=1, inter=None):
     return prefill.load_library().mk_prefill_workspace_bytes(ctypes.byref(shape))
 
 
-@pytest.mark.parametrize("hidden,most", [(2048, 1024), (1024, 2048), (512, 4096), (256, 4096), (64, 4096)])
+@pytest.mark.parametrize("hidden,most", [(2048, 4096), (1024, 4096), (512, 4096), (256, 4096), (64, 4096)])
 def test_prompts_beyond_the_measured_crossing_take_the_librarys_products(hidden, most):
     assert _workspace(most, hidden) > 0 and _workspace(most, hidden, batch=2) > 0
     assert _workspace(most + 1, hidden) == 0 and _workspace(8192, hidden, batch=4) == 0
     assert _workspace(40, 4096) == 0 and _workspace(40, hidden + 8) == 0
+    # what wide tiles do not take
+    inter, limit = (1 << 20) + 64, min(4096, (1 << 21) // hidden)
+    assert _workspace(limit, hidden, inter=inter) > 0 and _workspace(limit + 1, hidden, inter=inter) == 0
+
+
+@pytest.mark.parametrize("rows,hidden", [(257, 256), (1000, 2048), (4096, 1024), (513, 4096), (700, 8192)])
+def test_one_entry_chooses_between_the_tilings(rows, hidden):
+    assert _workspace(rows, hidden) == _wide_workspace(rows, hidden, max_len=rows) > 0
+    for product in range(5):
+        assert _plan(product, rows, hidden) == _wide_plan(product, rows, hidden)
 
 
 def _plan(product, rows, hidden=2048, inter=8192, heads=32, kv_heads=8, head_dim=64, vocab=128256):
@@ -170,15 +180,20 @@ def _plan(product, rows, hidden=2048, inter=8192, heads=32, kv_heads=8, head_dim
 def test_the_gpu_tests_reach_every_tiling_of_the_1b_layers_and_every_instance():
     import test_gpu_prefill as gpu
 
-    layers, head = range(4), 4
+    layers, head, square = range(4), 4, 3
     reached = {_plan(product, rows, vocab=8192) for rows in gpu.TILED_1B for product in layers}
     reached |= {_plan(head, rows, vocab=vocab) for vocab, rows in gpu.TILED_HEAD}
-    assert {_plan(product, rows) for rows in range(65, 1025) for product in range(5)} <= reached
-    reached |= {_plan(product, rows, hidden, 1024, head_dim=128) for hidden, rows in gpu.TILED_WIDE_HEADS for product in layers}
+    reached |= {_plan(head, rows, 512, 1024, 8, 2, vocab=vocab) for vocab, rows in gpu.WIDE_HEAD}
+    reached |= {_plan(product, rows, vocab=1024) for rows in gpu.WIDE_1B for product in range(5)}
+    assert {_plan(product, rows) for rows in range(65, 4097) for product in range(5)} <= reached
+    # up to 256 rows these plans are of the narrow tiles, which the sizes up to there reach by themselves
+    short = {_plan(product, rows, vocab=8192) for rows in gpu.TILED_1B if rows <= 256 for product in layers}
+    assert all(_wide_workspace(rows, 2048) == 0 for rows in (65, 256)) and {_plan(product, rows) for rows in range(65, 257) for product in layers} <= short
+    reached |= {_plan(product, rows, hidden, 1024, head_dim=128) for hidden, rows in gpu.TILED_WIDE_HEADS + gpu.TILED_NARROW for product in layers}
     reached |= {_plan(head, rows, 512, 1024, 8, 2, vocab=vocab) for vocab, rows in gpu.TILED_ARGMAX}
     epilogue = {0: "rope", 1: "residual", 2: "silu", 3: "residual", 4: "argmax"}
     instances = {(epilogue[product], shape) for product, shape, _ in reached}
-    assert instances == {(e, shape) for e in epilogue.values() for shape in range(4)} - {("residual", 3)}
+    assert instances == {(e, shape) for e in epilogue.values() for shape in range(5)} - {("residual", square)}
     assert {_plan(head, rows, 512, 1024, 8, 2, vocab=vocab)[1] for vocab, rows in gpu.TILED_ARGMAX} == {0, 1, 2, 3}
 
 
@@ -213,7 +228,9 @@ def test_the_gpu_tests_reach_every_wide_tiling_of_the_1b_and_8b_layers():
     assert {_wide_plan(product, rows) for rows in range(257, 4097) for product in range(4)} <= reached
     reached |= {_wide_plan(product, rows, vocab=4096, **of_8b) for rows in gpu.WIDE_8B for product in range(5)}
     assert {_wide_plan(product, rows, **of_8b) for rows in range(513, 2049) for product in range(4)} <= reached
-    reached |= {_wide_plan(head, rows, 512, 1024, 8, 2, vocab=vocab) for vocab, rows in gpu.WIDE_HEAD}
+    of_heads = {_wide_plan(head, rows, 512, 1024, 8, 2, vocab=vocab) for vocab, rows in gpu.WIDE_HEAD}
+    assert {shape for _, shape, _ in of_heads} >= {3, 4}   # 256 x 256 and 128 x 256, each with a last tile of 8 columns
+    reached |= of_heads
     assert {_wide_plan(head, rows) for rows in range(257, 4097)} <= reached
     # products that K is not split for run in 128 x 256 and 256 x 256, the residual ones in 128 x 256
     flat, square = 4, 3
@@ -224,7 +241,7 @@ def test_the_gpu_tests_reach_every_wide_tiling_of_the_1b_and_8b_layers():
 def test_tile_plans_are_refused_where_nothing_is_tiled():
     lib = prefill.load_library()
     plan = (ctypes.c_int32 * 4)()
-    for rows, hidden, product in ((64, 2048, 0), (1025, 2048, 0), (100, 4096, 0), (100, 2048, 5), (100, 2048, -1)):
+    for rows, hidden, product in ((64, 2048, 0), (4097, 2048, 0), (100, 4096, 0), (100, 2048, 5), (100, 2048, -1)):
         shape = prefill.Shape(1, rows, 32, 8, 64, hidden, 8192, 32768, rows, rows, 1, 1e-5)
         assert lib.mk_prefill_tile_plan(ctypes.byref(shape), product, plan) < 0 and lib.mk_prefill_last_error()
 
