@@ -566,8 +566,8 @@ bool whole_covers(const mk_prefill_shape &s) {
     return s.hidden_size <= 2048 && s.hidden_size % 64 == 0 && s.intermediate_size % 64 == 0;
 }
 bool rows_covers(const mk_prefill_shape &s) { return whole_covers(s) && (int64_t)s.batch * s.seq <= kRowsMax; }
-// From some thousand rows on the library's products are the faster ones.  Whole forwards of eight layers, intermediate size
-// four times the width, vocabulary 32768, library's products and tiles, us:
+// Narrow tiles alone, for what wide_covers leaves: from some thousand rows on the library's products are the faster ones.  Whole
+// forwards of eight layers, intermediate size four times the width, vocabulary 32768, library's products and tiles, us:
 //   2048 wide: 512 rows 1237 and 1176, 768 rows 1542 and 1555, 1024 rows 1808 and 1712, 1536 rows 2291 and 2567
 //   1024 wide: 1024 rows 1130 and 889, 2048 rows 1471 and 1365, 3000 rows 1886 and 1950, 4096 rows 2308 and 2430
 //    512 wide: 2048 rows 1150 and 866, 3000 rows 1268 and 1282, 4096 rows 1564 and 1536, 8192 rows 2664 and 2885

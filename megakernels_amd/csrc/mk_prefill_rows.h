@@ -15,6 +15,7 @@
 // 32 rows of a 2.5 GB model: 2225 us as library products with Python launches, 860 to 870 here (its bytes at the rate of a
 // copy, 4.9 TB/s: 507; at that of reads alone, 7.0 TB/s: 353).  60 rows: 1023.  More loads in flight (three or four stages,
 // twice the waves) change none of it: what is left is five launches a layer, each with its start from cold.
+// (Weights go past the caches there; through them, as those of a model that the last-level cache holds, 896.)
 // The blocks of a product read X again and again from L2 (M * K * 2 bytes each): the reason for the limit of kRowsMax.
 constexpr int kRowsMax = 64;
 

@@ -460,7 +460,7 @@ __global__ __launch_bounds__(512, 2) void square_kernel(TileArgs a) {
             finish(std::integral_constant<int, 2>{}, 0);
         } else {
             // per tile of K: one piece of rows, then both of columns, the second already the next tile's; three tiles ahead, past
-            // the end of K too, where nobody reads what arrives
+            // the end of K too, where nobody reads what arrives (of a buffer's last row zeros: its range check counts `at`, too)
             uint32_t off[2];
 #pragma unroll
             for (int j = 0; j < 2; j++) off[j] = item.rows == kLowerRows ? x_off[1][j] : x_off[0][j];
